@@ -40,8 +40,11 @@ struct kf_ctx {
   size_t grid_elems = 0;
   void *store = nullptr;  // per-state stores of the smoother (and track-state records)
   size_t store_bytes = 0;
-  void *carry = nullptr;    // forward -> backward kernel hand-over
+  void *carry = nullptr;    // forward -> backward kernel hand-over, kept first states
   size_t carry_bytes = 0;
+  void *redo = nullptr;     // fused fits: redo counters and list
+  size_t redo_bytes = 0;
+  bool redo_clean = false;  // its counters are zero (every complete fit leaves them so)
   void *adj = nullptr;      // chi2-adjoint buffers (step stack, plane adjoints, ...)
   size_t adj_bytes = 0;
   bool has_material = false;  // a plane of the table carries material
@@ -223,6 +226,7 @@ int kf_ctx_destroy(kf_ctx *ctx) {
   if (ctx->grid) (void)hipFree(ctx->grid);
   if (ctx->store) (void)hipFree(ctx->store);
   if (ctx->carry) (void)hipFree(ctx->carry);
+  if (ctx->redo) (void)hipFree(ctx->redo);
   if (ctx->adj) (void)hipFree(ctx->adj);
   if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
@@ -374,7 +378,8 @@ int setupArgs(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt, const cha
 
 constexpr size_t kCarryBytes = KF_CARRY_I * sizeof(int32_t) + KF_CARRY_D * sizeof(double);
 
-// Working-buffer bytes per track of the fit: per-state stores and hand-over.
+// Working-buffer bytes per track of the recording fit: per-state stores and
+// hand-over.
 size_t storeBytesPerTrack(const kfd::FitArgs &a, int precision, bool track_states,
                           bool checkpoints) {
   const size_t s_size = (precision == KF_PRECISION_FP64) ? sizeof(double) : sizeof(float);
@@ -383,6 +388,15 @@ size_t storeBytesPerTrack(const kfd::FitArgs &a, int precision, bool track_state
   if (checkpoints) per_state += KF_CK_N * sizeof(double);
   return (size_t)a.max_states * per_state + kCarryBytes;
 }
+
+// Whether a fit runs on the fused kernel (kf_fit_kernels.hpp).
+bool fitIsFused(int precision, bool track_states) {
+  return precision == KF_PRECISION_FP64 && !track_states;
+}
+
+// Working-buffer bytes per track of the fused fit: the kept first state and
+// the redo list.
+constexpr size_t kFusedBytesPerTrack = KF_FIRST_D * sizeof(double) + sizeof(uint32_t);
 
 // Positions per slice: the largest multiple of 64 whose working set fits the
 // budget (at least 64), or the whole batch.
@@ -439,12 +453,78 @@ int setupStores(kf_ctx *ctx, int precision, bool track_states, bool checkpoints,
   return KF_OK;
 }
 
+// Working storage of a fused fit for slices of up to `slice` positions: the
+// kept first states (carry), and for tracks that go to the RTS program the
+// list, and `waves` store chunks with their hand-over (redo).
+struct FusedLayout {
+  StoreLayout store;   // of waves x 64 lanes
+  size_t carry_bytes, list_bytes;
+  int64_t lanes;
+  size_t redo_bytes() const { return list_bytes + store.carry_bytes; }
+};
+FusedLayout fusedLayout(int precision, int64_t slice, int64_t waves, int32_t max_states) {
+  FusedLayout F;
+  F.lanes = waves * 64;
+  F.store = storeLayout(precision, false, false, F.lanes, max_states);
+  F.carry_bytes = ((size_t)slice * KF_FIRST_D * sizeof(double) + 255) / 256 * 256;
+  F.list_bytes = ((KF_REDO_LIST + (size_t)slice) * sizeof(uint32_t) + 255) / 256 * 256;
+  return F;
+}
+
+// Store chunks for tracks fitted again: as many as the slice has waves, within
+// the store budget and KF_REDO_WAVES (none or a few are used as a rule).
+int64_t redoWaves(int precision, int64_t slice, int32_t max_states, size_t budget) {
+  const size_t one = storeLayout(precision, false, false, 64, max_states).store();
+  int64_t w = (slice + 63) / 64;
+  if (w > KF_REDO_WAVES) w = KF_REDO_WAVES;
+  const int64_t fit = (int64_t)(budget / one);
+  if (w > fit) w = fit;
+  return w < 1 ? 1 : w;
+}
+
+void carveFused(const FusedLayout &F, void *store, void *carry, void *redo, kfd::FitArgs &a) {
+  a.tss = store;
+  a.tsd = (double *)((char *)store + F.store.s_bytes);
+  a.tsf = a.tsc = nullptr;
+  a.carry_d = (double *)carry;
+  a.carry_i = nullptr;
+  a.redo = (uint32_t *)redo;
+  a.redo_d = (double *)((char *)redo + F.list_bytes);
+  a.redo_i = (int32_t *)(a.redo_d + KF_CARRY_D * (size_t)F.lanes);
+  a.redo_lanes = F.lanes;
+}
+
+// The working storage of a fused fit, from the context's buffers (grown as
+// needed); the redo counters are zeroed when the buffer is new or a call failed
+// between the kernel that fills the list and the one that clears it.
+int setupFused(kf_ctx *ctx, int precision, int64_t slice, hipStream_t s, kfd::FitArgs &a) {
+  const size_t budget = (ctx->budget < KF_REDO_STORE_BYTES) ? (size_t)ctx->budget
+                                                            : (size_t)KF_REDO_STORE_BYTES;
+  const FusedLayout F = fusedLayout(precision, slice,
+                                    redoWaves(precision, slice, a.max_states, budget),
+                                    a.max_states);
+  int rc = grow(ctx, &ctx->store, &ctx->store_bytes, F.store.store(), s, "state store");
+  if (rc != KF_OK) return rc;
+  rc = grow(ctx, &ctx->carry, &ctx->carry_bytes, F.carry_bytes, s, "hand-over buffer");
+  if (rc != KF_OK) return rc;
+  if (F.redo_bytes() > ctx->redo_bytes) ctx->redo_clean = false;
+  rc = grow(ctx, &ctx->redo, &ctx->redo_bytes, F.redo_bytes(), s, "redo buffers");
+  if (rc != KF_OK) return rc;
+  carveFused(F, ctx->store, ctx->carry, ctx->redo, a);
+  if (!ctx->redo_clean) {
+    KF_HIP(ctx, kfd_launch_redo_reset(a.redo, s));
+    ctx->redo_clean = true;
+  }
+  return KF_OK;
+}
+
 // Sets positions first .. first + count - 1 as the launch's range; the
-// hand-over record is [30 doubles][count] followed by [6 ints][count].
+// hand-over record is [30 doubles][count] followed by [8 ints][count] (a fused
+// fit has its own, carveFused).
 void sliceRange(kfd::FitArgs &a, int64_t first, int64_t count) {
   a.first = first;
   a.count = count;
-  a.carry_i = (int32_t *)(a.carry_d + KF_CARRY_D * (size_t)count);
+  if (!a.redo) a.carry_i = (int32_t *)(a.carry_d + KF_CARRY_D * (size_t)count);
 }
 
 // The whole fit of a batch: the length sort over all positions, then the
@@ -501,8 +581,21 @@ int kf_fit_noalloc(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt,
     return fail(ctx, KF_E_HIP, "kf_fit_noalloc: workspace of device %d unavailable: %s",
                 ctx->device, hipGetErrorString(we));
   const bool ts = res->track_states != nullptr;
+  const bool fusedFit = fitIsFused(opt->precision, ts);
+  // a fused fit: the redo store takes at most half of the workspace (one
+  // chunk as a minimum)
+  auto fused = [&](int64_t slice) {
+    return fusedLayout(opt->precision, slice,
+                       redoWaves(opt->precision, slice, a.max_states,
+                                 (size_t)KF_NOALLOC_WORKSPACE_BYTES / 2),
+                       a.max_states);
+  };
   // the largest multiple of 64 positions whose storage fits the workspace
   auto fits = [&](int64_t slice) {
+    if (fusedFit) {
+      const FusedLayout F = fused(slice);
+      return F.store.store() + F.carry_bytes + F.redo_bytes() <= (size_t)KF_NOALLOC_WORKSPACE_BYTES;
+    }
     const StoreLayout L = storeLayout(opt->precision, ts, false, slice, a.max_states);
     return L.store() + L.carry_bytes <= (size_t)KF_NOALLOC_WORKSPACE_BYTES;
   };
@@ -527,12 +620,22 @@ int kf_fit_noalloc(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt,
     }
   }
   const int64_t slice = lo >= a.n ? a.n : lo;
-  const StoreLayout L = storeLayout(opt->precision, ts, false, slice, a.max_states);
-  carveStores(L, ws, (char *)ws + L.store(), ts, false, a);
   hipStream_t s = (hipStream_t)stream;
   KfdLaunch launch{};  // one thread per track, identity order
+  hipError_t e = hipSuccess;
   KF_HIP(ctx, hipEventRecord(ctx->ev0, s));
-  const hipError_t e = launchSlices(a, launch, opt->precision, res->track_states, slice,
+  if (!fusedFit) {
+    const StoreLayout L = storeLayout(opt->precision, ts, false, slice, a.max_states);
+    carveStores(L, ws, (char *)ws + L.store(), ts, false, a);
+  } else {
+    const FusedLayout F = fused(slice);
+    char *w = (char *)ws;
+    carveFused(F, w, w + F.store.store(), w + F.store.store() + F.carry_bytes, a);
+    // the workspace holds anything (an earlier call's slices)
+    e = kfd_launch_redo_reset(a.redo, s);
+  }
+  if (e == hipSuccess)
+    e = launchSlices(a, launch, opt->precision, res->track_states, slice,
                                     ctx->evm, s);
   if (e != hipSuccess)
     return fail(ctx, KF_E_HIP, "kf_fit_noalloc: launch failed: %s", hipGetErrorString(e));
@@ -550,8 +653,11 @@ int kf_fit(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt, const kf_res
   if (rc != KF_OK || tr->n_tracks == 0) return rc;
   hipStream_t s = (hipStream_t)stream;
   const bool ts = res->track_states != nullptr;
-  const int64_t slice = sliceTracks(ctx, a.n, storeBytesPerTrack(a, opt->precision, ts, false));
-  rc = setupStores(ctx, opt->precision, ts, false, slice, s, a);
+  const bool fused = fitIsFused(opt->precision, ts);
+  const int64_t slice = sliceTracks(
+      ctx, a.n, fused ? kFusedBytesPerTrack : storeBytesPerTrack(a, opt->precision, ts, false));
+  rc = fused ? setupFused(ctx, opt->precision, slice, s, a)
+             : setupStores(ctx, opt->precision, ts, false, slice, s, a);
   if (rc != KF_OK) return rc;
   const kf_schedule &sc = ctx->sched;
   KfdLaunch L{};
@@ -618,7 +724,10 @@ int kf_fit(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt, const kf_res
     e = launchSlices(a, L, opt->precision, res->track_states, slice, ctx->evm, s);
     ctx->phase_timed = slice >= a.n;
   }
-  if (e != hipSuccess) return fail(ctx, KF_E_HIP, "kf_fit: launch failed: %s", hipGetErrorString(e));
+  if (e != hipSuccess) {
+    ctx->redo_clean = false;
+    return fail(ctx, KF_E_HIP, "kf_fit: launch failed: %s", hipGetErrorString(e));
+  }
   KF_HIP(ctx, hipEventRecord(ctx->ev1, s));
   ctx->timed = true;
   return KF_OK;

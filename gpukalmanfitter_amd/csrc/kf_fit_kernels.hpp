@@ -1,0 +1,305 @@
+// kf_fit_kernels.hpp -- the batched Kalman-fit kernels for gfx950 and the
+// launcher of one precision, instantiated by kf_fit_fp64.hip and
+// kf_fit_mixed.hip.  The per-track program is TrackFit (kf_trackfit.hpp).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "kf_trackfit.hpp"
+
+namespace kfd {
+
+// Bases of the state stores of the 64-track chunk this wave works on.
+// Blocks are multiples of 64 work-items, so a wave covers exactly one chunk.
+template <typename S>
+struct ChunkBases {
+  double *d;
+  S *s;
+  double *f;
+  double *c;
+  KFD_INLINE ChunkBases(const FitArgs &a, int64_t i) {
+    const size_t chunk = __builtin_amdgcn_readfirstlane((uint32_t)(i >> 6));
+    const size_t per = (size_t)a.max_states * 64u;
+    d = a.tsd + chunk * per * KF_SD_N;
+    s = (S *)a.tss + chunk * per * KF_SS_N;
+    f = a.tsf ? a.tsf + chunk * per * KF_TS_STRIDE : nullptr;
+    c = a.tsc ? a.tsc + chunk * per * KF_CK_N : nullptr;
+  }
+};
+
+// Fits the track at position pos (pass FWD of the two kernels); `rank` is
+// the lane's index in the track's group of L lanes.
+template <typename S, bool FWD, int L, bool PS, int FK, int KEEP>
+KFD_INLINE void fitPosition(const FitArgs &a, int64_t local, uint32_t rank,
+                            const DevPlane *planes) {
+  const ChunkBases<S> cb(a, local);
+  if (local >= a.count) return;
+  const int64_t pos = a.first + local;
+  const int64_t i = a.order ? (int64_t)a.order[pos] : pos;
+  TrackFit<S, FWD, L, PS, false, FK, KEEP> tf(a, i, cb.d, cb.s, cb.f, cb.c,
+                                              (uint32_t)(local & 63), local);
+  tf.setRank(rank);
+  tf.pls = planes;
+  if constexpr (FWD)
+    tf.runForward();
+  else
+    tf.runBackward();
+}
+
+// One thread per position, or (persistent) resident waves that take
+// chunks_per_grab 64-position chunks at a time from a work-queue counter
+// until every chunk is taken; the grab is one vector atomic by lane 0.
+//
+// LDS = true: the block first copies the plane table (at most KF_LDS_PLANES
+// planes) to LDS and reads planes there.
+// PERS = false: one thread per position; true: the persistent work queue
+// (a separate instantiation, so the one-shot kernel does not carry the
+// queue loop's registers).
+// L: lanes per track (one-shot grid only): L consecutive lanes fit one
+// position, a wave covers 64 / L positions of one 64-position store chunk.
+// PS: store slots by plane position (kf_schedule.store_by_plane; one lane
+// per track).
+// FK, KEEP: the field kind and what is kept of the states.  A fit that asks
+// for neither track states nor checkpoints runs, in the mixed mode, on
+// (kFieldConst, kKeepStates) or (kFieldGrid, kKeepStates) for the batch's
+// field, so the step loop carries no code of the other field kind and the
+// filter none of the recording (FP64: kf_fused_kernel); every other one, and
+// plane tables read from global memory, on (kFieldAny, kKeepRecords).
+template <typename S, bool FWD, bool LDS, bool PERS, int L, bool PS, int FK, int KEEP>
+__global__ void __launch_bounds__(KF_BLOCK) kf_fit_kernel(FitArgs args) {
+  static_assert(L == 1 || !PERS, "lane groups run on the one-shot grid");
+  static_assert(L == 1 || !PS, "store slots by plane with one lane per track");
+  const DevPlane *planes = args.planes;
+  if constexpr (LDS) {
+    __shared__ DevPlane lds_planes[KF_LDS_PLANES];
+    const double *src = (const double *)args.planes;
+    double *dst = (double *)lds_planes;
+    const int words = args.n_planes * (int)(sizeof(DevPlane) / sizeof(double));
+    for (int w = threadIdx.x; w < words; w += KF_BLOCK) dst[w] = src[w];
+    __syncthreads();
+    planes = lds_planes;
+  }
+  const uint32_t lane = threadIdx.x & 63u;
+  if constexpr (!PERS) {
+    const int64_t t = (int64_t)blockIdx.x * KF_BLOCK + threadIdx.x;
+    fitPosition<S, FWD, L, PS, FK, KEEP>(args, t / L, (uint32_t)(t % L), planes);
+  } else {
+    const uint32_t nchunks = (uint32_t)((args.count + 63) >> 6);
+    const uint32_t grab = (uint32_t)args.chunks_per_grab;
+    uint32_t *q = args.queue + (FWD ? 0 : 1);
+    for (;;) {
+      uint32_t c0 = 0;
+      if (lane == 0) c0 = atomicAdd(q, grab);
+      c0 = (uint32_t)__shfl((int)c0, 0, 64);
+      if (c0 >= nchunks) break;
+      const uint32_t c1 = (c0 + grab < nchunks) ? c0 + grab : nchunks;
+      for (uint32_t c = c0; c < c1; ++c)
+        fitPosition<S, FWD, 1, PS, FK, KEEP>(args, (int64_t)c * 64 + lane, 0u, planes);
+    }
+  }
+}
+
+// The whole fit in one kernel, for FP64 fits that ask for neither track states
+// nor checkpoints: forward filter with the fixed-point smoother, then back to
+// the perigee (TrackFit::runFused).  Per-track state in registers (one wave
+// per SIMD), the smoother's sums in LDS (46 KB per block), the plane table in
+// dynamic LDS (PLDS) or global memory.  FK: the field kind, so the step loop
+// carries no code of the other one (either kind where the plane table is in
+// global memory).  PERS, L as in kf_fit_kernel.
+//
+// The mixed mode keeps the RTS kernels: its smoother starts from covariances
+// rounded to float, and the fixed-point sums, though no further from the
+// exact fit, do not round as the recursion over those does (1e-7 in the time
+// variance, single tracks 1e-4 mm in position where the perigee's on-surface
+// decision falls the other way).
+//
+// A track that the fixed-point smoother leaves to the RTS program (TrackFit::
+// fxSafe; 1 in 200,000 of the material workload) is fitted again by its own
+// wave while the others go on, over a store chunk it takes from a pool; when
+// the pool is used up it goes to the list of the redo kernel.  Waiting for
+// the redo kernel with all of them cost the material workload 0.9 ms per
+// call for a single track: the latency of one wave's fit of 40 planes.
+//
+// redoTrack is a call so that its code and registers stay out of the fit's;
+// it reads the kernel's arguments where the kernel finds them.
+template <typename S>
+__device__ __attribute__((noinline)) void redoTrack(const FitArgs *args, int64_t i,
+                                                    int64_t slot) {
+  const FitArgs &a = *args;
+  const uint32_t lane = (uint32_t)(slot & 63);
+  const ChunkBases<S> cb(a, slot);
+  {
+    TrackFit<S, true, 1, false, false, kFieldAny, kKeepStates> tf(a, i, cb.d, cb.s, nullptr, nullptr,
+                                                                  lane, slot);
+    tf.redoSlots();
+    tf.runForward();
+  }
+  {
+    TrackFit<S, false, 1, false, false, kFieldAny, kKeepStates> tf(a, i, cb.d, cb.s, nullptr,
+                                                                   nullptr, lane, slot);
+    tf.redoSlots();
+    tf.runBackward();
+  }
+}
+
+template <typename S, bool PLDS, int L, int FK>
+__global__ void __launch_bounds__(KF_FUSED_BLOCK) kf_fused_kernel(FitArgs args) {
+  using Fit = TrackFit<S, true, L, false, false, FK, kKeepFirst>;
+  __shared__ typename Fit::FxPair sums[Fit::kFxN * KF_FUSED_BLOCK];
+  extern __shared__ double lds_table[];
+  const DevPlane *planes = args.planes;
+  if constexpr (PLDS) {
+    const double *src = (const double *)args.planes;
+    const int words = args.n_planes * (int)(sizeof(DevPlane) / sizeof(double));
+    for (int w = threadIdx.x; w < words; w += KF_FUSED_BLOCK) lds_table[w] = src[w];
+    __syncthreads();
+    planes = (const DevPlane *)lds_table;
+  }
+  const int64_t t = (int64_t)blockIdx.x * KF_FUSED_BLOCK + threadIdx.x;
+  const int64_t local = t / L;
+  if (local >= args.count) return;
+  const int64_t pos = args.first + local;
+  const int64_t i = args.order ? (int64_t)args.order[pos] : pos;
+  bool redo;
+  {
+    Fit tf(args, i, nullptr, nullptr, nullptr, nullptr, threadIdx.x & 63u, local);
+    tf.setRank((uint32_t)(t % L));
+    tf.pls = planes;
+    tf.fx = sums + threadIdx.x;
+    redo = !tf.runFused() && tf.lead;
+  }
+  const uint64_t redoMask = __ballot(redo);
+  if (redoMask == 0) return;
+  const int first = __ffsll((unsigned long long)redoMask) - 1;
+  const int lane = (int)(threadIdx.x & 63u);
+  uint32_t chunk = 0;
+  if (lane == first) chunk = atomicAdd(args.redo, 1u);
+  chunk = (uint32_t)__shfl((int)chunk, first, 64);
+  if (!redo) return;
+  if ((int64_t)chunk * 64 < args.redo_lanes)
+    redoTrack<S>((const FitArgs *)__builtin_amdgcn_kernarg_segment_ptr(), i,
+                 (int64_t)chunk * 64 + lane);
+  else
+    args.redo[KF_REDO_LIST + atomicAdd(args.redo + 1, 1u)] = (uint32_t)local;
+}
+
+// The tracks that found no store chunk in the fused kernel, 64 at a time per
+// wave.  Usually the list is empty and the kernel ends at once.  The last
+// block zeroes the counters for the next fit (every block has read the count
+// when it takes its ticket).
+template <typename S>
+__global__ void __launch_bounds__(64) kf_redo_kernel(FitArgs args) {
+  const uint32_t n = __hip_atomic_load(args.redo + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const uint32_t lane = threadIdx.x;
+  const int64_t slot = (int64_t)blockIdx.x * 64 + lane;
+  for (int64_t e = slot; e < (int64_t)n; e += args.redo_lanes) {
+    const int64_t pos = args.first + (int64_t)args.redo[KF_REDO_LIST + e];
+    redoTrack<S>((const FitArgs *)__builtin_amdgcn_kernarg_segment_ptr(),
+                 args.order ? (int64_t)args.order[pos] : pos, slot);
+  }
+  __syncthreads();
+  if (lane == 0 && atomicAdd(args.redo + 2, 1u) == gridDim.x - 1) {
+    args.redo[0] = 0u;
+    args.redo[1] = 0u;
+    args.redo[2] = 0u;
+  }
+}
+
+// The launches of one precision.
+template <typename S>
+hipError_t launchFit(const FitArgs *args, hipStream_t stream, hipEvent_t between,
+                     const KfdLaunch *launch) {
+  const bool pers = launch && launch->persistent_blocks > 0;
+  const int lpt = (launch && !pers && launch->lanes_per_track > 1) ? launch->lanes_per_track : 1;
+  if (lpt != 1 && lpt != 2 && lpt != 4) return hipErrorInvalidValue;
+  const bool ps = launch && launch->store_by_plane != 0;
+  if (ps && lpt != 1) return hipErrorInvalidValue;
+  const int64_t blocks =
+      pers ? launch->persistent_blocks : (args->count * lpt + KF_BLOCK - 1) / KF_BLOCK;
+  const dim3 grid((unsigned)blocks), block(KF_BLOCK);
+  constexpr bool kFused = sizeof(S) == sizeof(double);
+  const bool rec = args->tsf != nullptr || args->tsc != nullptr;
+  if (!kFused || rec) {
+    const bool lds = args->n_planes <= KF_LDS_PLANES;
+#define KFD_LAUNCH2(FWD_, LDS_, PERS_, L_, PS_, FK_, KEEP_)                                     \
+  hipLaunchKernelGGL((kf_fit_kernel<S, FWD_, LDS_, PERS_, L_, PS_, FK_, KEEP_>), grid, block, 0, \
+                     stream, *args)
+#define KFD_LAUNCH1(FWD_, LDS_, FK_, KEEP_)                   \
+  do {                                                        \
+    if (pers && ps)                                           \
+      KFD_LAUNCH2(FWD_, LDS_, true, 1, true, FK_, KEEP_);     \
+    else if (pers)                                            \
+      KFD_LAUNCH2(FWD_, LDS_, true, 1, false, FK_, KEEP_);    \
+    else if (lpt == 1 && ps)                                  \
+      KFD_LAUNCH2(FWD_, LDS_, false, 1, true, FK_, KEEP_);    \
+    else if (lpt == 1)                                        \
+      KFD_LAUNCH2(FWD_, LDS_, false, 1, false, FK_, KEEP_);   \
+    else if (lpt == 2)                                        \
+      KFD_LAUNCH2(FWD_, LDS_, false, 2, false, FK_, KEEP_);   \
+    else                                                      \
+      KFD_LAUNCH2(FWD_, LDS_, false, 4, false, FK_, KEEP_);   \
+  } while (0)
+#define KFD_LAUNCH(FWD_)                                      \
+  do {                                                        \
+    if constexpr (!kFused) {                                  \
+      if (lds && !rec) {                                      \
+        if (args->field.grid)                                 \
+          KFD_LAUNCH1(FWD_, true, kFieldGrid, kKeepStates);   \
+        else                                                  \
+          KFD_LAUNCH1(FWD_, true, kFieldConst, kKeepStates);  \
+        break;                                                \
+      }                                                       \
+    }                                                         \
+    if (lds)                                                  \
+      KFD_LAUNCH1(FWD_, true, kFieldAny, kKeepRecords);       \
+    else                                                      \
+      KFD_LAUNCH1(FWD_, false, kFieldAny, kKeepRecords);      \
+  } while (0)
+    KFD_LAUNCH(true);
+    if (between) {
+      const hipError_t e = hipEventRecord(between, stream);
+      if (e != hipSuccess) return e;
+    }
+    // without smoothing the forward kernel finishes every track
+    if (args->smoothing) KFD_LAUNCH(false);
+#undef KFD_LAUNCH
+#undef KFD_LAUNCH1
+#undef KFD_LAUNCH2
+    return hipGetLastError();
+  }
+  if constexpr (kFused) {
+    const bool plds = args->n_planes <= KF_FUSED_LDS_PLANES;
+    const dim3 fgrid((unsigned)((args->count * lpt + KF_FUSED_BLOCK - 1) / KF_FUSED_BLOCK));
+    const unsigned table = plds ? (unsigned)(args->n_planes * sizeof(DevPlane)) : 0u;
+#define KFD_FUSED2(PLDS_, L_, FK_)                                                     \
+  hipLaunchKernelGGL((kf_fused_kernel<S, PLDS_, L_, FK_>), fgrid, dim3(KF_FUSED_BLOCK), table, \
+                     stream, *args)
+#define KFD_FUSED1(PLDS_, FK_)       \
+  do {                               \
+    if (lpt == 1)                    \
+      KFD_FUSED2(PLDS_, 1, FK_);     \
+    else if (lpt == 2)               \
+      KFD_FUSED2(PLDS_, 2, FK_);     \
+    else                             \
+      KFD_FUSED2(PLDS_, 4, FK_);     \
+  } while (0)
+    if (!plds)
+      KFD_FUSED1(false, kFieldAny);
+    else if (args->field.grid)
+      KFD_FUSED1(true, kFieldGrid);
+    else
+      KFD_FUSED1(true, kFieldConst);
+#undef KFD_FUSED1
+#undef KFD_FUSED2
+    if (between) {
+      const hipError_t e = hipEventRecord(between, stream);
+      if (e != hipSuccess) return e;
+    }
+    if (args->smoothing)
+      hipLaunchKernelGGL((kf_redo_kernel<S>), dim3((unsigned)(args->redo_lanes / 64)), dim3(64), 0,
+                         stream, *args);
+  }
+  return hipGetLastError();
+}
+
+}  // namespace kfd

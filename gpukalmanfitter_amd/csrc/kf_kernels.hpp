@@ -8,10 +8,24 @@
 #include "kf_device.hpp"
 
 #define KF_BLOCK 128  // multiple of 64: a wave covers one 64-track store chunk
-// Plane tables up to this size are copied to LDS by every fit block (plane
-// reads then wait on LDS only, not behind the store writes' vector-memory
-// count); larger tables are read from global memory.
+// Plane tables up to this size are copied to LDS by every block of the
+// recording fit kernels (plane reads then wait on LDS only, not behind the
+// store writes' vector-memory count); larger tables are read from global
+// memory.
 #define KF_LDS_PLANES 256
+#ifndef KF_FUSED_BLOCK
+#define KF_FUSED_BLOCK 128
+#endif
+// The same for the fused fit kernel, whose blocks also hold 46 KB of smoother
+// sums: the largest table with which two blocks (one wave per SIMD) still fit
+// the 160 KB of a compute unit.
+#define KF_FUSED_LDS_PLANES 224
+// Store chunks for tracks that the fused kernel hands to the RTS program, and
+// the memory they may take together.
+#define KF_REDO_WAVES 256
+#define KF_REDO_STORE_BYTES (256ull << 20)
+// doubles per track of the fused kernel's kept first state
+#define KF_FIRST_D 27
 
 // per-state store elements (see FitArgs).  A measured state sits in the
 // store slot of its plane's position in the track's surface sequence (when
@@ -119,7 +133,19 @@ struct FitArgs {
   int32_t persistent;
   int32_t chunks_per_grab;
   uint32_t *queue;
+  // Fused fits (FP64, no track states or checkpoints): carry_d holds the kept
+  // first states ([KF_FIRST_D][count]).  Tracks handed back to the RTS
+  // program use tsd, tss (redo_lanes slots, one store chunk per wave) and
+  // redo_d, redo_i ([KF_CARRY_D], [KF_CARRY_I][redo_lanes]).  redo[0]: store
+  // chunks taken by waves of the fused kernel itself, redo[1]: positions
+  // left in the list for the redo kernel, redo[2]: its ticket (all 0 between
+  // fits); redo[KF_REDO_LIST ...]: the positions.
+  double *redo_d;
+  int32_t *redo_i;
+  uint32_t *redo;
+  int64_t redo_lanes;
 };
+#define KF_REDO_LIST 64
 
 }  // namespace kfd
 
@@ -161,15 +187,26 @@ struct KfdLaunch {
   int32_t *order;          // [n] positions -> tracks (when sorting)
 };
 
-// Launches the fit of the positions args->first .. first + count - 1:
+// Launches the fit of the positions args->first .. first + count - 1.  With
+// track states or checkpoints (args->tsf, tsc) and in the mixed mode:
 // [work-queue reset] -> forward kernel -> record `between` (if not NULL) ->
-// smoother/back-propagation kernel -> track-state export (if
-// track_states_out is not NULL).  `launch` may be NULL (one thread per
+// smoother/back-propagation kernel (unless smoothing is off) -> track-state
+// export (if track_states_out is not NULL).  FP64 without them: [work-queue
+// reset] -> fused kernel -> record `between` -> redo kernel.  `launch` may be NULL (one thread per
 // track, identity order).  With a persistent grid, args->queue and
 // args->chunks_per_grab must be set; with sorting, args->order.
 extern "C" hipError_t kfd_launch_fit(const kfd::FitArgs *args, int precision, hipStream_t stream,
                                      double *track_states_out, hipEvent_t between,
                                      const KfdLaunch *launch);
+
+// The kernels of one precision (kf_fit_fp64.hip, kf_fit_mixed.hip).
+extern "C" hipError_t kfd_launch_fit_fp64(const kfd::FitArgs *args, hipStream_t stream,
+                                          hipEvent_t between, const KfdLaunch *launch);
+extern "C" hipError_t kfd_launch_fit_mixed(const kfd::FitArgs *args, hipStream_t stream,
+                                           hipEvent_t between, const KfdLaunch *launch);
+
+// Zeroes the redo counters (a new buffer, or after a failed call).
+extern "C" hipError_t kfd_launch_redo_reset(uint32_t *redo, hipStream_t stream);
 
 // The length sort of the whole batch (positions -> tracks into launch->order),
 // before the per-slice kfd_launch_fit calls.

@@ -29,9 +29,23 @@ enum { kResumeNone = 0, kResumePreLoop = 1, kResumeInLoop = 2, kResumePostLoop =
 // group run this program on the same data; the free transport matrix of each
 // RK step is built column by column across them, and only the group's first
 // lane writes to memory.
+//
+// KEEP: what a fit keeps of its measured states.
+//  kKeepRecords  the per-state store, from which the backward kernel runs the
+//                RTS smoother over all states, and the track-state records or
+//                adjoint checkpoints where asked for;
+//  kKeepStates   the store only (both record stores are null at compile time
+//                and their writes not in the code);
+//  kKeepFirst    only the smoothed state of the first measured surface is
+//                wanted (it is what propagates to the perigee): the forward
+//                pass carries a fixed-point smoother for it (below), nothing is
+//                stored per state, and one kernel runs the whole fit (runFused).
+enum { kKeepRecords = 0, kKeepStates = 1, kKeepFirst = 2 };
 template <typename S, bool FWD, int L = 1, bool PS = false, bool OOL = false, int FK = kFieldAny,
-          bool REC = true>
+          int KEEP = kKeepRecords>
 struct TrackFit {
+  static constexpr bool kRecords = KEEP == kKeepRecords;
+  static constexpr bool kStore = KEEP != kKeepFirst;
   static constexpr bool kMixed = sizeof(S) < sizeof(double);
   const FitArgs &a;
   const int64_t i;
@@ -105,8 +119,6 @@ struct TrackFit {
   }
   double chi2sum;
   double lc[3];  // perigee line point
-  double fpar[6];
-  double fcov[21];
 
   // quantities of the momentum used by every step, recomputed when p changes:
   // q/p, hypot(1, m/p) (dt/ds) and p hypot(1, m/p)
@@ -140,14 +152,23 @@ struct TrackFit {
   // slot of the forward -> backward hand-over record: the position within
   // the launch, so consecutive lanes use consecutive slots
   int64_t cpos;
+  // slots of the hand-over buffer (its field stride)
+  int64_t cslots;
+  int32_t *ciBase;
+  double *cdBase;
 
-  // REC = false: a build for fits that record neither track states nor
-  // checkpoints (both stores are then null at compile time, and their
-  // writes are not in the code)
   KFD_INLINE TrackFit(const FitArgs &args, int64_t idx, double *d_base, S *s_base, double *f_base,
                       double *c_base, uint32_t ln, int64_t carry_slot = 0)
-      : a(args), i(idx), tsd(d_base), tss(s_base), tsf(REC ? f_base : nullptr),
-        tsc(REC ? c_base : nullptr), pls(args.planes), lane(ln), cpos(carry_slot) {}
+      : a(args), i(idx), tsd(d_base), tss(s_base), tsf(kRecords ? f_base : nullptr),
+        tsc(kRecords ? c_base : nullptr), pls(args.planes), lane(ln), cpos(carry_slot), cslots(args.count),
+        ciBase(args.carry_i), cdBase(args.carry_d) {}
+
+  // The hand-over buffer of tracks fitted again after a fused fit.
+  KFD_INLINE void redoSlots() {
+    ciBase = a.redo_i;
+    cdBase = a.redo_d;
+    cslots = a.redo_lanes;
+  }
 
   // ------------------------------------------------------------ storage ----
   // Element f of state k: base[(k * F + f) * 64 + lane] -- a 32-bit lane
@@ -527,7 +548,7 @@ struct TrackFit {
     dtds = (S)dt;
 #pragma unroll
     for (int k = 0; k < 3; ++k) k4d[k] = (S)k4[k];
-    pathAcc = pathAcc + h;
+    if constexpr (kRecords) pathAcc = pathAcc + h;
     return true;
   }
 
@@ -691,6 +712,199 @@ struct TrackFit {
 #pragma unroll
       for (int k = 0; k < 3; ++k) out[k][c] = qop * r[k];
     }
+  }
+
+  // ------------------------------------------------ fixed-point smoother ----
+  // The smoothed state of the first measured surface (x0, C0), from sums that
+  // the forward pass accumulates.  With T the derivative of the current
+  // predicted spatial parameters (loc0, loc1, phi, theta, q/p) with respect to
+  // the filtered ones of state 0 -- T <- J T at a transport, T <- (I - K H) T
+  // at an update -- the covariance of state 0 with the current state is
+  // C_f0 T^T, and every later measurement (residual r, innovation S) adds
+  //   lambda += T^T H^T S^-1 r,   Lambda += T^T H^T S^-1 H T;
+  // at the end x0 = x_f0 + C_f0 lambda, C0 = C_f0 - C_f0 Lambda C_f0 (the
+  // fixed-point smoother of Kalman filtering, e.g. Anderson and Moore, Optimal
+  // Filtering, 1979, section 7.2).  In exact arithmetic it is the RTS
+  // recursion's result for state 0; the time parameter never acts on the
+  // spatial ones, so T is 5x5.  Per state ~210 multiply-adds and no memory,
+  // against ~1,100 and 512 B (mixed: 304 B) written and read back for the RTS
+  // step, whose 6x6 solve also loses more digits than the sums here.
+  //
+  // T, lambda and Lambda are double in both modes and sit in LDS (kFxN 16-byte
+  // pairs per lane, stride KF_FUSED_BLOCK: conflict-free 16-byte accesses), not in
+  // registers: they are used once per surface.
+  //
+  // Where the RTS recursion's discrete behaviour could show -- a phi wrap or a
+  // theta clamp of a smoothed state, a gain that is not finite, a covariance
+  // that is not clearly positive definite -- the track is handed to the RTS
+  // program instead (fxSafe, the redo list).
+  struct alignas(16) FxPair {
+    double a, b;
+  };
+  enum { kFxCol = 3, kFxSum = 15, kFxN = 23 };
+  FxPair *fx = nullptr;  // this lane's first pair
+  bool fxOk = true;
+  S fxVphi = (S)0, fxVth = (S)0;        // largest filtered variances of phi and theta
+  double fxPhi = 0.0, fxTheta = 0.0;    // largest |phi| and |theta - pi/2| of a filtered state
+
+  KFD_INLINE void fxLoad(int p, double &x, double &y) const {
+    const FxPair v = fx[p * KF_FUSED_BLOCK];
+    x = v.a;
+    y = v.b;
+  }
+  KFD_INLINE void fxStore(int p, double x, double y) const { fx[p * KF_FUSED_BLOCK] = FxPair{x, y}; }
+  // T column c: pairs 3c .. 3c + 2, the sixth element is lambda[c]
+  KFD_INLINE void fxInit() const {
+#pragma unroll
+    for (int c = 0; c < 5; ++c)
+#pragma unroll
+      for (int g = 0; g < 3; ++g)
+        fxStore(kFxCol * c + g, (c == 2 * g) ? 1.0 : 0.0, (c == 2 * g + 1) ? 1.0 : 0.0);
+#pragma unroll
+    for (int p = kFxSum; p < kFxN; ++p) fxStore(p, 0.0, 0.0);
+  }
+  // T <- J T (row 4 of J is e4; the time row does not enter)
+  KFD_INLINE void fxTransport(const S jb[6][6]) const {
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+      double t[6], n[4];
+#pragma unroll
+      for (int g = 0; g < 3; ++g) fxLoad(kFxCol * c + g, t[2 * g], t[2 * g + 1]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        double v = (double)jb[r][0] * t[0];
+#pragma unroll
+        for (int m = 1; m < 5; ++m) v = v + (double)jb[r][m] * t[m];
+        n[r] = v;
+      }
+      fxStore(kFxCol * c, n[0], n[1]);
+      fxStore(kFxCol * c + 1, n[2], n[3]);
+    }
+  }
+  // a measurement with gain K, S^-1 (i00, i01, i11) and u = S^-1 r: the sums,
+  // then T <- (I - K H) T
+  KFD_INLINE void fxMeasure(const double K0[6], const double K1[6], double i00, double i01,
+                            double i11, double u0, double u1) const {
+    double a[5], b[5];
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+      double t[6];
+#pragma unroll
+      for (int g = 0; g < 3; ++g) fxLoad(kFxCol * c + g, t[2 * g], t[2 * g + 1]);
+      a[c] = t[0];
+      b[c] = t[1];
+      t[5] = t[5] + (a[c] * u0 + b[c] * u1);
+#pragma unroll
+      for (int r = 0; r < 5; ++r) t[r] = t[r] - (K0[r] * a[c] + K1[r] * b[c]);
+#pragma unroll
+      for (int g = 0; g < 3; ++g) fxStore(kFxCol * c + g, t[2 * g], t[2 * g + 1]);
+    }
+    double l[16];
+#pragma unroll
+    for (int p = 0; p < 8; ++p) fxLoad(kFxSum + p, l[2 * p], l[2 * p + 1]);
+    int m = 0;
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+      const double w0 = i00 * a[c] + i01 * b[c], w1 = i01 * a[c] + i11 * b[c];
+#pragma unroll
+      for (int d = c; d < 5; ++d, ++m) l[m] = l[m] + (w0 * a[d] + w1 * b[d]);
+    }
+#pragma unroll
+    for (int p = 0; p < 8; ++p) fxStore(kFxSum + p, l[2 * p], l[2 * p + 1]);
+  }
+  // packed index of Lambda (c, d)
+  KFD_INLINE static constexpr int lidx(int c, int d) {
+    return (c <= d) ? (c * 5 - (c * (c - 1)) / 2 + (d - c)) : (d * 5 - (d * (d - 1)) / 2 + (c - d));
+  }
+  // the filtered state 0, kept from its update to the end of the forward pass
+  // in this position's column of the hand-over buffer: x_f0 (6), C_f0 (21)
+  KFD_INLINE void fxKeepFirst(const double xf[6]) const {
+    if (!lead) return;
+#pragma unroll
+    for (int m = 0; m < 6; ++m) cd(m) = xf[m];
+#pragma unroll
+    for (int m = 0; m < 21; ++m) cd(6 + m) = (double)cov[m];
+  }
+  KFD_INLINE void fxSmooth(double xs[6], double cs[21]) const {
+    double x0[6], c0[21];
+#pragma unroll
+    for (int m = 0; m < 6; ++m) x0[m] = cd(m);
+#pragma unroll
+    for (int m = 0; m < 21; ++m) c0[m] = cd(6 + m);
+    double lam[5], l[16];
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+      double t4;
+      fxLoad(kFxCol * c + 2, t4, lam[c]);
+    }
+#pragma unroll
+    for (int p = 0; p < 8; ++p) fxLoad(kFxSum + p, l[2 * p], l[2 * p + 1]);
+#pragma unroll
+    for (int r = 0; r < 6; ++r) {
+      double v = c0[sidx(r, 0)] * lam[0];
+#pragma unroll
+      for (int m = 1; m < 5; ++m) v = v + c0[sidx(r, m)] * lam[m];
+      xs[r] = x0[r] + v;
+      double w[5];  // row r of C_f0 Lambda
+#pragma unroll
+      for (int c = 0; c < 5; ++c) {
+        double q = c0[sidx(r, 0)] * l[lidx(0, c)];
+#pragma unroll
+        for (int m = 1; m < 5; ++m) q = q + c0[sidx(r, m)] * l[lidx(m, c)];
+        w[c] = q;
+      }
+#pragma unroll
+      for (int c = r; c < 6; ++c) {
+        double q = w[0] * c0[sidx(0, c)];
+#pragma unroll
+        for (int m = 1; m < 5; ++m) q = q + w[m] * c0[sidx(m, c)];
+        cs[sidx(r, c)] = c0[sidx(r, c)] - q;
+      }
+    }
+    correctParams(xs);
+  }
+  // Whether the start covariance is positive definite with room to spare: the
+  // pivots of the diagonally scaled matrix above the rounding of the mode.
+  KFD_INLINE bool fxDefinite() const {
+    const double low = kMixed ? 1e-5 : 1e-11;
+    double sc[6], Lo[6][6], W[6][6];
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) sc[k] = scaleOf((double)cov[sidx(k, k)]);
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+      double dj = (sc[j] * (double)cov[sidx(j, j)]) * sc[j];
+#pragma unroll
+      for (int k = 0; k < j; ++k) dj = dj - W[j][k] * Lo[j][k];
+      ok = ok && dj > low;
+      const double id = 1.0 / dj;
+#pragma unroll
+      for (int r = j + 1; r < 6; ++r) {
+        double w = (sc[r] * (double)cov[sidx(r, j)]) * sc[j];
+#pragma unroll
+        for (int k = 0; k < j; ++k) w = w - W[r][k] * Lo[j][k];
+        W[r][j] = w;
+        Lo[r][j] = w * id;
+      }
+    }
+    return ok;
+  }
+  // Whether the RTS recursion over this track's states is free of wraps,
+  // clamps and non-finite gains, so that its result for state 0 is this
+  // smoother's.  A smoothed state lies within sqrt(X) of the filtered one in
+  // units of the filtered errors, X the chi2 the later measurements add (it
+  // minimises that distance squared plus a sum of squares, whose minimum is
+  // X), so |phi| and |theta - pi/2| of every smoothed state are below the
+  // largest filtered value plus sqrt(largest filtered variance X); 2 % and
+  // 1e-6 cover rounding.  False on NaN.
+  KFD_INLINE bool fxSafe(const double xs[6], const double cs[21]) const {
+    bool ok = fxOk && fxPhi + (1.02 * sqrt((double)fxVphi * chi2sum) + 1e-6) < kPi &&
+              fxTheta + (1.02 * sqrt((double)fxVth * chi2sum) + 1e-6) < 0.5 * kPi;
+#pragma unroll
+    for (int m = 0; m < 6; ++m) ok = ok && fabs(xs[m]) < kDblMax;
+#pragma unroll
+    for (int m = 0; m < 21; ++m) ok = ok && fabs(cs[m]) < kDblMax;
+    return ok;
   }
 
   // ------------------------------------------------- bound-state transport ----
@@ -991,8 +1205,13 @@ struct TrackFit {
   }
 
   // PathLimitReached, StandardAborters.hpp:24-57
+  // The limit is DBL_MAX, and an accumulated path is below 2^970 (a step whose
+  // square overflows is refused), so DBL_MAX minus it rounds to DBL_MAX and the
+  // update changes no number (a NaN: surfaceReached): only the builds that
+  // record the path do it.
   KFD_INLINE bool pathLimit() {
     if (targetReached) return true;
+    if constexpr (!kRecords) return false;
     const double distance = (double)navDir * kDblMax - pathAcc;
     ss.update(distance, kAborter);
     const bool reached = distance * distance < a.target_tolerance * a.target_tolerance;
@@ -1026,6 +1245,9 @@ struct TrackFit {
       targetReached = true;
     } else {
       ss.update(nd * distance, kAborter);
+      // pathLimit's update follows and replaces a NaN by its limit
+      if constexpr (!kRecords)
+        if (distance != distance) ss.v[kAborter] = nd * kDblMax;
     }
     return onSurface;
   }
@@ -1168,8 +1390,8 @@ struct TrackFit {
     boundStatePlane(pl, xp, jb);
     // predicted parameters and the transport Jacobian to the store, with the
     // slot of the state two measurements back (the smoother's look-ahead)
-    storePar(s, KF_SD_XP, xp);
-    {
+    if constexpr (kStore) {
+      storePar(s, KF_SD_XP, xp);
       S jv[KF_SS_CF - KF_SS_J];
 #pragma unroll
       for (int r = 0; r < 6; ++r)
@@ -1180,6 +1402,11 @@ struct TrackFit {
 #pragma unroll
       for (int m = KF_SS_LINK + 1; m < KF_SS_CF - KF_SS_J; ++m) jv[m] = (S)0;
       storeS<KF_SS_CF - KF_SS_J>(s, KF_SS_J, jv);
+    } else {
+      if (k == 0)
+        fxInit();
+      else
+        fxTransport(jb);
     }
     if (tsf && lead) {
       storeBoundF(k, KF_TS_PREDICTED, xp, cov);
@@ -1199,6 +1426,14 @@ struct TrackFit {
     const double r0 = m0 - xp[0], r1 = m1 - xp[1];
     const double chi2 = r0 * (i00 * r0 + i01 * r1) + r1 * (i10 * r0 + i11 * r1);
     double xf[6];
+    if constexpr (!kStore) {
+      // the predicted covariance and the hit's are positive definite, and the
+      // hit is not so much more precise that the update loses definiteness
+      fxOk = fxOk && (S)0 < cov[sidx(0, 0)] && (S)0 < cov[sidx(1, 1)] && (S)0 < cov[sidx(2, 2)] &&
+             (S)0 < cov[sidx(3, 3)] && (S)0 < cov[sidx(4, 4)] && (S)0 < cov[sidx(5, 5)] &&
+             V00 > 1e-12 * S00 && V11 > 1e-12 * S11 &&
+             V00 * V11 - V01 * V01 > 1e-12 * (V00 * V11);
+    }
     // outlier finder: above the cut the state keeps its prediction (no
     // update, the covariance stays the predicted one) and stays out of the
     // chi2 sum and ndf; 0 disables it (the reference's void finder)
@@ -1215,6 +1450,9 @@ struct TrackFit {
     }
 #pragma unroll
     for (int r = 0; r < 6; ++r) xf[r] = xp[r] + (K0[r] * r0 + K1[r] * r1);
+    if constexpr (!kStore) {
+      if (k > 0) fxMeasure(K0, K1, i00, i01, i11, i00 * r0 + i01 * r1, i10 * r0 + i11 * r1);
+    }
     // the update in place on cov: rows 0 and 1 of the result go to t01 first
     // (every entry reads the old rows 0 and 1), then rows 2..5 overwrite
     // cov, then rows 0 and 1 are written back
@@ -1266,8 +1504,19 @@ struct TrackFit {
     for (int c = 1; c < 6; ++c) cov[sidx(1, c)] = (S)t01[5 + c];
     chi2sum = chi2sum + chi2;
     }
+    if constexpr (!kStore) {
+      const double ap = fabs(xf[2]), at = fabs(xf[3] - 0.5 * kPi);
+      fxPhi = (ap < fxPhi) ? fxPhi : ap;
+      fxTheta = (at < fxTheta) ? fxTheta : at;
+      fxVphi = (cov[sidx(2, 2)] < fxVphi) ? fxVphi : cov[sidx(2, 2)];
+      fxVth = (cov[sidx(3, 3)] < fxVth) ? fxVth : cov[sidx(3, 3)];
+    }
     correctParams(xf);
-    storePar(s, KF_SD_XF, xf);
+    if constexpr (kStore) {
+      storePar(s, KF_SD_XF, xf);
+    } else {
+      if (k == 0) fxKeepFirst(xf);
+    }
     if (tsf && lead) {
       storeBoundF(k, KF_TS_FILTERED, xf, cov);
       *recF(k, KF_TS_CHI2) = chi2;
@@ -1276,14 +1525,18 @@ struct TrackFit {
     // diagonal entries in which the covariance the next transport starts
     // from differs from it
     S cm[KF_SS_N - KF_SS_CF];
+    if constexpr (kStore) {
 #pragma unroll
-    for (int m = 0; m < 21; ++m) cm[m] = cov[m];
+      for (int m = 0; m < 21; ++m) cm[m] = cov[m];
+    }
     updateFromFiltered(pl, xf, xp);
     material(pl);
-    cm[KF_SS_MD - KF_SS_CF + 0] = cov[sidx(2, 2)];
-    cm[KF_SS_MD - KF_SS_CF + 1] = cov[sidx(3, 3)];
-    cm[KF_SS_MD - KF_SS_CF + 2] = cov[sidx(4, 4)];
-    storeS<KF_SS_N - KF_SS_CF>(s, KF_SS_CF, cm);
+    if constexpr (kStore) {
+      cm[KF_SS_MD - KF_SS_CF + 0] = cov[sidx(2, 2)];
+      cm[KF_SS_MD - KF_SS_CF + 1] = cov[sidx(3, 3)];
+      cm[KF_SS_MD - KF_SS_CF + 2] = cov[sidx(4, 4)];
+      storeS<KF_SS_N - KF_SS_CF>(s, KF_SS_CF, cm);
+    }
     if (tsc) saveCheckpoint(k);
     if constexpr (PS) {
       slotPrev = slotLast;
@@ -1545,71 +1798,47 @@ struct TrackFit {
     return true;
   }
 
-  // Actor::operator(), KalmanFitter.hpp:216-273.  Forward kernel: filter and
-  // the finalisation check; returns true where finalize() must run (the
-  // backward kernel does it).  Backward kernel: only the post-finalisation
-  // part can act (smoothed is set).
+  // Actor::operator(), KalmanFitter.hpp:216-273, of the forward pass: filter
+  // and the finalisation check; returns true where finalize() must run.
   KFD_INLINE bool actor() {
-    if constexpr (FWD) {
-      if (cur >= 0 && !smoothed && !finished) {
-        if (!filter(cur)) result = false;
-      }
-      if (finalizeCond()) {
-        if (!a.smoothing) {
-          finished = true;
-        } else {
-          return true;
-        }
-      }
-      return false;
-    } else {
-      actorPost();
-      return false;
+    if (cur >= 0 && !smoothed && !finished) {
+      if (!filter(cur)) result = false;
     }
+    if (finalizeCond()) {
+      if (!a.smoothing) {
+        finished = true;
+      } else {
+        return true;
+      }
+    }
+    return false;
   }
 
+  // The same of the backward pass: only the part after the finalisation can
+  // act (smoothed is set).
   KFD_INLINE void actorPost() {
     if (smoothed && !finished && surfaceReached()) {
-      boundStateLine(fpar);
-#pragma unroll
-      for (int m = 0; m < 21; ++m) fcov[m] = cov[m];
+      double par[6];
+      boundStateLine(par);
+      writeFit(par, cov);
       finished = true;
     }
   }
 
-  // The propagation loop (Propagator.ipp:39-69) with the cheap iterations in
-  // an inner loop.  Returns true if the forward kernel must hand over to the
-  // backward kernel (finalize due inside the actor).
-  KFD_INLINE bool loop(int &steps, bool &terminated) {
+  // Iterations of the propagation loop (Propagator.ipp:39-69) in which the
+  // actor has nothing to do.  Stops where it has (true), or where the loop
+  // ends: terminated by an aborter or after max_steps.
+  template <bool F>
+  KFD_INLINE bool cheapSteps(int &steps, bool &terminated) {
     while (steps < a.max_steps) {
-      bool event = false;
-      while (steps < a.max_steps) {
-        step();
-        navStatus();
-        if (FWD && cur >= 0 && !smoothed && !finished) {
-          event = true;
-          break;
-        }
-        if (FWD && finalizeCond()) {
-          event = true;
-          break;
-        }
-        if (!FWD && smoothed && !finished && surfaceReached()) {
-          event = true;
-          break;
-        }
-        if (kalmanAbort() || pathLimit()) {
-          terminated = true;
-          break;
-        }
-        navTarget();
-        ++steps;
-      }
-      if (!event) break;
-      if (actor()) return true;
+      step();
+      navStatus();
+      if (F && cur >= 0 && !smoothed && !finished) return true;
+      if (F && finalizeCond()) return true;
+      if (!F && smoothed && !finished && surfaceReached()) return true;
       if (kalmanAbort() || pathLimit()) {
         terminated = true;
-        break;
+        return false;
       }
       navTarget();
       ++steps;
@@ -1625,8 +1854,8 @@ struct TrackFit {
   };
   enum { kCD_q = 0, kCD_J = 1, kCD_k4 = 26, kCD_dtds = 29, kCD_N = 30 };
   static_assert(kCI_N == KF_CARRY_I && kCD_N == KF_CARRY_D, "hand-over record layout");
-  KFD_INLINE int32_t &ci(int f) const { return a.carry_i[(size_t)f * a.count + cpos]; }
-  KFD_INLINE double &cd(int f) const { return a.carry_d[(size_t)f * a.count + cpos]; }
+  KFD_INLINE int32_t &ci(int f) const { return ciBase[(size_t)f * cslots + cpos]; }
+  KFD_INLINE double &cd(int f) const { return cdBase[(size_t)f * cslots + cpos]; }
 
   KFD_INLINE void saveCarry(int resume, int steps, bool terminated) const {
     if (!lead) return;
@@ -1705,15 +1934,32 @@ struct TrackFit {
     return status;
   }
 
-  KFD_INLINE void writeFinal(uint32_t status) const {
+  // The fitted parameters and covariance go out where they are computed (27
+  // doubles that would otherwise stay in registers through the last steps).
+  template <typename T>
+  KFD_INLINE void writeFit(const double par[6], const T c[21]) const {
     if (!lead) return;
     if (a.out_params)
 #pragma unroll
-      for (int k = 0; k < 6; ++k) a.out_params[(size_t)k * a.n + i] = fpar[k];
+      for (int k = 0; k < 6; ++k) a.out_params[(size_t)k * a.n + i] = par[k];
     if (a.out_cov)
 #pragma unroll
-      for (int k = 0; k < 21; ++k) a.out_cov[(size_t)k * a.n + i] = fcov[k];
-    if (a.out_status) a.out_status[i] = status;
+      for (int k = 0; k < 21; ++k) a.out_cov[(size_t)k * a.n + i] = (double)c[k];
+  }
+  // The end of a track: its status, and zeros where no fit came out.
+  // `written`: writeFit has run.
+  KFD_INLINE void writeFinal(uint32_t status, bool written) const {
+    if (!written) {
+      const double par[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+      const double c[21] = {0.0};
+      writeFit(par, c);
+    }
+    if (lead && a.out_status) a.out_status[i] = status;
+  }
+
+  KFD_INLINE void loadPerigee() {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) lc[k] = a.perigee[(size_t)k * a.n + i];
   }
 
   KFD_INLINE void loadTrack() {
@@ -1724,20 +1970,15 @@ struct TrackFit {
     pfValid = false;
     seqFirst = a.seq_first[i];
     size = a.seq_count[i];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) lc[k] = a.perigee[(size_t)k * a.n + i];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) fpar[k] = 0.0;
-#pragma unroll
-    for (int k = 0; k < 21; ++k) fcov[k] = 0.0;
+    loadPerigee();
     smoothed = finished = smootherNaN = false;
     cur = -1;
     targetReached = false;
   }
 
-  // Forward kernel body: Propagator::propagate (Propagator.ipp:3-96) up to
-  // the finalisation.
-  KFD_INLINE void runForward() {
+  // The forward pass: Propagator::propagate (Propagator.ipp:3-96) up to the
+  // finalisation.  Returns where the finalisation is due (kResume*).
+  KFD_INLINE int forwardPass(int &steps, bool &terminated, bool &bad) {
     loadTrack();
     double pv[6];
 #pragma unroll
@@ -1754,25 +1995,37 @@ struct TrackFit {
     next = 0;
     navBreak = false;
     stepFailed = false;
-    bool terminated = false;
-    int steps = 0;
+    terminated = false;
+    steps = 0;
+    bad = size <= 0 || seqFirst < 0 || seqFirst + size > a.n_planes || h0 < 0 || h1 <= h0 ||
+          h1 > a.n_hits || pv[4] == 0.0 || a.max_states < 1;
+    // Before the loop, in it and after it the actor is called from one place
+    // (its code is most of the kernel): `at` says which of the three this is.
     int resume = kResumeNone;
-    const bool bad = size <= 0 || seqFirst < 0 || seqFirst + size > a.n_planes || h0 < 0 ||
-                     h1 <= h0 || h1 > a.n_hits || pv[4] == 0.0 || a.max_states < 1;
     if (!bad) {
+      if constexpr (!kStore) fxOk = fxDefinite();
       prefetchHit();
       start(pv);
       navStatus();
-      if (actor()) {
-        resume = kResumePreLoop;
-      } else {
-        if (!(kalmanAbort() || pathLimit())) {
-          navTarget();
-          if (loop(steps, terminated)) resume = kResumeInLoop;
+      int at = kResumePreLoop;
+      for (;;) {
+        if (actor()) {
+          resume = at;
+          break;
         }
-        if (resume == kResumeNone) {
+        if (at == kResumePostLoop) break;
+        bool more = !(kalmanAbort() || pathLimit());
+        if (more) {
+          navTarget();
+          if (at == kResumeInLoop) ++steps;
+          at = kResumeInLoop;
+          more = cheapSteps<true>(steps, terminated);
+        } else if (at == kResumeInLoop) {
+          terminated = true;
+        }
+        if (!more) {
+          at = kResumePostLoop;
           if (!terminated) navBreak = true;
-          if (actor()) resume = kResumePostLoop;
         }
       }
     }
@@ -1781,57 +2034,96 @@ struct TrackFit {
       if (a.out_ndf) a.out_ndf[i] = 2 * (measured - outliers);
       if (a.out_nmeas) a.out_nmeas[i] = measured;
     }
+    return resume;
+  }
+
+  // The state of the smoothed first surface (xs, cs), from which the
+  // propagation back to the perigee starts.
+  KFD_INLINE void fromSmoothed(const double xs[6], const double cs[21]) {
+    updateFromBound(plane(firstPlane), xs);
+#pragma unroll
+    for (int m = 0; m < 21; ++m) cov[m] = (S)cs[m];
+    navDir = -1;
+    moved();
+    ss.init(-1.0 * fabs(a.max_step_size));
+    pathAcc = 0.0;
+  }
+
+  // The rest of the actor call that finalised, and the propagation back to
+  // the perigee; the actor is called from one place, as in forwardPass.
+  KFD_INLINE void backwardPass(int resume, int steps, bool terminated) {
+    int at = resume;
+    for (;;) {
+      actorPost();
+      if (at == kResumePostLoop) break;
+      bool more = !(kalmanAbort() || pathLimit());
+      if (more) {
+        navTarget();
+        if (at == kResumeInLoop) ++steps;
+        at = kResumeInLoop;
+        more = cheapSteps<false>(steps, terminated);
+      } else if (at == kResumeInLoop) {
+        terminated = true;
+      }
+      if (!more) {
+        at = kResumePostLoop;
+        if (!terminated) navBreak = true;
+      }
+    }
+    writeFinal(statusBits(steps, terminated), finished);
+  }
+
+  // Forward kernel body (with the store).
+  KFD_INLINE void runForward() {
+    int steps;
+    bool terminated, bad;
+    const int resume = forwardPass(steps, terminated, bad);
     if (resume != kResumeNone) {
       saveCarry(resume, steps, terminated);
     } else {
       if (lead) ci(kCI_resume) = kResumeNone;
-      writeFinal(bad ? KF_STATUS_BAD_INPUT : statusBits(steps, terminated));
+      writeFinal(bad ? KF_STATUS_BAD_INPUT : statusBits(steps, terminated), false);
     }
   }
 
-  // Backward kernel body: Actor::finalize (KalmanFitter.hpp:360-393), the
-  // rest of that actor call, and the propagation back to the perigee.
+  // Backward kernel body (with the store): Actor::finalize (KalmanFitter.hpp:
+  // 360-393) and what follows it.
   KFD_INLINE void runBackward() {
     int steps = 0;
     bool terminated = false;
     loadTrack();
     const int resume = loadCarry(steps, terminated);
     if (resume == kResumeNone) return;
-    // finalize
     smoothed = true;
     double xs[6], cs[21];
-    if (smooth(xs, cs)) {
-      updateFromBound(plane(firstPlane), xs);
-#pragma unroll
-      for (int m = 0; m < 21; ++m) cov[m] = (S)cs[m];
-      navDir = -1;
-      moved();
-      ss.init(-1.0 * fabs(a.max_step_size));
-      pathAcc = 0.0;
-    } else {
+    if (smooth(xs, cs))
+      fromSmoothed(xs, cs);
+    else
       result = false;
-    }
     loadCarryJacobian();
-    actorPost();
-    if (resume == kResumePreLoop) {
-      if (!(kalmanAbort() || pathLimit())) {
-        navTarget();
-        loop(steps, terminated);
-      }
-      if (!terminated) navBreak = true;
-      actor();
-    } else if (resume == kResumeInLoop) {
-      if (kalmanAbort() || pathLimit()) {
-        terminated = true;
-      } else {
-        navTarget();
-        ++steps;
-        loop(steps, terminated);
-      }
-      if (!terminated) navBreak = true;
-      actor();
+    backwardPass(resume, steps, terminated);
+  }
+
+  // The whole fit with the fixed-point smoother (kKeepFirst).  False: the
+  // track is left to the RTS program (its outputs are not final).
+  KFD_INLINE bool runFused() {
+    int steps;
+    bool terminated, bad;
+    const int resume = forwardPass(steps, terminated, bad);
+    if (resume == kResumeNone) {
+      writeFinal(bad ? KF_STATUS_BAD_INPUT : statusBits(steps, terminated), false);
+      return true;
     }
-    writeFinal(statusBits(steps, terminated));
+    double xs[6], cs[21];
+    fxSmooth(xs, cs);
+    if (!fxSafe(xs, cs)) return false;
+    smoothed = true;
+    cur = -1;
+    targetReached = false;
+    loadPerigee();  // again: it need not stay in registers through the forward pass
+    fromSmoothed(xs, cs);
+    backwardPass(resume, steps, terminated);
+    return true;
   }
 };
 

@@ -223,7 +223,7 @@ int kf_fit(kf_ctx *ctx, const kf_tracks *tracks, const kf_options *opt,
 /* kf_fit without any device allocation.  No counterpart in the reference:
  * for callers that cannot allocate (code under HIP graph capture, serving
  * loops, harnesses that forbid hipMalloc).  The working storage (smoother
- * store, hand-over records, track-state staging) comes from a fixed
+ * store, hand-over and kept-state records, track-state staging) comes from a fixed
  * device-resident workspace of KF_NOALLOC_WORKSPACE_BYTES that the library
  * holds on every device it runs on until the process ends; batches larger
  * than it holds run in consecutive slices of 64-track multiples, with the
@@ -300,10 +300,13 @@ int kf_set_memory_budget(kf_ctx *ctx, uint64_t bytes);
  * on the launch stream); < 0 if unknown. */
 double kf_last_kernel_ms(const kf_ctx *ctx);
 
-/* The same split at the hand-over between the two kernels of a fit: the
+/* The same split at the hand-over between the kernels of a fit: the
  * forward filter (up to the reference's finalize()) and the smoother plus
  * back-propagation to the perigee.  The backward time includes the
- * track-state export when track states were requested.  No reference
+ * track-state export when track states were requested.  An FP64 fit without
+ * track states runs as one kernel: its time is the forward time, and the
+ * backward time is that of the pass over tracks it left for the RTS smoother
+ * (none as a rule).  No reference
  * counterpart (the reference times the whole batch from the host,
  * Run/GPU/KalmanFitterGPUTest.cu:382-513). */
 int kf_last_phase_ms(const kf_ctx *ctx, double *forward_ms, double *backward_ms);

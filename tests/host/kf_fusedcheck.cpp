@@ -1,0 +1,32 @@
+// kf_fusedcheck.cpp -- CPU build of the fused fit program (TrackFit with the
+// fixed-point smoother), for the tests: the same source the GPU runs, one
+// track at a time.  Test infrastructure only: the library never loads it.
+#include "kf_hostcheck.cpp"
+
+extern "C" {
+
+// The fit of every track by the fused program: params [6][n], cov [21][n],
+// chi2, n_measured, status [n], and redo [n], nonzero for a track that it
+// leaves to the RTS program (its params, cov and status are not set).
+int kfh_fit_fused(const kf_plane *planes, int32_t n_planes, const kfh_field *f,
+                  const kf_tracks *tr, const kf_options *opt, double *params, double *cov,
+                  double *chi2, int32_t *n_measured, uint32_t *status, int32_t *redo) {
+  Host h(planes, n_planes, f, tr, opt, true);
+  h.a.out_params = params;
+  h.a.out_cov = cov;
+  h.a.out_chi2 = chi2;
+  h.a.out_nmeas = n_measured;
+  h.a.out_status = status;
+  h.a.out_ndf = nullptr;
+  using Fit = TrackFit<double, true, 1, false, false, kFieldAny, kKeepFirst>;
+  std::vector<Fit::FxPair> sums((size_t)Fit::kFxN * KF_FUSED_BLOCK);
+  for (int64_t i = 0; i < tr->n_tracks; ++i) {
+    Fit tf(h.a, i, nullptr, nullptr, nullptr, nullptr, 0u, i);
+    tf.pls = h.planes.data();
+    tf.fx = sums.data();
+    redo[i] = tf.runFused() ? 0 : 1;
+  }
+  return 0;
+}
+
+}  // extern "C"
