@@ -26,9 +26,9 @@ namespace kfd {
 enum { kResumeNone = 0, kResumePreLoop = 1, kResumeInLoop = 2, kResumePostLoop = 3 };
 
 // L: lanes per track (1, 2 or 4; kf_device.hpp, lane groups).  The lanes of a
-// group run this program on the same data; the free transport matrix of each
-// RK step is built column by column across them, and only the group's first
-// lane writes to memory.
+// group run this program on the same data; in the mixed mode the free
+// transport matrix of each RK step is built column by column across them, and
+// only the group's first lane writes to memory.
 //
 // KEEP: what a fit keeps of its measured states.
 //  kKeepRecords  the per-state store, from which the backward kernel runs the
@@ -121,16 +121,30 @@ struct TrackFit {
   double lc[3];  // perigee line point
 
   // quantities of the momentum used by every step, recomputed when p changes:
-  // q/p, hypot(1, m/p) (dt/ds) and p hypot(1, m/p)
-  double cacheP = -1.0, cacheQ = 0.0, cacheQop = 0.0, cacheDtds = 0.0, cacheDen = 0.0;
+  // q/p, sqrt(1 + (m/p)^2) (dt/ds), and the transport's d(time)/d(q/p) per
+  // unit step, m^2 q / (p sqrt(1 + (m/p)^2)) times q^2 = 1
+  double cacheP = -1.0, cacheQ = 0.0, cacheQop = 0.0, cacheDtds = 0.0, cacheD37 = 0.0;
   KFD_INLINE void momentumCache() {
     if (p != cacheP || q != cacheQ) {
       cacheP = p;
       cacheQ = q;
-      cacheQop = q / p;
-      cacheDtds = hypot(1.0, a.mass / p);
-      cacheDen = p * cacheDtds;
+      cacheQop = divD(q, p);
+      const double mp = divD(a.mass, p);
+      double is;
+      rootD(1.0 + mp * mp, cacheDtds, is);
+      cacheD37 = (a.mass * q) * (mp * is);
     }
+  }
+  // The direction and angles after the last update (or of the start
+  // parameters): the angles at the next plane follow from the rotation
+  // between the two directions (planeAngles).
+  double refPhi = 0.0, refTheta = 0.0, refX = 0.0, refY = 0.0, refZ = 0.0;
+  KFD_INLINE void setReference(const double par[6]) {
+    refPhi = par[2];
+    refTheta = par[3];
+    refX = dir[0];
+    refY = dir[1];
+    refZ = dir[2];
   }
   // the last plane intersection computed by surfaceStatus (path length along
   // the direction, denominator n.d): navStatus and navTarget of one
@@ -376,6 +390,8 @@ struct TrackFit {
     p = mn;
     q = charge;
     t = pc[5];
+    setReference(pc);
+    if (pc[3] != pv[3]) refX = refY = 0.0;  // theta was clamped: not the direction's
     navDir = 1;
     moved();
     ss.init(1.0 * fabs(a.max_step_size));
@@ -470,6 +486,12 @@ struct TrackFit {
   // -------------------------------------------------------------- step ----
   // EigenStepper::step, EigenStepper.ipp:226-332, with the transport of
   // transportMatrix (:50-124) applied to J directly.
+  //
+  // In a constant field the stages are polynomials of x -> x x w, w = q/p B,
+  // on the direction: with v1 = d x w, v2 = v1 x w and v2 x w = -w^2 v1,
+  //   k1 = v1,  k2 = v1 + h/2 v2,  k3 = (1 - c) v1 + h/2 v2,
+  //   k4 = (1 - 2c) v1 + h (1 - c) v2,  c = (h w / 2)^2,
+  // and the error estimate k1 - k2 - k3 + k4 is -c (v1 + h v2).
   KFD_INLINE bool step() {
     double B1[3], Bm[3], Bl[3];
     field(pos, B1);
@@ -477,44 +499,65 @@ struct TrackFit {
     momentumCache();
     const double qop = cacheQop;
     double k1[3], k2[3], k3[3], k4[3];
-    cross(dir, B1, k1);
+    double u1[3], u2[3], v2[3], w[3], w2 = 0.0, c = 0.0;  // constant field
+    if constexpr (FK == kFieldConst) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) k1[k] = qop * k1[k];
+      for (int k = 0; k < 3; ++k) w[k] = qop * B1[k];
+      w2 = dot3(w, w);
+      cross(dir, B1, u1);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) k1[k] = qop * u1[k];
+      cross(u1, w, u2);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) v2[k] = qop * u2[k];
+    } else {
+      cross(dir, B1, k1);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) k1[k] = qop * k1[k];
+    }
     double err = 0.0;
     unsigned nTrials = 0;
     for (;;) {
       const double h = ss.get();
       const double h2 = h * h;
       const double half_h = h * 0.5;
-      double p1[3], tv[3];
+      if constexpr (FK == kFieldConst) {
+        c = (0.25 * h2) * w2;
+        double e1 = fabs(k1[0] + h * v2[0]);
 #pragma unroll
-      for (int k = 0; k < 3; ++k) p1[k] = pos[k] + half_h * dir[k] + (h2 * 0.125) * k1[k];
-      field(p1, Bm);
+        for (int k = 1; k < 3; ++k) e1 = e1 + fabs(k1[k] + h * v2[k]);
+        err = h2 * (c * e1);
+      } else {
+        double p1[3], tv[3];
 #pragma unroll
-      for (int k = 0; k < 3; ++k) tv[k] = dir[k] + half_h * k1[k];
-      cross(tv, Bm, k2);
+        for (int k = 0; k < 3; ++k) p1[k] = pos[k] + half_h * dir[k] + (h2 * 0.125) * k1[k];
+        field(p1, Bm);
 #pragma unroll
-      for (int k = 0; k < 3; ++k) k2[k] = qop * k2[k];
+        for (int k = 0; k < 3; ++k) tv[k] = dir[k] + half_h * k1[k];
+        cross(tv, Bm, k2);
 #pragma unroll
-      for (int k = 0; k < 3; ++k) tv[k] = dir[k] + half_h * k2[k];
-      cross(tv, Bm, k3);
+        for (int k = 0; k < 3; ++k) k2[k] = qop * k2[k];
 #pragma unroll
-      for (int k = 0; k < 3; ++k) k3[k] = qop * k3[k];
+        for (int k = 0; k < 3; ++k) tv[k] = dir[k] + half_h * k2[k];
+        cross(tv, Bm, k3);
 #pragma unroll
-      for (int k = 0; k < 3; ++k) p1[k] = pos[k] + h * dir[k] + (h2 * 0.5) * k3[k];
-      field(p1, Bl);
+        for (int k = 0; k < 3; ++k) k3[k] = qop * k3[k];
 #pragma unroll
-      for (int k = 0; k < 3; ++k) tv[k] = dir[k] + h * k3[k];
-      cross(tv, Bl, k4);
+        for (int k = 0; k < 3; ++k) p1[k] = pos[k] + h * dir[k] + (h2 * 0.5) * k3[k];
+        field(p1, Bl);
 #pragma unroll
-      for (int k = 0; k < 3; ++k) k4[k] = qop * k4[k];
-      double e1 = 0.0;
+        for (int k = 0; k < 3; ++k) tv[k] = dir[k] + h * k3[k];
+        cross(tv, Bl, k4);
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const double e = k1[k] - k2[k] - k3[k] + k4[k];
-        e1 = (k == 0) ? fabs(e) : e1 + fabs(e);
+        for (int k = 0; k < 3; ++k) k4[k] = qop * k4[k];
+        double e1 = 0.0;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const double e = k1[k] - k2[k] - k3[k] + k4[k];
+          e1 = (k == 0) ? fabs(e) : e1 + fabs(e);
+        }
+        err = h2 * e1;
       }
-      err = h2 * e1;
       err = (err < 1e-20) ? 1e-20 : err;
       if (err <= a.tolerance) break;
       // std::min(std::max(0.25, x), 4.) with its NaN behaviour: a NaN error
@@ -531,17 +574,44 @@ struct TrackFit {
     // propagationTime, EigenStepper.ipp:36-47
     const double dt = cacheDtds;
     t = t + h * dt;
-    transport(B1, Bm, Bl, k1, k2, k3, h, qop);
-    // h^2/6 and h/6 as products with 1/6, one division for the
-    // normalisation (within an ulp of the quotients)
     const double h6 = h * (1.0 / 6.0);
     const double hh6 = h * h6;
+    // b row of J <- D J
+    b = b + (S)(h * cacheD37);
+    if constexpr (FK == kFieldConst && !kMixed) {
+      transportConst(w, u1, u2, h, h6, hh6, c);
+    } else if constexpr (!kMixed) {
+      transportColumns(B1, Bm, Bl, k1, k2, k3, h, h6, hh6, qop);
+    } else {
+      if constexpr (FK == kFieldConst) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) pos[k] = pos[k] + h * dir[k] + hh6 * (k1[k] + k2[k] + k3[k]);
+        for (int k = 0; k < 3; ++k) {
+          k2[k] = k1[k] + (0.5 * h) * v2[k];
+          k3[k] = k2[k] - c * k1[k];
+          Bm[k] = Bl[k] = B1[k];
+        }
+      }
+      transport(B1, Bm, Bl, k1, k2, k3, h, qop);
+    }
+    if constexpr (FK == kFieldConst) {
+      // the sums of the stages below, collected by v1 and v2
+      const double f1 = hh6 * (3.0 - c), f2 = hh6 * h, g1 = h6 * (6.0 - 4.0 * c);
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-      dir[k] = dir[k] + h6 * (k1[k] + 2.0 * (k2[k] + k3[k]) + k4[k]);
-    const double idn = 1.0 / sqrt(dir[0] * dir[0] + dir[1] * dir[1] + dir[2] * dir[2]);
+      for (int k = 0; k < 3; ++k) {
+        pos[k] = pos[k] + h * dir[k] + (f1 * k1[k] + f2 * v2[k]);
+        k4[k] = (1.0 - 2.0 * c) * k1[k] + (h * (1.0 - c)) * v2[k];
+        dir[k] = dir[k] + (g1 * k1[k] + f1 * v2[k]);
+      }
+    } else {
+      // h^2/6 and h/6 as products with 1/6 (within an ulp of the quotients)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) pos[k] = pos[k] + h * dir[k] + hh6 * (k1[k] + k2[k] + k3[k]);
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        dir[k] = dir[k] + h6 * (k1[k] + 2.0 * (k2[k] + k3[k]) + k4[k]);
+    }
+    double dn, idn;
+    rootD(dir[0] * dir[0] + dir[1] * dir[1] + dir[2] * dir[2], dn, idn);
 #pragma unroll
     for (int k = 0; k < 3; ++k) dir[k] = dir[k] * idn;
     derivSet = true;
@@ -552,9 +622,99 @@ struct TrackFit {
     return true;
   }
 
+  // J <- D J in a constant field, double: D's direction blocks are the
+  // polynomials of step() applied to each column g of J's direction rows
+  // (with v1 = g x w, v2 = v1 x w: dF g = h g + h^2/6 ((3 - c) v1 + h v2),
+  // dG g = g + h/6 ((6 - 4c) v1 + h (3 - c) v2)), and the q/p column adds
+  // their derivatives with respect to q/p at fixed d, in u1 = d x B and
+  // u2 = u1 x w.  ~100 operations where building the 3x3 blocks from the four
+  // stage matrices takes ~300.
+  KFD_INLINE void transportConst(const double w[3], const double u1[3], const double u2[3],
+                                 double h, double h6, double hh6, double c) {
+    const double f1 = hh6 * (3.0 - c), f2 = hh6 * h, g1 = h6 * (6.0 - 4.0 * c);
+#pragma unroll
+    for (int col = 0; col < 3; ++col) {
+      const double g[3] = {(double)G[0][col], (double)G[1][col], (double)G[2][col]};
+      double v1[3], v2[3];
+      cross(g, w, v1);
+      cross(v1, w, v2);
+#pragma unroll
+      for (int r = 0; r < 3; ++r) {
+        A[r][2 + col] = A[r][2 + col] + (h * g[r] + (f1 * v1[r] + f2 * v2[r]));
+        G[r][col] = g[r] + (g1 * v1[r] + f1 * v2[r]);
+      }
+    }
+    const double a1 = hh6 * (3.0 - 3.0 * c), a2 = 2.0 * f2, b1 = h6 * (6.0 - 12.0 * c),
+                 b2 = h * g1;
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      A[r][4] = A[r][4] + (a1 * u1[r] + a2 * u2[r]);
+      G[r][2] = G[r][2] + (b1 * u1[r] + b2 * u2[r]);
+    }
+  }
+
+  // J <- D J in any field, double: the stage chain of the
+  // direction block run on each column g of J's direction rows, with
+  // w = q/p B of the stage: v1 = g x w1, v2 = (g + h/2 v1) x wm,
+  // v3 = (g + h/2 v2) x wm, v4 = (g + h v3) x wl; the q/p column adds the
+  // derivatives of the stages with respect to q/p.  ~210 operations where the
+  // 3x3 blocks take ~300.  Lane groups run it whole on every lane: gathering a
+  // column costs what computing it does.
+  KFD_INLINE void transportColumns(const double B1[3], const double Bm[3], const double Bl[3],
+                                   const double k1[3], const double k2[3], const double k3[3],
+                                   double h, double h6, double hh6, double qop) {
+    const double hh = 0.5 * h;
+    double w1[3], wm[3], wl[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      w1[k] = qop * B1[k];
+      wm[k] = qop * Bm[k];
+      wl[k] = qop * Bl[k];
+    }
+#pragma unroll
+    for (int col = 0; col < 3; ++col) {
+      const double g[3] = {(double)G[0][col], (double)G[1][col], (double)G[2][col]};
+      double v1[3], v2[3], v3[3], v4[3], x[3];
+      cross(g, w1, v1);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) x[k] = g[k] + hh * v1[k];
+      cross(x, wm, v2);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) x[k] = g[k] + hh * v2[k];
+      cross(x, wm, v3);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) x[k] = g[k] + h * v3[k];
+      cross(x, wl, v4);
+#pragma unroll
+      for (int r = 0; r < 3; ++r) {
+        const double m = v2[r] + v3[r];
+        A[r][2 + col] = A[r][2 + col] + (h * g[r] + hh6 * (v1[r] + m));
+        G[r][col] = g[r] + h6 * ((v1[r] + v4[r]) + 2.0 * m);
+      }
+    }
+    // dk/d(q/p): L1 = d x B1, L2 = (d + h/2 k1 + h/2 qop L1) x Bm, ...
+    double L1[3], L2[3], L3[3], L4[3], x[3];
+    cross(dir, B1, L1);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) x[k] = dir[k] + h * k1[k];  // qop L1 = k1
+    cross(x, Bm, L2);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) x[k] = dir[k] + hh * (k2[k] + qop * L2[k]);
+    cross(x, Bm, L3);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) x[k] = dir[k] + h * (k3[k] + qop * L3[k]);
+    cross(x, Bl, L4);
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      const double m = L2[r] + L3[r];
+      A[r][4] = A[r][4] + hh6 * (L1[r] + m);
+      G[r][2] = G[r][2] + h6 * ((L1[r] + L4[r]) + 2.0 * m);
+    }
+  }
+
   // J <- D J for the free transport matrix D of one RK step
   // (EigenStepper.ipp:50-124 builds D; its identity / zero blocks are used
-  // implicitly).
+  // implicitly): the mixed mode's, in float.
   KFD_INLINE void transport(const double Bfd[3], const double Bmd[3], const double Bld[3],
                             const double k1d[3], const double k2d[3], const double k3d[3],
                             double hd, double qopd) {
@@ -679,9 +839,6 @@ struct TrackFit {
       dFdL[r] = hh6 * (dk1dL[r] + dk2dL[r] + dk3dL[r]);
       dGdL[r] = h6 * (dk1dL[r] + (S)2.0 * (dk2dL[r] + dk3dL[r]) + dk4dL[r]);
     }
-    const double m = a.mass;
-    const S d37 = (S)(hd * m * m * q / cacheDen);
-
     // J <- D J on the non-constant entries
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
@@ -698,7 +855,6 @@ struct TrackFit {
         G[r][c] = ga;
       }
     }
-    b = b + d37;
   }
 
   // qop * cross_cols(I + hh * M, B)  (Helpers.hpp:168-176)
@@ -917,9 +1073,10 @@ struct TrackFit {
     S dr[8];
 #pragma unroll
     for (int k = 0; k < 3; ++k) dr[k] = derivSet ? (S)dir[k] : (S)0;
-    dr[3] = derivSet ? dtds : (S)0;
+    // dtds and k4d are zero while derivSet is not
+    dr[3] = dtds;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) dr[4 + k] = derivSet ? k4d[k] : (S)0;
+    for (int k = 0; k < 3; ++k) dr[4 + k] = k4d[k];
     const S l20 = (S)(-sinP * invSinT), l21 = (S)(cosP * invSinT);
     const S l30 = (S)(cosP * cosT), l31 = (S)(sinP * cosT), l32 = (S)(-sinT);
 #pragma unroll
@@ -987,15 +1144,15 @@ struct TrackFit {
   // 345-371) including the Jacobian re-initialisation on the plane.
   KFD_INLINE void boundStatePlane(const DevPlane &pl, double par[6], S jb[6][6]) {
     const double cosT = dir[2];
-    const double sinT = sqrt(dir[0] * dir[0] + dir[1] * dir[1]);
-    const double invSinT = 1.0 / sinT;
+    double sinT, invSinT;
+    rootD(dir[0] * dir[0] + dir[1] * dir[1], sinT, invSinT);
     const double cosP = dir[0] * invSinT, sinP = dir[1] * invSinT;
     const double u0[3] = {pl.r[0], pl.r[3], pl.r[6]};
     const double u1[3] = {pl.r[1], pl.r[4], pl.r[7]};
     const double nr[3] = {pl.r[2], pl.r[5], pl.r[8]};
     // PlaneSurface::derivativeFactors, PlaneSurface.ipp:191-204
     const double dp = nr[0] * dir[0] + nr[1] * dir[1] + nr[2] * dir[2];
-    const double idp = 1.0 / dp;
+    const double idp = recipD(dp);
     const double nv[3] = {nr[0] * idp, nr[1] * idp, nr[2] * idp};
     double sVec[6];
 #pragma unroll
@@ -1004,21 +1161,46 @@ struct TrackFit {
     sVec[5] = 0.0;
     covarianceTransport(sVec, u0, u1, cosT, sinT, invSinT, cosP, sinP, jb);
     // bound parameters: global2parameters on the plane
-    const double qop = q / p;
-    const double pabs = fabs(1.0 / qop);
-    const double mom[3] = {pabs * dir[0], pabs * dir[1], pabs * dir[2]};
-    const double charge = copysign(1.0, qop);
     const double dd[3] = {pos[0] - pl.c[0], pos[1] - pl.c[1], pos[2] - pl.c[2]};
     par[0] = pl.r[0] * dd[0] + pl.r[3] * dd[1] + pl.r[6] * dd[2];
     par[1] = pl.r[1] * dd[0] + pl.r[4] * dd[1] + pl.r[7] * dd[2];
-    par[2] = atan2D(mom[1], mom[0]);
-    par[3] = atan2D(sqrt(mom[0] * mom[0] + mom[1] * mom[1]), mom[2]);
-    const double mn = sqrt(mom[0] * mom[0] + mom[1] * mom[1] + mom[2] * mom[2]);
-    par[4] = ((fabs(charge) < 1e-4) ? 1.0 : charge) / mn;
+    planeAngles(sinT, par);
     par[5] = t;
     correctParams(par);
     // reinitializeJacobians on the plane (PlaneSurface.ipp:122-156)
     initJacobianPlane(pl, cosT, sinT, cosP, sinP);
+  }
+
+  // phi, theta and q/p of the direction at a plane (sinT = its transverse
+  // length): the reference's conversions of the momentum vector, whose angles
+  // are taken from those after the last update plus the arc tangents of the
+  // rotation since, in the transverse plane and in theta.  Over a segment the
+  // rotation is small, so each is a division (one shared reciprocal) and a
+  // short series, ~50 instructions for both angles where two library arc
+  // tangents take ~270; a rotation with a tangent above 1/16 (or no
+  // reference, or a stopped particle) takes the library.  Agrees with it to
+  // an ulp of the angle per segment.
+  KFD_INLINE void planeAngles(double sinT, double par[6]) {
+    const double n1 = refX * dir[1] - refY * dir[0], d1 = refX * dir[0] + refY * dir[1];
+    double refS, refIS;
+    rootD(refX * refX + refY * refY, refS, refIS);
+    const double n2 = sinT * refZ - dir[2] * refS, d2 = dir[2] * refZ + sinT * refS;
+    const double i12 = recipD(d1 * d2);
+    const double r1 = n1 * (d2 * i12), r2 = n2 * (d1 * i12);
+    if (0.0 < d1 && 0.0 < d2 && fabs(r1) <= 0.0625 && fabs(r2) <= 0.0625 && 0.0 < p) {
+      par[2] = refPhi + atanSmall(r1);
+      par[3] = refTheta + atanSmall(r2);
+      par[4] = divD(q, p);
+      return;
+    }
+    const double qop = q / p;
+    const double pabs = fabs(1.0 / qop);
+    const double mom[3] = {pabs * dir[0], pabs * dir[1], pabs * dir[2]};
+    const double charge = copysign(1.0, qop);
+    par[2] = atan2D(mom[1], mom[0]);
+    par[3] = atan2D(sqrt(mom[0] * mom[0] + mom[1] * mom[1]), mom[2]);
+    const double mn = sqrt(mom[0] * mom[0] + mom[1] * mom[1] + mom[2] * mom[2]);
+    par[4] = ((fabs(charge) < 1e-4) ? 1.0 : charge) / mn;
   }
 
   // boundState on the perigee line (LineSurface.ipp:114-220); the Jacobians
@@ -1120,12 +1302,13 @@ struct TrackFit {
     else if (dphi < -kPi)
       dphi += 2.0 * kPi;
     const double dth = xf[3] - xp[3];
-    const double sinT = sqrt(dir[0] * dir[0] + dir[1] * dir[1]), cosT = dir[2];
+    const double cosT = dir[2];
+    double sinT, iS;
+    rootD(dir[0] * dir[0] + dir[1] * dir[1], sinT, iS);
     if (!(fabs(dphi) < 0.0625 && fabs(dth) < 0.0625 && sinT > 1e-3)) {
       updateFromBound(pl, xf);
       return;
     }
-    const double iS = 1.0 / sinT;
     const double cosP = dir[0] * iS, sinP = dir[1] * iS;
     double sp, cp, st, ct;
     sinCosSmall(dphi, sp, cp);
@@ -1135,7 +1318,8 @@ struct TrackFit {
 #pragma unroll
     for (int k = 0; k < 3; ++k) pos[k] = (pl.r[3 * k] * xf[0] + pl.r[3 * k + 1] * xf[1]) + pl.c[k];
     const double d0 = cPf * sTf, d1 = sPf * sTf, d2 = cTf;
-    const double idn = 1.0 / sqrt(d0 * d0 + d1 * d1 + d2 * d2);
+    double dn, idn;
+    rootD(d0 * d0 + d1 * d1 + d2 * d2, dn, idn);
     dir[0] = d0 * idn;
     dir[1] = d1 * idn;
     dir[2] = d2 * idn;
@@ -1161,7 +1345,7 @@ struct TrackFit {
       const double nr[3] = {pl.r[2], pl.r[5], pl.r[8]};
       denom = dot3(d, nr);
       const double cm[3] = {pl.c[0] - pos[0], pl.c[1] - pos[1], pl.c[2] - pos[2]};
-      path = (denom != 0.0) ? dot3(nr, cm) / denom : 0.0;
+      path = (denom != 0.0) ? divD(dot3(nr, cm), denom) : 0.0;
       pathPlane = idx;
       pathDenom = denom;
       pathLen = path;
@@ -1530,6 +1714,7 @@ struct TrackFit {
       for (int m = 0; m < 21; ++m) cm[m] = cov[m];
     }
     updateFromFiltered(pl, xf, xp);
+    setReference(xf);
     material(pl);
     if constexpr (kStore) {
       cm[KF_SS_MD - KF_SS_CF + 0] = cov[sidx(2, 2)];

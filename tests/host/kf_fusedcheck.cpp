@@ -3,14 +3,32 @@
 // track at a time.  Test infrastructure only: the library never loads it.
 #include "kf_hostcheck.cpp"
 
+namespace {
+
+template <int FK>
+void fusedTracks(Host &h, int32_t *redo) {
+  using Fit = TrackFit<double, true, 1, false, false, FK, kKeepFirst>;
+  std::vector<typename Fit::FxPair> sums((size_t)Fit::kFxN * KF_FUSED_BLOCK);
+  for (int64_t i = 0; i < h.a.n; ++i) {
+    Fit tf(h.a, i, nullptr, nullptr, nullptr, nullptr, 0u, i);
+    tf.pls = h.planes.data();
+    tf.fx = sums.data();
+    redo[i] = tf.runFused() ? 0 : 1;
+  }
+}
+
+}  // namespace
+
 extern "C" {
 
-// The fit of every track by the fused program: params [6][n], cov [21][n],
+// The fit of every track by the fused program, built for either field kind
+// (0), the constant field (1) or the grid (2): params [6][n], cov [21][n],
 // chi2, n_measured, status [n], and redo [n], nonzero for a track that it
 // leaves to the RTS program (its params, cov and status are not set).
-int kfh_fit_fused(const kf_plane *planes, int32_t n_planes, const kfh_field *f,
-                  const kf_tracks *tr, const kf_options *opt, double *params, double *cov,
-                  double *chi2, int32_t *n_measured, uint32_t *status, int32_t *redo) {
+int kfh_fit_fused_kind(const kf_plane *planes, int32_t n_planes, const kfh_field *f,
+                       const kf_tracks *tr, const kf_options *opt, int32_t field_kind,
+                       double *params, double *cov, double *chi2, int32_t *n_measured,
+                       uint32_t *status, int32_t *redo) {
   Host h(planes, n_planes, f, tr, opt, true);
   h.a.out_params = params;
   h.a.out_cov = cov;
@@ -18,15 +36,20 @@ int kfh_fit_fused(const kf_plane *planes, int32_t n_planes, const kfh_field *f,
   h.a.out_nmeas = n_measured;
   h.a.out_status = status;
   h.a.out_ndf = nullptr;
-  using Fit = TrackFit<double, true, 1, false, false, kFieldAny, kKeepFirst>;
-  std::vector<Fit::FxPair> sums((size_t)Fit::kFxN * KF_FUSED_BLOCK);
-  for (int64_t i = 0; i < tr->n_tracks; ++i) {
-    Fit tf(h.a, i, nullptr, nullptr, nullptr, nullptr, 0u, i);
-    tf.pls = h.planes.data();
-    tf.fx = sums.data();
-    redo[i] = tf.runFused() ? 0 : 1;
-  }
+  if (field_kind == kFieldGrid)
+    fusedTracks<kFieldGrid>(h, redo);
+  else if (field_kind == kFieldConst)
+    fusedTracks<kFieldConst>(h, redo);
+  else
+    fusedTracks<kFieldAny>(h, redo);
   return 0;
+}
+
+int kfh_fit_fused(const kf_plane *planes, int32_t n_planes, const kfh_field *f,
+                  const kf_tracks *tr, const kf_options *opt, double *params, double *cov,
+                  double *chi2, int32_t *n_measured, uint32_t *status, int32_t *redo) {
+  return kfh_fit_fused_kind(planes, n_planes, f, tr, opt, kFieldAny, params, cov, chi2,
+                            n_measured, status, redo);
 }
 
 }  // extern "C"
