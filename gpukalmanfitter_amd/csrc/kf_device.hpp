@@ -32,6 +32,29 @@ namespace kfd {
 // point (bounds the number of live registers in load-heavy phases).
 #define KFD_PHASE_FENCE() __asm__ volatile("" ::: "memory")
 
+// Keeps a kernel argument in a vector register: left in the argument segment,
+// an option that a loop needs once per iteration is loaded again each time (the
+// scalar registers are full) and waited for, ~200 cycles that nothing hides at
+// one wave per SIMD.
+KFD_INLINE double inVgpr(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __asm__ volatile("" : "+v"(x));
+#endif
+  return x;
+}
+KFD_INLINE int inVgpr(int x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __asm__ volatile("" : "+v"(x));
+#endif
+  return x;
+}
+// Waits for every vector-memory load issued so far.
+KFD_INLINE void waitLoads() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), the other counters at their maximum
+#endif
+}
+
 // --------------------------------------------------------- lane groups ----
 // A track may be fitted by a group of L = 1, 2 or 4 consecutive lanes of a
 // quad (the counterpart of the reference's block-per-track kernel): every
@@ -137,7 +160,17 @@ KFD_INLINE void fieldConst(const DevField &f, double B[3]) {
 
 // Grid: trilinear, last axis first (the reference's
 // interpolation_impl.hpp:98-131), positions clamped to the box.
-KFD_INLINE void fieldGrid(const DevField &f, double x, double y, double z, double B[3]) {
+//
+// The four (x, y) corner columns of a cell, six floats each (the z pair).  A
+// track's RK step looks up three points, and the short step that ends on a
+// plane, like the start of the step after it, stays in the cell of the last
+// lookup: the lanes whose cell is still the one they hold read nothing.
+struct GridCell {
+  int64_t at = -1;  // index of the cell's lowest corner; -1: none held
+  float v[4][6];
+};
+KFD_INLINE void fieldGrid(const DevField &f, double x, double y, double z, double B[3],
+                          GridCell &cell) {
   const double p[3] = {x, y, z};
   int idx[3];
   double fr[3];
@@ -153,22 +186,23 @@ KFD_INLINE void fieldGrid(const DevField &f, double x, double y, double z, doubl
     const double ll = f.lo[d] + (double)i * f.w[d];
     fr[d] = (v - ll) * f.iw[d];
   }
-  // the four (x, y) corner columns: six floats each (the z pair), all
-  // loads issued before any is used, so one memory latency per lookup
-  float v[4][6];
+  const int64_t at = ((int64_t)idx[0] * f.n[1] + idx[1]) * f.n[2] + idx[2];
+  if (at != cell.at) {
+    cell.at = at;
+    // all loads issued before any is used, so one memory latency per lookup
+    const float *c0 = f.values + 3 * at;
+    const int64_t sy = 3 * (int64_t)f.n[2], sx = sy * f.n[1];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int ix = idx[0] + (c >> 1), iy = idx[1] + (c & 1);
-    const size_t b0 = (((size_t)ix * f.n[1] + iy) * f.n[2] + idx[2]) * 3;
+    for (int c = 0; c < 4; ++c)
 #pragma unroll
-    for (int k = 0; k < 6; ++k) v[c][k] = f.values[b0 + k];
+      for (int k = 0; k < 6; ++k) cell.v[c][k] = c0[(c >> 1) * sx + (c & 1) * sy + k];
   }
   double cz[4][3];
 #pragma unroll
   for (int c = 0; c < 4; ++c)
 #pragma unroll
     for (int k = 0; k < 3; ++k)
-      cz[c][k] = (1.0 - fr[2]) * (double)v[c][k] + fr[2] * (double)v[c][3 + k];
+      cz[c][k] = (1.0 - fr[2]) * (double)cell.v[c][k] + fr[2] * (double)cell.v[c][3 + k];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const double y0 = (1.0 - fr[1]) * cz[0][k] + fr[1] * cz[1][k];
@@ -180,10 +214,12 @@ KFD_INLINE void fieldGrid(const DevField &f, double x, double y, double z, doubl
 
 // Either kind, chosen by f.grid at run time.
 KFD_INLINE void fieldAt(const DevField &f, double x, double y, double z, double B[3]) {
-  if (!f.grid)
+  if (!f.grid) {
     fieldConst(f, B);
-  else
-    fieldGrid(f, x, y, z, B);
+  } else {
+    GridCell cell;
+    fieldGrid(f, x, y, z, B, cell);
+  }
 }
 
 // Field and its spatial derivative dB[k][axis] = dB_k / dx_axis (the chi2

@@ -153,6 +153,15 @@ struct TrackFit {
   int pathPlane = -1;
   double pathLen = 0.0, pathDenom = 0.0;
   KFD_INLINE void moved() { pathPlane = -1; }
+  // options read in every iteration
+  double tol, negOverstep, outlierCut;
+  int maxSteps;
+  KFD_INLINE void loadOptions() {
+    tol = inVgpr(a.tolerance);
+    negOverstep = inVgpr(-a.overstep_limit);
+    outlierCut = inVgpr(a.outlier_chi2_cut);
+    maxSteps = inVgpr(a.max_steps);
+  }
 
   // per-state stores of this wave's 64-track chunk (wave-uniform bases) and
   // this lane's slot in them
@@ -330,11 +339,14 @@ struct TrackFit {
   // -------------------------------------------------------------- field ----
   // FK: the field kind the kernel was built for (kFieldConst and
   // kFieldGrid leave the other kind's code out of the step loop)
-  KFD_INLINE void field(const double x[3], double B[3]) const {
+  // The grid cell of the last lookup; only in the grid builds (the either-kind
+  // builds are at the register limit, its 26 registers cost them 7 %).
+  GridCell cell;
+  KFD_INLINE void field(const double x[3], double B[3]) {
     if constexpr (FK == kFieldConst)
       fieldConst(a.field, B);
     else if constexpr (FK == kFieldGrid)
-      fieldGrid(a.field, x[0], x[1], x[2], B);
+      fieldGrid(a.field, x[0], x[1], x[2], B, cell);
     else
       fieldAt(a.field, x[0], x[1], x[2], B);
   }
@@ -559,10 +571,10 @@ struct TrackFit {
         err = h2 * e1;
       }
       err = (err < 1e-20) ? 1e-20 : err;
-      if (err <= a.tolerance) break;
+      if (err <= tol) break;
       // std::min(std::max(0.25, x), 4.) with its NaN behaviour: a NaN error
       // estimate (h = DBL_MAX after an actor release) scales by 0.25
-      ss.assign(ss.get() * stepScale(a.tolerance, err));
+      ss.assign(ss.get() * stepScale(tol, err));
       const double hn = ss.get();
       if (hn * hn < a.step_size_cutoff * a.step_size_cutoff || nTrials > a.max_rk_trials) {
         stepFailed = true;
@@ -1340,12 +1352,16 @@ struct TrackFit {
       denom = pathDenom;
       path = pathLen;
     } else {
+      // the plane's normal and centre read at once, and the quotient formed
+      // whatever the denominator: one wait for the table instead of three
       const DevPlane &pl = plane(idx);
-      const double d[3] = {nd * dir[0], nd * dir[1], nd * dir[2]};
       const double nr[3] = {pl.r[2], pl.r[5], pl.r[8]};
+      const double pc[3] = {pl.c[0], pl.c[1], pl.c[2]};
+      const double d[3] = {nd * dir[0], nd * dir[1], nd * dir[2]};
       denom = dot3(d, nr);
-      const double cm[3] = {pl.c[0] - pos[0], pl.c[1] - pos[1], pl.c[2] - pos[2]};
-      path = (denom != 0.0) ? divD(dot3(nr, cm), denom) : 0.0;
+      const double cm[3] = {pc[0] - pos[0], pc[1] - pos[1], pc[2] - pos[2]};
+      const double quot = divD(dot3(nr, cm), denom);
+      path = (denom != 0.0) ? quot : 0.0;
       pathPlane = idx;
       pathDenom = denom;
       pathLen = path;
@@ -1356,7 +1372,7 @@ struct TrackFit {
         return 2;
       }
       const double pLimit = ss.v[kAborter];
-      if (path > -a.overstep_limit && path * path < pLimit * pLimit) {
+      if (path > negOverstep && path * path < pLimit * pLimit) {
         ss.release(kActor);
         ss.update(nd * path, kActor);
         return 1;
@@ -1555,6 +1571,9 @@ struct TrackFit {
       V00 = a.hit_cov[hit];
       V01 = a.hit_cov[a.n_hits + hit];
       V11 = a.hit_cov[2 * a.n_hits + hit];
+      // waited for here: left pending, every filter would wait before its gain
+      // for all loads in flight, the next hit's among them
+      waitLoads();
       inOrder = inOrder && hit == hitNext;
     }
     if (inOrder) {
@@ -1621,7 +1640,7 @@ struct TrackFit {
     // outlier finder: above the cut the state keeps its prediction (no
     // update, the covariance stays the predicted one) and stays out of the
     // chi2 sum and ndf; 0 disables it (the reference's void finder)
-    if (a.outlier_chi2_cut > 0.0 && chi2 > a.outlier_chi2_cut) {
+    if (outlierCut > 0.0 && chi2 > outlierCut) {
 #pragma unroll
       for (int r = 0; r < 6; ++r) xf[r] = xp[r];
       ++outliers;
@@ -2015,7 +2034,7 @@ struct TrackFit {
   // ends: terminated by an aborter or after max_steps.
   template <bool F>
   KFD_INLINE bool cheapSteps(int &steps, bool &terminated) {
-    while (steps < a.max_steps) {
+    while (steps < maxSteps) {
       step();
       navStatus();
       if (F && cur >= 0 && !smoothed && !finished) return true;
@@ -2113,7 +2132,7 @@ struct TrackFit {
     if (finished) status |= KF_STATUS_FINISHED;
     if (!result) status |= KF_STATUS_RESULT_FAIL;
     if (stepFailed) status |= KF_STATUS_STEP_FAIL;
-    if (!terminated && steps >= a.max_steps) status |= KF_STATUS_MAX_STEPS;
+    if (!terminated && steps >= maxSteps) status |= KF_STATUS_MAX_STEPS;
     if (navBreak && measured != (int)(h1 - h0)) status |= KF_STATUS_NAV_BREAK;
     if (smootherNaN) status |= KF_STATUS_SMOOTHER_NAN;
     return status;
@@ -2148,6 +2167,7 @@ struct TrackFit {
   }
 
   KFD_INLINE void loadTrack() {
+    loadOptions();
     h0 = a.hit_offset[i];
     h1 = a.hit_offset[i + 1];
     hitNext = h0;

@@ -75,3 +75,27 @@ def test_low_momentum_rotations_match_oracle(built, p):
     if fin.any():
         pd, cd, c2 = compare_fit(f, o, mask=fin)
         assert max(pd, cd, c2) <= 1e-9, (pd, cd, c2)
+
+
+@pytest.mark.parametrize("n,half", [((2, 2, 2), 2000.0), ((3, 2, 5), 150.0), ((40, 40, 40), 290.0)])
+def test_grid_lookups_match_oracle(built, n, half):
+    """The grid build, which keeps the cell of its last lookup: one cell for the
+    whole detector, boxes that end inside it (lookups clamped to the edge), and
+    cells smaller than a step.  Bar: 1e-9."""
+    b = G.generate(1, n_tracks=300)
+    rng = np.random.default_rng(3)
+    v = np.zeros(n + (3,), dtype=np.float32)
+    v[..., 2] = 2.0 * T
+    v += (0.2 * T * rng.standard_normal(v.shape)).astype(np.float32)
+    fld = G.FieldSpec(kind="grid", values=v, lo=(-half,) * 3, hi=(half,) * 3, scale=1.01)
+    b = dataclasses.replace(b, field=fld)
+    opt = abi.default_options(**W)
+    f = fit_kind(b, opt, 2)
+    o, _, _, _ = oracle.fit(b, opt)
+    keep = f["redo"] == 0
+    assert keep.sum() > 250
+    assert np.array_equal(f["status"][keep], o.status[keep])
+    fin = keep & ((o.status & abi.KF_STATUS_OK) != 0)
+    assert fin.sum() > 250
+    pd, cd, c2 = compare_fit(f, o, mask=fin)
+    assert max(pd, cd, c2) <= 1e-9, (pd, cd, c2)
