@@ -7,16 +7,29 @@
 
 namespace kfd {
 
+// FK: the batch's field kind.  PLDS: the plane table in dynamic LDS (where two
+// blocks of the kernel still fit a compute unit with it).
+template <int FK, bool PLDS>
 __global__ void __launch_bounds__(KF_BLOCK) kf_adjoint_kernel(FitArgs args, AdjArgs adj) {
   __shared__ double lds[kLDS_N * KF_BLOCK];
-  __shared__ float ldf[kLDSF_N * KF_BLOCK];
+  __shared__ float ldf[FK == kFieldConst ? 1 : kLDSF_N * KF_BLOCK];
+  extern __shared__ double lds_table[];
+  const DevPlane *planes = args.planes;
+  if constexpr (PLDS) {
+    const double *src = (const double *)args.planes;
+    const int words = args.n_planes * (int)(sizeof(DevPlane) / sizeof(double));
+    for (int w = threadIdx.x; w < words; w += KF_BLOCK) lds_table[w] = src[w];
+    __syncthreads();
+    planes = (const DevPlane *)lds_table;
+  }
   const int64_t local = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const size_t chunk = __builtin_amdgcn_readfirstlane((uint32_t)(local >> 6));
   double *ck = args.tsc + chunk * (size_t)args.max_states * KF_CK_N * 64u;
   double *stk = adj.stack + chunk * (size_t)adj.max_seg_steps * kSR_N * 64u;
   if (local >= args.count) return;
-  TrackAdjoint ta(args, adj, args.first + local, local, ck, stk, (uint32_t)(local & 63),
-                  lds + threadIdx.x, ldf + threadIdx.x);
+  TrackAdjoint<FK> ta(args, adj, args.first + local, local, ck, stk, (uint32_t)(local & 63),
+                      lds + threadIdx.x, FK == kFieldConst ? nullptr : ldf + threadIdx.x);
+  ta.tf.pls = planes;
   ta.run();
 }
 
@@ -115,8 +128,19 @@ extern "C" hipError_t kfd_launch_adjoint(const kfd::FitArgs *args, const kfd::Ad
                                          double *sums, int accumulate, hipStream_t stream) {
   const int64_t blocks = (args->count + KF_BLOCK - 1) / KF_BLOCK;
   if (blocks > 0)
-    hipLaunchKernelGGL(kfd::kf_adjoint_kernel, dim3((unsigned)blocks), dim3(KF_BLOCK), 0, stream,
-                       *args, *adj);
+  {
+    const bool grid = args->field.grid != 0;
+    const size_t table = (size_t)args->n_planes * sizeof(kfd::DevPlane);
+    const size_t held = kfd::kLDS_N * KF_BLOCK * sizeof(double) +
+                        (grid ? kfd::kLDSF_N * KF_BLOCK : 1) * sizeof(float);
+    const bool plds = held + table <= 160 * 1024 / 2 - 256;
+    auto *kernel = grid ? (plds ? kfd::kf_adjoint_kernel<kfd::kFieldGrid, true>
+                                : kfd::kf_adjoint_kernel<kfd::kFieldGrid, false>)
+                        : (plds ? kfd::kf_adjoint_kernel<kfd::kFieldConst, true>
+                                : kfd::kf_adjoint_kernel<kfd::kFieldConst, false>);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(KF_BLOCK),
+                       plds ? (unsigned)table : 0u, stream, *args, *adj);
+  }
   double *partial = sums + (size_t)(args->n_planes + 2) * kfd::kPG_N;
   hipLaunchKernelGGL(kfd::kf_adjoint_reduce, dim3((unsigned)(args->n_planes + 2), kfd::kRedSlices),
                      dim3(kfd::kRedThreads), 0, stream, *args, *adj, partial);

@@ -50,12 +50,15 @@ enum { kPG_C = 0, kPG_R = 3, kPG_N = 12 };
 
 // per-lane LDS slots (doubles, stride KF_BLOCK) for adjoint state of the
 // reverse step loop, so that it does not occupy registers there: the
-// covariance adjoint (carried across the loop, unused in it), the adjoint of
-// the Jacobian's position rows A (constant over a segment's steps), of its
-// direction rows G, and the next G adjoint while a step builds it
-enum { kLDS_CB = 0, kLDS_AB = 25, kLDS_GB = 40, kLDS_GT = 49, kLDS_N = 58 };
+// covariance adjoint (upper triangle; carried across the loop, unused in it),
+// the adjoint of the Jacobian's position rows A (constant over a segment's
+// steps), of its direction rows G, the next G adjoint while a step builds it,
+// and the adjoint of the segment's measured plane (centre, rotation), which
+// goes to memory once per segment: added up there, it was three dependent
+// round trips to memory per plane
+enum { kLDS_CB = 0, kLDS_AB = 15, kLDS_GB = 30, kLDS_GT = 39, kLDS_PL = 48, kLDS_N = 60 };
 // float slots: the grid-field gradient at a reversed step's three stage
-// points (27); with the double slots 73.2 KB per 128-lane block, two blocks
+// points (27); with the double slots 75.3 KB per 128-lane block, two blocks
 // (four waves) per CU
 enum { kLDSF_N = 27 };
 
@@ -70,6 +73,11 @@ struct AdjArgs {
   uint32_t *status;       // [n]: 0 ok, else KF_ADJ_* bits
 };
 
+
+// packed index of (r, c) of a symmetric 5x5 matrix
+KFD_INLINE constexpr int cidx(int r, int c) {
+  return (r <= c) ? (r * 5 - (r * (r - 1)) / 2 + (c - r)) : (c * 5 - (c * (c - 1)) / 2 + (r - c));
+}
 
 // a x b
 KFD_INLINE void crs(const double a[3], const double b[3], double r[3]) {
@@ -89,9 +97,11 @@ KFD_INLINE void crsVJP(const double a[3], const double b[3], const double cb[3],
   for (int k = 0; k < 3; ++k) bb[k] += t[k];
 }
 // B = s F(x): sb += Bb . F(x) = Bb . B / s; xb += (dB/dx)^T Bb on a grid.
+template <int FK>
 KFD_INLINE void fieldVJP(const DevField &fld, const double x[3], const double B[3],
                          const double Bb[3], double xb[3], double &sb) {
   sb += (Bb[0] * B[0] + Bb[1] * B[1] + Bb[2] * B[2]) / fld.scale;
+  if constexpr (FK == kFieldConst) return;
   if (fld.grid) {
     double Bg[3], dB[3][3];
     fieldAtGrad(fld, x, Bg, dB);
@@ -115,6 +125,7 @@ KFD_INLINE void fieldVJPStored(const DevField &fld, const float *dBs, int pt, co
 
 // One RK4 step (EigenStepper.ipp:226-332 at its accepted length) with every
 // intermediate the backward step needs.
+template <int FK>
 struct StepFwd {
   double B1[3], Bm[3], Bl[3];
   double k1[3], k2[3], k3[3], k4[3];
@@ -128,6 +139,10 @@ struct StepFwd {
   // backward reads the corners again
   KFD_INLINE void lookup(const DevField &fld, const double x[3], double B[3], float *dBs,
                          int pt) {
+    if constexpr (FK == kFieldConst) {
+      fieldConst(fld, B);
+      return;
+    }
     if (dBs && fld.grid) {
       double dB[3][3];
       fieldAtGrad(fld, x, B, dB);
@@ -197,7 +212,8 @@ struct StepFwd {
 // (the matrices of EigenStepper.ipp:50-124 applied to a vector).  This is the
 // backward of that map: aF, aG are the adjoints of dFdT g and dGdT g; it
 // accumulates gb, the field adjoints, hb and qb.
-KFD_INLINE void dirColumnVJP(const StepFwd &F, double h, double qop, const double g[3],
+template <int FK>
+KFD_INLINE void dirColumnVJP(const StepFwd<FK> &F, double h, double qop, const double g[3],
                              const double aF[3], const double aG[3], double gb[3], double B1b[3],
                              double Bmb[3], double Blb[3], double &hb, double &qb) {
   const double hh = 0.5 * h;
@@ -290,7 +306,8 @@ KFD_INLINE void dirColumnVJP(const StepFwd &F, double h, double qop, const doubl
 // the A adjoint passes through a step unchanged), and accumulated hb, qb
 // (q/p) and sb (field scale).  Gin: the J direction rows before the step,
 // element (r, c) at Gin[(3 r + c) * gstride].
-KFD_INLINE void stepVJP(const DevField &fld, const StepFwd &F, const double pos[3],
+template <int FK>
+KFD_INLINE void stepVJP(const DevField &fld, const StepFwd<FK> &F, const double pos[3],
                         const double d[3], double h, double qop, const double *Gin,
                         uint32_t gstride, double pb[3], double db[3], double *lj,
                         const double k4bIn[3], double &hb, double &qb, double &sb,
@@ -411,10 +428,10 @@ KFD_INLINE void stepVJP(const DevField &fld, const StepFwd &F, const double pos[
   }
   // Bl = s F(p2)
   double p2b[3] = {0, 0, 0};
-  if (dBs && fld.grid)
+  if (FK != kFieldConst && dBs && fld.grid)
     fieldVJPStored(fld, dBs, 2, F.Bl, Blb, p2b, sb);
   else
-    fieldVJP(fld, F.p2, F.Bl, Blb, p2b, sb);
+    fieldVJP<FK>(fld, F.p2, F.Bl, Blb, p2b, sb);
   // p2 = pos + h d + h^2/2 k3
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
@@ -451,10 +468,10 @@ KFD_INLINE void stepVJP(const DevField &fld, const StepFwd &F, const double pos[
   }
   // Bm = s F(p1)
   double p1b[3] = {0, 0, 0};
-  if (dBs && fld.grid)
+  if (FK != kFieldConst && dBs && fld.grid)
     fieldVJPStored(fld, dBs, 1, F.Bm, Bmb, p1b, sb);
   else
-    fieldVJP(fld, F.p1, F.Bm, Bmb, p1b, sb);
+    fieldVJP<FK>(fld, F.p1, F.Bm, Bmb, p1b, sb);
   // p1 = pos + hh d + h^2/8 k1
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
@@ -470,10 +487,10 @@ KFD_INLINE void stepVJP(const DevField &fld, const StepFwd &F, const double pos[
   for (int k = 0; k < 3; ++k) w[k] = qop * k1b[k];
   crsVJP(d, F.B1, w, dInb, B1b);
   // B1 = s F(pos)
-  if (dBs && fld.grid)
+  if (FK != kFieldConst && dBs && fld.grid)
     fieldVJPStored(fld, dBs, 0, F.B1, B1b, posInb, sb);
   else
-    fieldVJP(fld, pos, F.B1, B1b, posInb, sb);
+    fieldVJP<FK>(fld, pos, F.B1, B1b, posInb, sb);
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     pb[k] = posInb[k];
@@ -959,7 +976,8 @@ struct MaterialFwd {
 };
 
 // ---------------------------------------------------------------------------
-// The reverse sweep of one track.
+// The reverse sweep of one track.  FK: the field kind it is built for.
+template <int FK = kFieldAny>
 struct TrackAdjoint {
   const FitArgs &a;
   const AdjArgs &g;
@@ -969,7 +987,7 @@ struct TrackAdjoint {
   uint32_t lane;
   double *lds;  // this lane's LDS slots: lds[f * KF_BLOCK]
   float *ldf;   // this lane's float LDS slots: the grid-field gradient of a reversed step
-  TrackFit<double, true, 1, false, true> tf;  // recomputes segments from the checkpoints
+  TrackFit<double, true, 1, false, true, FK> tf;  // recomputes segments from the checkpoints
 
   KFD_INLINE TrackAdjoint(const FitArgs &args, const AdjArgs &adj, int64_t idx, int64_t local,
                           double *ckpt, double *stack, uint32_t ln, double *ldsLane,
@@ -983,6 +1001,7 @@ struct TrackAdjoint {
   KFD_INLINE double *pg(int q, int f) const {
     return g.plane_adj + ((size_t)q * kPG_N + f) * (size_t)a.count + loc;
   }
+  // adds to the adjoint of a plane passed without a hit (zeroed before)
   KFD_INLINE void addPlane(int plane, const double cb[3], const double Rb[3][3]) const {
     const int q = plane - tf.seqFirst;
     if (q < 0 || q >= g.max_seq) return;
@@ -993,22 +1012,19 @@ struct TrackAdjoint {
 #pragma unroll
       for (int c = 0; c < 3; ++c) *pg(q, kPG_R + 3 * r + c) += Rb[r][c];
   }
-  KFD_INLINE int64_t hitOn(int plane) const {
-    const int32_t id = a.planes[plane].geo_id;
-    for (int64_t h = tf.h0; h < tf.h1; ++h)
-      if (a.hit_geo_id[h] == id) return h;
-    return -1;
+  KFD_INLINE void zeroPlanes(int q0, int q1) const {
+    for (int q = q0; q < q1; ++q)
+      for (int f = 0; f < kPG_N; ++f) *pg(q, f) = 0.0;
   }
 
   KFD_INLINE void run() {
     tf.loadTrack();
     const int nmeas = a.out_nmeas[i];
     const int slots = (tf.size < g.max_seq) ? tf.size : g.max_seq;
-    for (int q = 0; q < slots; ++q)
-      for (int f = 0; f < kPG_N; ++f) *pg(q, f) = 0.0;
     uint32_t st = 0;
     double sb = 0.0;
     if (nmeas <= 0) {
+      zeroPlanes(0, slots);
       g.scale_adj[loc] = 0.0;
       if (g.status) g.status[i] = KF_ADJ_SKIPPED;
       return;
@@ -1023,6 +1039,13 @@ struct TrackAdjoint {
     // the stepper charge is set once from the start parameters and never
     // updated (the checkpoints do not carry it)
     const double charge = (a.start_params[(size_t)4 * a.n + i] > 0.0) ? 1.0 : -1.0;
+    // the measured plane that ends the segment and its hit, from the
+    // checkpoint written there (searching the track's hits for every plane
+    // passed was most of the sweep on long tracks); the next segment's are
+    // read with its own checkpoint
+    int plane = tf.seqFirst + (int)*tf.recC(nmeas - 1, KF_CK_NEXT) - 1;
+    int hitRel = (int)*tf.recC(nmeas - 1, KF_CK_HIT);
+    zeroPlanes(plane - tf.seqFirst + 1, slots);
     for (int k = nmeas - 1; k >= 0 && st == 0; --k) {
       // ---- recompute segment k from the checkpoint of surface k - 1
       tf.result = true;
@@ -1031,6 +1054,7 @@ struct TrackAdjoint {
       tf.stepFailed = false;
       tf.targetReached = false;
       tf.cur = -1;
+      int planePrev = tf.seqFirst - 1, hitPrev = 0;
       if (k == 0) {
         double pv[6];
 #pragma unroll
@@ -1042,20 +1066,23 @@ struct TrackAdjoint {
         tf.next = 0;
         tf.start(pv);
         tf.navStatus();
-        if (tf.cur >= 0 && hitOn(tf.cur) >= 0) {  // measured without a step
+        if (tf.cur == plane) {  // measured without a step
           st |= KF_ADJ_LOST;
           break;
         }
       } else {
         tf.loadCheckpoint(k - 1);
+        hitPrev = (int)*tf.recC(k - 1, KF_CK_HIT);
+        planePrev = tf.seqFirst + tf.next - 1;
         tf.q = charge;
         tf.measured = k;
       }
+      const int64_t hit = tf.h0 + hitRel;
+      zeroPlanes(planePrev - tf.seqFirst + 1, plane - tf.seqFirst);
       tf.pathLimit();
       tf.navTarget();
       const double qop = tf.q / tf.p;
       int nst = 0;
-      int plane = -1;
       for (;;) {
         if (nst >= g.max_seg_steps) {
           st |= KF_ADJ_OVERFLOW;
@@ -1080,10 +1107,7 @@ struct TrackAdjoint {
         *sr(nst, kSR_TGT) = (target >= 0 && h == tf.ss.v[kActor]) ? (double)(target + 1) : 0.0;
         ++nst;
         tf.navStatus();
-        if (tf.cur >= 0 && hitOn(tf.cur) >= 0) {
-          plane = tf.cur;
-          break;
-        }
+        if (tf.cur == plane) break;
         if (tf.pathLimit()) {
           st |= KF_ADJ_LOST;
           break;
@@ -1096,8 +1120,7 @@ struct TrackAdjoint {
       }
       if (st) break;
       // ---- bound state, chi2, update at the measured plane
-      const DevPlane &pl = a.planes[plane];
-      const int64_t hit = hitOn(plane);
+      const DevPlane &pl = tf.pls[plane];
       double dEnd[3], posEnd[3], k4[3], AEnd[3][5], GEnd[3][3];
 #pragma unroll
       for (int m = 0; m < 3; ++m) {
@@ -1147,9 +1170,9 @@ struct TrackAdjoint {
       // adjoint of the momentum after the plane from that of q/p
       const double pAfterb = -qb * tf.q / (Mt.pOut * Mt.pOut);
       double dbm[3] = {db[0], db[1], db[2]}, nbm[3] = {0, 0, 0};
-      const double pFb = Mt.vjp(a, pl, dF, pAfterb, lds[(kLDS_CB + 12) * KF_BLOCK],
-                                lds[(kLDS_CB + 18) * KF_BLOCK], lds[(kLDS_CB + 24) * KF_BLOCK],
-                                dbm, nbm);
+      const double pFb = Mt.vjp(a, pl, dF, pAfterb, lds[(kLDS_CB + cidx(2, 2)) * KF_BLOCK],
+                                lds[(kLDS_CB + cidx(3, 3)) * KF_BLOCK],
+                                lds[(kLDS_CB + cidx(4, 4)) * KF_BLOCK], dbm, nbm);
 #pragma unroll
       for (int m = 0; m < 3; ++m) Rb[m][2] += nbm[m];
       double xfb[5] = {0, 0, 0, 0, 0};
@@ -1161,23 +1184,23 @@ struct TrackAdjoint {
 #pragma unroll
         for (int r = 0; r < 5; ++r)
 #pragma unroll
-          for (int c = 0; c < 5; ++c) Cb[r][c] = lds[(kLDS_CB + 5 * r + c) * KF_BLOCK];
+          for (int c = 0; c < 5; ++c) Cb[r][c] = lds[(kLDS_CB + cidx(r, c)) * KF_BLOCK];
         P.vjp(dEnd, posEnd, AEnd, k4, xfb, Cb, posb, dbb, Abb, Gbb, k4b, qbb, Cmb, cb2, Rb2);
       }
 #pragma unroll
       for (int m = 0; m < 3; ++m) {
-        cb[m] += cb2[m];
         dbb[m] += dPre[m];
+        lds[(kLDS_PL + kPG_C + m) * KF_BLOCK] = cb[m] + cb2[m];
 #pragma unroll
-        for (int c = 0; c < 3; ++c) Rb[m][c] += Rb2[m][c];
+        for (int c = 0; c < 3; ++c)
+          lds[(kLDS_PL + kPG_R + 3 * m + c) * KF_BLOCK] = Rb[m][c] + Rb2[m][c];
       }
-      addPlane(plane, cb, Rb);
       // the covariance adjoint waits in LDS while the steps are reversed; the
       // Jacobian adjoints are kept there during the loop
 #pragma unroll
       for (int r = 0; r < 5; ++r)
 #pragma unroll
-        for (int c = 0; c < 5; ++c) lds[(kLDS_CB + 5 * r + c) * KF_BLOCK] = Cmb[r][c];
+        for (int c = r; c < 5; ++c) lds[(kLDS_CB + cidx(r, c)) * KF_BLOCK] = Cmb[r][c];
 #pragma unroll
       for (int r = 0; r < 3; ++r) {
 #pragma unroll
@@ -1195,7 +1218,7 @@ struct TrackAdjoint {
         }
         const double h = *sr(j, kSR_H);
         const int tgt = (int)*sr(j, kSR_TGT) - 1;
-        StepFwd F;
+        StepFwd<FK> F;
         F.run(a.field, pin, din, h, qop, ldf);
         double hb = 0.0;
         stepVJP(a.field, F, pin, din, h, qop, sr(j, kSR_G), 64u, posb, dbb, lds, k4b, hb, qbb,
@@ -1204,21 +1227,36 @@ struct TrackAdjoint {
         for (int m = 0; m < 3; ++m) k4b[m] = 0.0;
         if (tgt >= 0) {
           // h = n . (c - pos) / (n . d) towards plane tgt
-          const DevPlane &tp = a.planes[tgt];
+          const DevPlane &tp = tf.pls[tgt];
           const double n[3] = {tp.r[2], tp.r[5], tp.r[8]};
           const double den = n[0] * din[0] + n[1] * din[1] + n[2] * din[2];
+          const double hd = divD(hb, den);
           double tcb[3], tRb[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
 #pragma unroll
           for (int m = 0; m < 3; ++m) {
-            const double g1 = hb * n[m] / den;
+            const double g1 = hd * n[m];
             posb[m] -= g1;
             dbb[m] -= g1 * h;
             tcb[m] = g1;
-            tRb[m][2] = hb * ((tp.c[m] - pin[m]) - h * din[m]) / den;
+            tRb[m][2] = hd * ((tp.c[m] - pin[m]) - h * din[m]);
           }
-          addPlane(tgt, tcb, tRb);
+          if (tgt == plane) {
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+              lds[(kLDS_PL + kPG_C + m) * KF_BLOCK] += tcb[m];
+              lds[(kLDS_PL + kPG_R + 3 * m + 2) * KF_BLOCK] += tRb[m][2];
+            }
+          } else {
+            addPlane(tgt, tcb, tRb);
+          }
         }
       }
+      if (plane - tf.seqFirst < g.max_seq) {
+#pragma unroll
+        for (int f = 0; f < kPG_N; ++f) *pg(plane - tf.seqFirst, f) = lds[(kLDS_PL + f) * KF_BLOCK];
+      }
+      plane = planePrev;
+      hitRel = hitPrev;
       // ---- adjoint of the state after the update at the previous surface
 #pragma unroll
       for (int m = 0; m < 3; ++m) {
@@ -1228,8 +1266,7 @@ struct TrackAdjoint {
       qb = qbb;
     }
     if (st) {
-      for (int q = 0; q < slots; ++q)
-        for (int f = 0; f < kPG_N; ++f) *pg(q, f) = 0.0;
+      zeroPlanes(0, slots);
       sb = 0.0;
     }
     g.scale_adj[loc] = sb;

@@ -379,13 +379,13 @@ int setupArgs(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt, const cha
 constexpr size_t kCarryBytes = KF_CARRY_I * sizeof(int32_t) + KF_CARRY_D * sizeof(double);
 
 // Working-buffer bytes per track of the recording fit: per-state stores and
-// hand-over.
+// hand-over (the adjoint's forward pass: its checkpoints only).
 size_t storeBytesPerTrack(const kfd::FitArgs &a, int precision, bool track_states,
                           bool checkpoints) {
+  if (checkpoints) return (size_t)a.max_states * KF_CK_N * sizeof(double);
   const size_t s_size = (precision == KF_PRECISION_FP64) ? sizeof(double) : sizeof(float);
   size_t per_state = KF_SD_N * sizeof(double) + KF_SS_N * s_size;
   if (track_states) per_state += KF_TS_STRIDE * sizeof(double);
-  if (checkpoints) per_state += KF_CK_N * sizeof(double);
   return (size_t)a.max_states * per_state + kCarryBytes;
 }
 
@@ -418,11 +418,11 @@ StoreLayout storeLayout(int precision, bool track_states, bool checkpoints, int6
   const size_t slots = ((size_t)slice + 63) / 64 * 64 * (size_t)max_states;
   const size_t s_size = (precision == KF_PRECISION_FP64) ? sizeof(double) : sizeof(float);
   StoreLayout L;
-  L.s_bytes = (slots * KF_SS_N * s_size + 255) / 256 * 256;
-  L.d_bytes = slots * KF_SD_N * sizeof(double);
+  L.s_bytes = checkpoints ? 0 : (slots * KF_SS_N * s_size + 255) / 256 * 256;
+  L.d_bytes = checkpoints ? 0 : slots * KF_SD_N * sizeof(double);
   L.f_bytes = track_states ? slots * KF_TS_STRIDE * sizeof(double) : 0;
   L.c_bytes = checkpoints ? slots * KF_CK_N * sizeof(double) : 0;
-  L.carry_bytes = ((size_t)slice * kCarryBytes + 255) / 256 * 256;
+  L.carry_bytes = checkpoints ? 0 : ((size_t)slice * kCarryBytes + 255) / 256 * 256;
   return L;
 }
 
@@ -431,8 +431,8 @@ StoreLayout storeLayout(int precision, bool track_states, bool checkpoints, int6
 void carveStores(const StoreLayout &L, void *store, void *carry, bool track_states,
                  bool checkpoints, kfd::FitArgs &a) {
   char *base = (char *)store;
-  a.tss = base;
-  a.tsd = (double *)(base + L.s_bytes);
+  a.tss = checkpoints ? nullptr : base;
+  a.tsd = checkpoints ? nullptr : (double *)(base + L.s_bytes);
   a.tsf = track_states ? (double *)(base + L.s_bytes + L.d_bytes) : nullptr;
   a.tsc = checkpoints ? (double *)(base + L.s_bytes + L.d_bytes + L.f_bytes) : nullptr;
   // [field][count] of each slice (sliceCarry)
@@ -524,7 +524,7 @@ int setupFused(kf_ctx *ctx, int precision, int64_t slice, hipStream_t s, kfd::Fi
 void sliceRange(kfd::FitArgs &a, int64_t first, int64_t count) {
   a.first = first;
   a.count = count;
-  if (!a.redo) a.carry_i = (int32_t *)(a.carry_d + KF_CARRY_D * (size_t)count);
+  if (!a.redo && a.carry_d) a.carry_i = (int32_t *)(a.carry_d + KF_CARRY_D * (size_t)count);
 }
 
 // The whole fit of a batch: the length sort over all positions, then the
@@ -857,10 +857,10 @@ int kf_chi2_gradient(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt, do
   if (rc != KF_OK) return rc;
   const size_t sl = (size_t)(slice > 0 ? slice : 1);
   const size_t chunks = (sl + 63) / 64;
-  // forward outputs of the batch (params, cov, chi2, ndf, n_measured,
-  // status) and flags; per slice: step stack, plane adjoints, field-scale
+  // forward outputs of the batch that the sweep and the sums read (chi2,
+  // n_measured) and flags; per slice: step stack, plane adjoints, field-scale
   // adjoints; the sums
-  const size_t b_out = n * (6 + 21 + 1) * sizeof(double) + n * 3 * sizeof(int32_t);
+  const size_t b_out = n * sizeof(double) + n * sizeof(int32_t);
   const size_t b_stack = chunks * 64 * (size_t)max_seg * kfd::kSR_N * sizeof(double);
   const size_t b_pg = nplanes * kfd::kPG_N * sl * sizeof(double);
   const size_t b_scale = sl * sizeof(double);
@@ -873,12 +873,8 @@ int kf_chi2_gradient(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt, do
             "adjoint buffers");
   if (rc != KF_OK) return rc;
   char *p = (char *)ctx->adj;
-  a.out_params = (double *)p;
-  a.out_cov = a.out_params + 6 * n;
-  a.out_chi2 = a.out_cov + 21 * n;
-  a.out_ndf = (int32_t *)(a.out_chi2 + n);
-  a.out_nmeas = a.out_ndf + n;
-  a.out_status = (uint32_t *)(a.out_nmeas + n);
+  a.out_chi2 = (double *)p;
+  a.out_nmeas = (int32_t *)(a.out_chi2 + n);
   p += al(b_out);
   kfd::AdjArgs g;
   g.stack = (double *)p;

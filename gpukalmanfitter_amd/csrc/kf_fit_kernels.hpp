@@ -20,8 +20,8 @@ struct ChunkBases {
   KFD_INLINE ChunkBases(const FitArgs &a, int64_t i) {
     const size_t chunk = __builtin_amdgcn_readfirstlane((uint32_t)(i >> 6));
     const size_t per = (size_t)a.max_states * 64u;
-    d = a.tsd + chunk * per * KF_SD_N;
-    s = (S *)a.tss + chunk * per * KF_SS_N;
+    d = a.tsd ? a.tsd + chunk * per * KF_SD_N : nullptr;
+    s = a.tss ? (S *)a.tss + chunk * per * KF_SS_N : nullptr;
     f = a.tsf ? a.tsf + chunk * per * KF_TS_STRIDE : nullptr;
     c = a.tsc ? a.tsc + chunk * per * KF_CK_N : nullptr;
   }
@@ -59,12 +59,14 @@ KFD_INLINE void fitPosition(const FitArgs &a, int64_t local, uint32_t rank,
 // position, a wave covers 64 / L positions of one 64-position store chunk.
 // PS: store slots by plane position (kf_schedule.store_by_plane; one lane
 // per track).
-// FK, KEEP: the field kind and what is kept of the states.  A fit that asks
-// for neither track states nor checkpoints runs, in the mixed mode, on
-// (kFieldConst, kKeepStates) or (kFieldGrid, kKeepStates) for the batch's
-// field, so the step loop carries no code of the other field kind and the
-// filter none of the recording (FP64: kf_fused_kernel); every other one, and
-// plane tables read from global memory, on (kFieldAny, kKeepRecords).
+// FK, KEEP: the field kind and what is kept of the states.  The build is the
+// one for the batch's field, so the step loop carries no code of the other
+// kind, with kKeepRecords where track states are asked for and kKeepStates, the
+// mixed mode's, where not (FP64: kf_fused_kernel); plane tables read from
+// global memory run on (kFieldAny, kKeepRecords).  The chi2 adjoint's forward
+// pass is the kKeepCheckpoints build: without the smoother's store and with
+// the checkpoint's constant half left out it writes 248 B per state instead
+// of 1,000.
 template <typename S, bool FWD, bool LDS, bool PERS, int L, bool PS, int FK, int KEEP>
 __global__ void __launch_bounds__(KF_BLOCK) kf_fit_kernel(FitArgs args) {
   static_assert(L == 1 || !PERS, "lane groups run on the one-shot grid");
@@ -218,7 +220,27 @@ hipError_t launchFit(const FitArgs *args, hipStream_t stream, hipEvent_t between
       pers ? launch->persistent_blocks : (args->count * lpt + KF_BLOCK - 1) / KF_BLOCK;
   const dim3 grid((unsigned)blocks), block(KF_BLOCK);
   constexpr bool kFused = sizeof(S) == sizeof(double);
-  const bool rec = args->tsf != nullptr || args->tsc != nullptr;
+  const bool rec = args->tsf != nullptr;
+  if constexpr (kFused) {
+    if (args->tsc) {
+      const unsigned nb = (unsigned)((args->count + KF_BLOCK - 1) / KF_BLOCK);
+#define KFD_CHECKPOINTS(LDS_, FK_)                                                             \
+  hipLaunchKernelGGL((kf_fit_kernel<S, true, LDS_, false, 1, false, FK_, kKeepCheckpoints>), \
+                     dim3(nb), block, 0, stream, *args)
+      if (args->n_planes > KF_LDS_PLANES)
+        KFD_CHECKPOINTS(false, kFieldAny);
+      else if (args->field.grid)
+        KFD_CHECKPOINTS(true, kFieldGrid);
+      else
+        KFD_CHECKPOINTS(true, kFieldConst);
+#undef KFD_CHECKPOINTS
+      if (between) {
+        const hipError_t e = hipEventRecord(between, stream);
+        if (e != hipSuccess) return e;
+      }
+      return hipGetLastError();
+    }
+  }
   if (!kFused || rec) {
     const bool lds = args->n_planes <= KF_LDS_PLANES;
 #define KFD_LAUNCH2(FWD_, LDS_, PERS_, L_, PS_, FK_, KEEP_)                                     \
@@ -250,8 +272,10 @@ hipError_t launchFit(const FitArgs *args, hipStream_t stream, hipEvent_t between
         break;                                                \
       }                                                       \
     }                                                         \
-    if (lds)                                                  \
-      KFD_LAUNCH1(FWD_, true, kFieldAny, kKeepRecords);       \
+    if (lds && args->field.grid)                              \
+      KFD_LAUNCH1(FWD_, true, kFieldGrid, kKeepRecords);      \
+    else if (lds)                                             \
+      KFD_LAUNCH1(FWD_, true, kFieldConst, kKeepRecords);     \
     else                                                      \
       KFD_LAUNCH1(FWD_, false, kFieldAny, kKeepRecords);      \
   } while (0)

@@ -45,17 +45,21 @@
 #define KF_CARRY_I 8
 #define KF_CARRY_D 30
 // per-surface checkpoints of the chi2 adjoint (state after the update and
-// material at a measured surface; see FitArgs::tsc)
+// material at a measured surface; see FitArgs::tsc).  Only what is not a
+// constant there: the Jacobian was re-initialised on the surface, so its
+// position rows are the plane's axes and five of its direction entries are
+// free; the chi2 never sees the time row of the covariance; the aborter and
+// user limits of the step are fixed.
 #define KF_CK_POS 0    // 3
 #define KF_CK_DIR 3    // 3
 #define KF_CK_P 6
-#define KF_CK_T 7
-#define KF_CK_PATH 8
-#define KF_CK_SS 9     // ConstrainedStep values (4)
-#define KF_CK_COV 13   // 21
-#define KF_CK_J 34     // A (15), b, G (9)
-#define KF_CK_NEXT 59  // navigation index (as a double)
-#define KF_CK_N 60
+#define KF_CK_ACC 7    // ConstrainedStep: accuracy and actor values
+#define KF_CK_ACT 8
+#define KF_CK_COV 9    // spatial 5x5 (15, packed upper triangle)
+#define KF_CK_G 24     // Jacobian direction rows: (0,0) (0,1) (1,0) (1,1) (2,1)
+#define KF_CK_NEXT 29  // navigation index (as a double)
+#define KF_CK_HIT 30   // index of the surface's hit within the track (as a double)
+#define KF_CK_N 31
 
 namespace kfd {
 
@@ -188,7 +192,9 @@ struct KfdLaunch {
 };
 
 // Launches the fit of the positions args->first .. first + count - 1.  With
-// track states or checkpoints (args->tsf, tsc) and in the mixed mode:
+// checkpoints (args->tsc; FP64, smoothing off): [work-queue reset] -> forward
+// kernel -> record `between`.  With track states (args->tsf) and in the mixed
+// mode:
 // [work-queue reset] -> forward kernel -> record `between` (if not NULL) ->
 // smoother/back-propagation kernel (unless smoothing is off) -> track-state
 // export (if track_states_out is not NULL).  FP64 without them: [work-queue

@@ -36,16 +36,18 @@ enum { kResumeNone = 0, kResumePreLoop = 1, kResumeInLoop = 2, kResumePostLoop =
 //                adjoint checkpoints where asked for;
 //  kKeepStates   the store only (both record stores are null at compile time
 //                and their writes not in the code);
+//  kKeepCheckpoints  the adjoint's checkpoints only (no smoother follows);
 //  kKeepFirst    only the smoothed state of the first measured surface is
 //                wanted (it is what propagates to the perigee): the forward
 //                pass carries a fixed-point smoother for it (below), nothing is
 //                stored per state, and one kernel runs the whole fit (runFused).
-enum { kKeepRecords = 0, kKeepStates = 1, kKeepFirst = 2 };
+enum { kKeepRecords = 0, kKeepStates = 1, kKeepFirst = 2, kKeepCheckpoints = 3 };
 template <typename S, bool FWD, int L = 1, bool PS = false, bool OOL = false, int FK = kFieldAny,
           int KEEP = kKeepRecords>
 struct TrackFit {
   static constexpr bool kRecords = KEEP == kKeepRecords;
-  static constexpr bool kStore = KEEP != kKeepFirst;
+  static constexpr bool kStore = KEEP == kKeepRecords || KEEP == kKeepStates;
+  static constexpr bool kFirst = KEEP == kKeepFirst;
   static constexpr bool kMixed = sizeof(S) < sizeof(double);
   const FitArgs &a;
   const int64_t i;
@@ -183,7 +185,7 @@ struct TrackFit {
   KFD_INLINE TrackFit(const FitArgs &args, int64_t idx, double *d_base, S *s_base, double *f_base,
                       double *c_base, uint32_t ln, int64_t carry_slot = 0)
       : a(args), i(idx), tsd(d_base), tss(s_base), tsf(kRecords ? f_base : nullptr),
-        tsc(kRecords ? c_base : nullptr), pls(args.planes), lane(ln), cpos(carry_slot), cslots(args.count),
+        tsc(kRecords || KEEP == kKeepCheckpoints ? c_base : nullptr), pls(args.planes), lane(ln), cpos(carry_slot), cslots(args.count),
         ciBase(args.carry_i), cdBase(args.carry_d) {}
 
   // The hand-over buffer of tracks fitted again after a fused fit.
@@ -268,7 +270,7 @@ struct TrackFit {
 
   // Checkpoint k: the state right after the update and material of measured
   // surface k, from which the adjoint recomputes the next segment.
-  KFD_INLINE void saveCheckpoint(int k) const {
+  KFD_INLINE void saveCheckpoint(int k, int64_t hit) const {
     if (!lead) return;
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
@@ -276,22 +278,20 @@ struct TrackFit {
       *recC(k, KF_CK_DIR + m) = dir[m];
     }
     *recC(k, KF_CK_P) = p;
-    *recC(k, KF_CK_T) = t;
-    *recC(k, KF_CK_PATH) = pathAcc;
+    *recC(k, KF_CK_ACC) = ss.v[kAccuracy];
+    *recC(k, KF_CK_ACT) = ss.v[kActor];
+    int m = 0;
 #pragma unroll
-    for (int m = 0; m < 4; ++m) *recC(k, KF_CK_SS + m) = ss.v[m];
+    for (int r = 0; r < 5; ++r)
 #pragma unroll
-    for (int m = 0; m < 21; ++m) *recC(k, KF_CK_COV + m) = cov[m];
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-      for (int c = 0; c < 5; ++c) *recC(k, KF_CK_J + 5 * r + c) = (double)A[r][c];
-    *recC(k, KF_CK_J + 15) = (double)b;
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) *recC(k, KF_CK_J + 16 + 3 * r + c) = (double)G[r][c];
+      for (int c = r; c < 5; ++c, ++m) *recC(k, KF_CK_COV + m) = cov[sidx(r, c)];
+    *recC(k, KF_CK_G + 0) = (double)G[0][0];
+    *recC(k, KF_CK_G + 1) = (double)G[0][1];
+    *recC(k, KF_CK_G + 2) = (double)G[1][0];
+    *recC(k, KF_CK_G + 3) = (double)G[1][1];
+    *recC(k, KF_CK_G + 4) = (double)G[2][1];
     *recC(k, KF_CK_NEXT) = (double)next;
+    *recC(k, KF_CK_HIT) = (double)(hit - h0);
   }
 
   KFD_INLINE void loadCheckpoint(int k) {
@@ -301,25 +301,37 @@ struct TrackFit {
       dir[m] = *recC(k, KF_CK_DIR + m);
     }
     p = *recC(k, KF_CK_P);
-    t = *recC(k, KF_CK_T);
-    pathAcc = *recC(k, KF_CK_PATH);
-#pragma unroll
-    for (int m = 0; m < 4; ++m) ss.v[m] = *recC(k, KF_CK_SS + m);
+    t = 0.0;
+    pathAcc = 0.0;
+    ss.init(1.0 * fabs(a.max_step_size));
+    ss.v[kAccuracy] = *recC(k, KF_CK_ACC);
+    ss.v[kActor] = *recC(k, KF_CK_ACT);
     ss.dir = 1;
     navDir = 1;
     moved();
 #pragma unroll
-    for (int m = 0; m < 21; ++m) cov[m] = *recC(k, KF_CK_COV + m);
+    for (int m = 0; m < 21; ++m) cov[m] = (S)0;
+    int m = 0;
 #pragma unroll
-    for (int r = 0; r < 3; ++r)
+    for (int r = 0; r < 5; ++r)
 #pragma unroll
-      for (int c = 0; c < 5; ++c) A[r][c] = (S)*recC(k, KF_CK_J + 5 * r + c);
-    b = (S)*recC(k, KF_CK_J + 15);
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) G[r][c] = (S)*recC(k, KF_CK_J + 16 + 3 * r + c);
+      for (int c = r; c < 5; ++c, ++m) cov[sidx(r, c)] = *recC(k, KF_CK_COV + m);
     next = (int)*recC(k, KF_CK_NEXT);
+    const DevPlane &pl = pls[seqFirst + next - 1];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      A[r][0] = (S)pl.r[3 * r + 0];
+      A[r][1] = (S)pl.r[3 * r + 1];
+      A[r][2] = A[r][3] = A[r][4] = (S)0;
+      G[r][2] = (S)0;
+    }
+    b = (S)0;
+    G[0][0] = (S)*recC(k, KF_CK_G + 0);
+    G[0][1] = (S)*recC(k, KF_CK_G + 1);
+    G[1][0] = (S)*recC(k, KF_CK_G + 2);
+    G[1][1] = (S)*recC(k, KF_CK_G + 3);
+    G[2][0] = (S)0;
+    G[2][1] = (S)*recC(k, KF_CK_G + 4);
     derivSet = false;
     k4d[0] = k4d[1] = k4d[2] = (S)0;
     dtds = (S)0;
@@ -339,13 +351,14 @@ struct TrackFit {
   // -------------------------------------------------------------- field ----
   // FK: the field kind the kernel was built for (kFieldConst and
   // kFieldGrid leave the other kind's code out of the step loop)
-  // The grid cell of the last lookup; only in the grid builds (the either-kind
-  // builds are at the register limit, its 26 registers cost them 7 %).
+  // The grid cell of the last lookup; only in the fits' grid builds (the
+  // either-kind builds and the adjoint are at the register limit, its 26
+  // registers cost them 7 %).
   GridCell cell;
   KFD_INLINE void field(const double x[3], double B[3]) {
     if constexpr (FK == kFieldConst)
       fieldConst(a.field, B);
-    else if constexpr (FK == kFieldGrid)
+    else if constexpr (FK == kFieldGrid && !OOL)
       fieldGrid(a.field, x[0], x[1], x[2], B, cell);
     else
       fieldAt(a.field, x[0], x[1], x[2], B);
@@ -1605,7 +1618,7 @@ struct TrackFit {
 #pragma unroll
       for (int m = KF_SS_LINK + 1; m < KF_SS_CF - KF_SS_J; ++m) jv[m] = (S)0;
       storeS<KF_SS_CF - KF_SS_J>(s, KF_SS_J, jv);
-    } else {
+    } else if constexpr (kFirst) {
       if (k == 0)
         fxInit();
       else
@@ -1629,7 +1642,7 @@ struct TrackFit {
     const double r0 = m0 - xp[0], r1 = m1 - xp[1];
     const double chi2 = r0 * (i00 * r0 + i01 * r1) + r1 * (i10 * r0 + i11 * r1);
     double xf[6];
-    if constexpr (!kStore) {
+    if constexpr (kFirst) {
       // the predicted covariance and the hit's are positive definite, and the
       // hit is not so much more precise that the update loses definiteness
       fxOk = fxOk && (S)0 < cov[sidx(0, 0)] && (S)0 < cov[sidx(1, 1)] && (S)0 < cov[sidx(2, 2)] &&
@@ -1653,7 +1666,7 @@ struct TrackFit {
     }
 #pragma unroll
     for (int r = 0; r < 6; ++r) xf[r] = xp[r] + (K0[r] * r0 + K1[r] * r1);
-    if constexpr (!kStore) {
+    if constexpr (kFirst) {
       if (k > 0) fxMeasure(K0, K1, i00, i01, i11, i00 * r0 + i01 * r1, i10 * r0 + i11 * r1);
     }
     // the update in place on cov: rows 0 and 1 of the result go to t01 first
@@ -1707,7 +1720,7 @@ struct TrackFit {
     for (int c = 1; c < 6; ++c) cov[sidx(1, c)] = (S)t01[5 + c];
     chi2sum = chi2sum + chi2;
     }
-    if constexpr (!kStore) {
+    if constexpr (kFirst) {
       const double ap = fabs(xf[2]), at = fabs(xf[3] - 0.5 * kPi);
       fxPhi = (ap < fxPhi) ? fxPhi : ap;
       fxTheta = (at < fxTheta) ? fxTheta : at;
@@ -1717,7 +1730,7 @@ struct TrackFit {
     correctParams(xf);
     if constexpr (kStore) {
       storePar(s, KF_SD_XF, xf);
-    } else {
+    } else if constexpr (kFirst) {
       if (k == 0) fxKeepFirst(xf);
     }
     if (tsf && lead) {
@@ -1741,7 +1754,7 @@ struct TrackFit {
       cm[KF_SS_MD - KF_SS_CF + 2] = cov[sidx(4, 4)];
       storeS<KF_SS_N - KF_SS_CF>(s, KF_SS_CF, cm);
     }
-    if (tsc) saveCheckpoint(k);
+    if (tsc) saveCheckpoint(k, hit);
     if constexpr (PS) {
       slotPrev = slotLast;
       slotLast = s;
@@ -2208,7 +2221,7 @@ struct TrackFit {
     // (its code is most of the kernel): `at` says which of the three this is.
     int resume = kResumeNone;
     if (!bad) {
-      if constexpr (!kStore) fxOk = fxDefinite();
+      if constexpr (kFirst) fxOk = fxDefinite();
       prefetchHit();
       start(pv);
       navStatus();
@@ -2286,7 +2299,7 @@ struct TrackFit {
     if (resume != kResumeNone) {
       saveCarry(resume, steps, terminated);
     } else {
-      if (lead) ci(kCI_resume) = kResumeNone;
+      if (kStore && lead) ci(kCI_resume) = kResumeNone;
       writeFinal(bad ? KF_STATUS_BAD_INPUT : statusBits(steps, terminated), false);
     }
   }
