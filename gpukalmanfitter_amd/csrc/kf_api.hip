@@ -390,13 +390,14 @@ size_t storeBytesPerTrack(const kfd::FitArgs &a, int precision, bool track_state
 }
 
 // Whether a fit runs on the fused kernel (kf_fit_kernels.hpp).
-bool fitIsFused(int precision, bool track_states) {
-  return precision == KF_PRECISION_FP64 && !track_states;
-}
+bool fitIsFused(bool track_states) { return !track_states; }
 
-// Working-buffer bytes per track of the fused fit: the kept first state and
-// the redo list.
-constexpr size_t kFusedBytesPerTrack = KF_FIRST_D * sizeof(double) + sizeof(uint32_t);
+// Working-buffer bytes per track of the fused fit: the kept first state (FP64;
+// the mixed mode has it in LDS) and the redo list.
+size_t firstBytes(int precision) {
+  return precision == KF_PRECISION_FP64 ? KF_FIRST_D * sizeof(double) : 0;
+}
+size_t fusedBytesPerTrack(int precision) { return firstBytes(precision) + sizeof(uint32_t); }
 
 // Positions per slice: the largest multiple of 64 whose working set fits the
 // budget (at least 64), or the whole batch.
@@ -466,7 +467,7 @@ FusedLayout fusedLayout(int precision, int64_t slice, int64_t waves, int32_t max
   FusedLayout F;
   F.lanes = waves * 64;
   F.store = storeLayout(precision, false, false, F.lanes, max_states);
-  F.carry_bytes = ((size_t)slice * KF_FIRST_D * sizeof(double) + 255) / 256 * 256;
+  F.carry_bytes = ((size_t)slice * firstBytes(precision) + 255) / 256 * 256;
   F.list_bytes = ((KF_REDO_LIST + (size_t)slice) * sizeof(uint32_t) + 255) / 256 * 256;
   return F;
 }
@@ -581,7 +582,7 @@ int kf_fit_noalloc(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt,
     return fail(ctx, KF_E_HIP, "kf_fit_noalloc: workspace of device %d unavailable: %s",
                 ctx->device, hipGetErrorString(we));
   const bool ts = res->track_states != nullptr;
-  const bool fusedFit = fitIsFused(opt->precision, ts);
+  const bool fusedFit = fitIsFused(ts);
   // a fused fit: the redo store takes at most half of the workspace (one
   // chunk as a minimum)
   auto fused = [&](int64_t slice) {
@@ -653,9 +654,10 @@ int kf_fit(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt, const kf_res
   if (rc != KF_OK || tr->n_tracks == 0) return rc;
   hipStream_t s = (hipStream_t)stream;
   const bool ts = res->track_states != nullptr;
-  const bool fused = fitIsFused(opt->precision, ts);
+  const bool fused = fitIsFused(ts);
   const int64_t slice = sliceTracks(
-      ctx, a.n, fused ? kFusedBytesPerTrack : storeBytesPerTrack(a, opt->precision, ts, false));
+      ctx, a.n,
+      fused ? fusedBytesPerTrack(opt->precision) : storeBytesPerTrack(a, opt->precision, ts, false));
   rc = fused ? setupFused(ctx, opt->precision, slice, s, a)
              : setupStores(ctx, opt->precision, ts, false, slice, s, a);
   if (rc != KF_OK) return rc;

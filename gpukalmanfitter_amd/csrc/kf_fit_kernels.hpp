@@ -61,9 +61,9 @@ KFD_INLINE void fitPosition(const FitArgs &a, int64_t local, uint32_t rank,
 // per track).
 // FK, KEEP: the field kind and what is kept of the states.  The build is the
 // one for the batch's field, so the step loop carries no code of the other
-// kind, with kKeepRecords where track states are asked for and kKeepStates, the
-// mixed mode's, where not (FP64: kf_fused_kernel); plane tables read from
-// global memory run on (kFieldAny, kKeepRecords).  The chi2 adjoint's forward
+// kind, with kKeepRecords where track states are asked for (where not:
+// kf_fused_kernel); plane tables read from global memory run on (kFieldAny,
+// kKeepRecords).  The chi2 adjoint's forward
 // pass is the kKeepCheckpoints build: without the smoother's store and with
 // the checkpoint's constant half left out it writes 248 B per state instead
 // of 1,000.
@@ -101,19 +101,22 @@ __global__ void __launch_bounds__(KF_BLOCK) kf_fit_kernel(FitArgs args) {
   }
 }
 
-// The whole fit in one kernel, for FP64 fits that ask for neither track states
+// The whole fit in one kernel, for fits that ask for neither track states
 // nor checkpoints: forward filter with the fixed-point smoother, then back to
 // the perigee (TrackFit::runFused).  Per-track state in registers (one wave
-// per SIMD), the smoother's sums in LDS (46 KB per block), the plane table in
+// per SIMD), the smoother's sums in LDS (46 KB per block in FP64, 64 KB in the
+// mixed mode), the plane table in
 // dynamic LDS (PLDS) or global memory.  FK: the field kind, so the step loop
 // carries no code of the other one (either kind where the plane table is in
 // global memory).  PERS, L as in kf_fit_kernel.
 //
-// The mixed mode keeps the RTS kernels: its smoother starts from covariances
-// rounded to float, and the fixed-point sums, though no further from the
-// exact fit, do not round as the recursion over those does (1e-7 in the time
-// variance, single tracks 1e-4 mm in position where the perigee's on-surface
-// decision falls the other way).
+// Bound by instruction issue: a wave of ten planes issues 24,300 vector
+// instructions in FP64 (1,048,576 tracks: 1.32 ms) and ~40,000 in the mixed
+// mode, a third of them the RTS gain and its sums (TrackFit::fxRtsStep; the
+// FP64 sums round differently from the recursion over float covariances, 1e-7
+// in the time variance).  Mixed, against the forward and backward kernels that
+// passed 304 B per state through memory: 1,048,576 tracks 2.03 -> 1.75 ms,
+// 500,003 ragged ones 2.81 -> 2.30 ms, 100,003 with material 1.93 -> 1.70 ms.
 //
 // A track that the fixed-point smoother leaves to the RTS program (TrackFit::
 // fxSafe; 1 in 200,000 of the material workload) is fitted again by its own
@@ -219,9 +222,8 @@ hipError_t launchFit(const FitArgs *args, hipStream_t stream, hipEvent_t between
   const int64_t blocks =
       pers ? launch->persistent_blocks : (args->count * lpt + KF_BLOCK - 1) / KF_BLOCK;
   const dim3 grid((unsigned)blocks), block(KF_BLOCK);
-  constexpr bool kFused = sizeof(S) == sizeof(double);
   const bool rec = args->tsf != nullptr;
-  if constexpr (kFused) {
+  if constexpr (sizeof(S) == sizeof(double)) {
     if (args->tsc) {
       const unsigned nb = (unsigned)((args->count + KF_BLOCK - 1) / KF_BLOCK);
 #define KFD_CHECKPOINTS(LDS_, FK_)                                                             \
@@ -241,7 +243,7 @@ hipError_t launchFit(const FitArgs *args, hipStream_t stream, hipEvent_t between
       return hipGetLastError();
     }
   }
-  if (!kFused || rec) {
+  if (rec) {
     const bool lds = args->n_planes <= KF_LDS_PLANES;
 #define KFD_LAUNCH2(FWD_, LDS_, PERS_, L_, PS_, FK_, KEEP_)                                     \
   hipLaunchKernelGGL((kf_fit_kernel<S, FWD_, LDS_, PERS_, L_, PS_, FK_, KEEP_>), grid, block, 0, \
@@ -263,15 +265,6 @@ hipError_t launchFit(const FitArgs *args, hipStream_t stream, hipEvent_t between
   } while (0)
 #define KFD_LAUNCH(FWD_)                                      \
   do {                                                        \
-    if constexpr (!kFused) {                                  \
-      if (lds && !rec) {                                      \
-        if (args->field.grid)                                 \
-          KFD_LAUNCH1(FWD_, true, kFieldGrid, kKeepStates);   \
-        else                                                  \
-          KFD_LAUNCH1(FWD_, true, kFieldConst, kKeepStates);  \
-        break;                                                \
-      }                                                       \
-    }                                                         \
     if (lds && args->field.grid)                              \
       KFD_LAUNCH1(FWD_, true, kFieldGrid, kKeepRecords);      \
     else if (lds)                                             \
@@ -291,38 +284,37 @@ hipError_t launchFit(const FitArgs *args, hipStream_t stream, hipEvent_t between
 #undef KFD_LAUNCH2
     return hipGetLastError();
   }
-  if constexpr (kFused) {
-    const bool plds = args->n_planes <= KF_FUSED_LDS_PLANES;
-    const dim3 fgrid((unsigned)((args->count * lpt + KF_FUSED_BLOCK - 1) / KF_FUSED_BLOCK));
-    const unsigned table = plds ? (unsigned)(args->n_planes * sizeof(DevPlane)) : 0u;
-#define KFD_FUSED2(PLDS_, L_, FK_)                                                     \
+  const bool plds = args->n_planes <= (sizeof(S) == sizeof(double) ? KF_FUSED_LDS_PLANES_FP64
+                                                                   : KF_FUSED_LDS_PLANES_MIXED);
+  const dim3 fgrid((unsigned)((args->count * lpt + KF_FUSED_BLOCK - 1) / KF_FUSED_BLOCK));
+  const unsigned table = plds ? (unsigned)(args->n_planes * sizeof(DevPlane)) : 0u;
+#define KFD_FUSED2(PLDS_, L_, FK_)                                                             \
   hipLaunchKernelGGL((kf_fused_kernel<S, PLDS_, L_, FK_>), fgrid, dim3(KF_FUSED_BLOCK), table, \
                      stream, *args)
-#define KFD_FUSED1(PLDS_, FK_)       \
-  do {                               \
-    if (lpt == 1)                    \
-      KFD_FUSED2(PLDS_, 1, FK_);     \
-    else if (lpt == 2)               \
-      KFD_FUSED2(PLDS_, 2, FK_);     \
-    else                             \
-      KFD_FUSED2(PLDS_, 4, FK_);     \
+#define KFD_FUSED1(PLDS_, FK_)     \
+  do {                             \
+    if (lpt == 1)                  \
+      KFD_FUSED2(PLDS_, 1, FK_);   \
+    else if (lpt == 2)             \
+      KFD_FUSED2(PLDS_, 2, FK_);   \
+    else                           \
+      KFD_FUSED2(PLDS_, 4, FK_);   \
   } while (0)
-    if (!plds)
-      KFD_FUSED1(false, kFieldAny);
-    else if (args->field.grid)
-      KFD_FUSED1(true, kFieldGrid);
-    else
-      KFD_FUSED1(true, kFieldConst);
+  if (!plds)
+    KFD_FUSED1(false, kFieldAny);
+  else if (args->field.grid)
+    KFD_FUSED1(true, kFieldGrid);
+  else
+    KFD_FUSED1(true, kFieldConst);
 #undef KFD_FUSED1
 #undef KFD_FUSED2
-    if (between) {
-      const hipError_t e = hipEventRecord(between, stream);
-      if (e != hipSuccess) return e;
-    }
-    if (args->smoothing)
-      hipLaunchKernelGGL((kf_redo_kernel<S>), dim3((unsigned)(args->redo_lanes / 64)), dim3(64), 0,
-                         stream, *args);
+  if (between) {
+    const hipError_t e = hipEventRecord(between, stream);
+    if (e != hipSuccess) return e;
   }
+  if (args->smoothing)
+    hipLaunchKernelGGL((kf_redo_kernel<S>), dim3((unsigned)(args->redo_lanes / 64)), dim3(64), 0,
+                       stream, *args);
   return hipGetLastError();
 }
 

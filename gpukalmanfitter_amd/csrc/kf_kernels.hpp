@@ -16,10 +16,11 @@
 #ifndef KF_FUSED_BLOCK
 #define KF_FUSED_BLOCK 128
 #endif
-// The same for the fused fit kernel, whose blocks also hold 46 KB of smoother
-// sums: the largest table with which two blocks (one wave per SIMD) still fit
-// the 160 KB of a compute unit.
-#define KF_FUSED_LDS_PLANES 224
+// The same for the fused fit kernel, whose blocks also hold the smoother's sums
+// (46 KB in FP64, 64 KB in the mixed mode): the largest tables with which two
+// blocks (one wave per SIMD) still fit the 160 KB of a compute unit.
+#define KF_FUSED_LDS_PLANES_FP64 224
+#define KF_FUSED_LDS_PLANES_MIXED 112
 // Store chunks for tracks that the fused kernel hands to the RTS program, and
 // the memory they may take together.
 #define KF_REDO_WAVES 256
@@ -137,8 +138,8 @@ struct FitArgs {
   int32_t persistent;
   int32_t chunks_per_grab;
   uint32_t *queue;
-  // Fused fits (FP64, no track states or checkpoints): carry_d holds the kept
-  // first states ([KF_FIRST_D][count]).  Tracks handed back to the RTS
+  // Fused fits (no track states or checkpoints): carry_d holds the kept
+  // first states of FP64 ([KF_FIRST_D][count]).  Tracks handed back to the RTS
   // program use tsd, tss (redo_lanes slots, one store chunk per wave) and
   // redo_d, redo_i ([KF_CARRY_D], [KF_CARRY_I][redo_lanes]).  redo[0]: store
   // chunks taken by waves of the fused kernel itself, redo[1]: positions
@@ -193,11 +194,10 @@ struct KfdLaunch {
 
 // Launches the fit of the positions args->first .. first + count - 1.  With
 // checkpoints (args->tsc; FP64, smoothing off): [work-queue reset] -> forward
-// kernel -> record `between`.  With track states (args->tsf) and in the mixed
-// mode:
+// kernel -> record `between`.  With track states (args->tsf):
 // [work-queue reset] -> forward kernel -> record `between` (if not NULL) ->
 // smoother/back-propagation kernel (unless smoothing is off) -> track-state
-// export (if track_states_out is not NULL).  FP64 without them: [work-queue
+// export (if track_states_out is not NULL).  Without them: [work-queue
 // reset] -> fused kernel -> record `between` -> redo kernel.  `launch` may be NULL (one thread per
 // track, identity order).  With a persistent grid, args->queue and
 // args->chunks_per_grab must be set; with sorting, args->order.

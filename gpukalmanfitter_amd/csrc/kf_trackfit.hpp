@@ -776,10 +776,10 @@ struct TrackFit {
 #pragma unroll
     for (int k = 0; k < 3; ++k) dk4dL[k] = c1[k] + (qop * h) * c2[k];
 
-    // divisions: a float 1/6 constant is biased by 3e-8 relative, which
+    // quotients: a float 1/6 constant is biased by 3e-8 relative, which
     // accumulates over the steps of a track
-    const S h6 = h / (S)6.0;
-    const S hh6 = (h * h) / (S)6.0;
+    const S h6 = sixthOf(h);
+    const S hh6 = sixthOf(h * h);
     S dFdT[3][3], dGdT[3][3], dFdL[3], dGdL[3];
     if constexpr (L == 1) {
       // dk/dT matrices (row r, column c)
@@ -882,6 +882,18 @@ struct TrackFit {
     }
   }
 
+  // x / 6 in float, correctly rounded: the product with the rounded 1/6 and one
+  // residual correction (Markstein's division theorem), 3 operations where the
+  // library's quotient takes ~10
+  KFD_INLINE static S sixthOf(S x) {
+    if constexpr (kMixed) {
+      const float q = x * (1.0f / 6.0f);
+      return fmaf(fmaf(-6.0f, q, x), 1.0f / 6.0f, q);
+    } else {
+      return x / (S)6.0;
+    }
+  }
+
   // qop * cross_cols(I + hh * M, B)  (Helpers.hpp:168-176)
   KFD_INLINE static void crossStep(const S M[3][3], S hh, const S B[3], S qop, S out[3][3]) {
 #pragma unroll
@@ -908,12 +920,12 @@ struct TrackFit {
   // Filtering, 1979, section 7.2).  In exact arithmetic it is the RTS
   // recursion's result for state 0; the time parameter never acts on the
   // spatial ones, so T is 5x5.  Per state ~210 multiply-adds and no memory,
-  // against ~1,100 and 512 B (mixed: 304 B) written and read back for the RTS
+  // against ~1,100 and 512 B written and read back for the RTS
   // step, whose 6x6 solve also loses more digits than the sums here.
   //
-  // T, lambda and Lambda are double in both modes and sit in LDS (kFxN 16-byte
-  // pairs per lane, stride KF_FUSED_BLOCK: conflict-free 16-byte accesses), not in
-  // registers: they are used once per surface.
+  // T, lambda and Lambda sit in LDS (kFxN 16-byte pairs per lane, stride
+  // KF_FUSED_BLOCK: conflict-free 16-byte accesses), not in registers: they are
+  // used once per surface.
   //
   // Where the RTS recursion's discrete behaviour could show -- a phi wrap or a
   // theta clamp of a smoothed state, a gain that is not finite, a covariance
@@ -922,9 +934,22 @@ struct TrackFit {
   struct alignas(16) FxPair {
     double a, b;
   };
-  enum { kFxCol = 3, kFxSum = 15, kFxN = 23 };
+  enum { kFxCol = 3, kFxSum = 15 };
+  // The mixed mode's sums.  Its covariances are rounded to float between
+  // surfaces, so J C_f J^T is not exactly the predicted covariance and the
+  // identities above hold to 1e-7 only; the RTS gains G_k = C_f J^T C_p^-1 of
+  // the rounded matrices still give state 0 as sums over the later states:
+  // with P_k = G_0 G_1 ... G_(k-1),
+  //   x0 = x_f0 + sum P_k (x_fk - x_pk),  C0 = C_f0 + sum P_k (C_fk - C_pk) P_k^T,
+  // the recursion's result in exact arithmetic, whatever the matrices.  Per
+  // state the ~1,100 multiply-adds of the RTS step (the same gain, from the
+  // same numbers) and no memory.  P by rows of three pairs, then x0 and C0.
+  enum { kFxRow = 3, kFxX0 = 18, kFxC0 = 21 };
+  static constexpr bool kFxRts = kFirst && kMixed;
+  static constexpr int kFxN = kMixed ? 32 : 23;
   FxPair *fx = nullptr;  // this lane's first pair
   bool fxOk = true;
+  S fxDiag[3];                          // kFxRts: (2,2), (3,3), (4,4) before the material update
   S fxVphi = (S)0, fxVth = (S)0;        // largest filtered variances of phi and theta
   double fxPhi = 0.0, fxTheta = 0.0;    // largest |phi| and |theta - pi/2| of a filtered state
 
@@ -1006,7 +1031,94 @@ struct TrackFit {
 #pragma unroll
     for (int m = 0; m < 21; ++m) cd(6 + m) = (double)cov[m];
   }
+  // kFxRts: P = 1, x0 = x_f0, C0 = C_f0
+  KFD_INLINE void fxRtsInit(const double xf[6]) const {
+#pragma unroll
+    for (int r = 0; r < 6; ++r)
+#pragma unroll
+      for (int g = 0; g < 3; ++g)
+        fxStore(kFxRow * r + g, (r == 2 * g) ? 1.0 : 0.0, (r == 2 * g + 1) ? 1.0 : 0.0);
+#pragma unroll
+    for (int g = 0; g < 3; ++g) fxStore(kFxX0 + g, xf[2 * g], xf[2 * g + 1]);
+#pragma unroll
+    for (int g = 0; g < 11; ++g)
+      fxStore(kFxC0 + g, (double)cov[2 * g], (g < 10) ? (double)cov[2 * g + 1] : 0.0);
+  }
+  // kFxRts: a later state with the transport J from the filtered covariance cf
+  // of the state before, predicted x_p and C_p (cp), filtered x_f and C_f (cov)
+  KFD_INLINE void fxRtsStep(const S J[6][6], const S cf[21], const S cp[21], const double xp[6],
+                            const double xf[6]) {
+    double X[6][6];
+    {
+      double cfd[21], cpd[21];
+#pragma unroll
+      for (int m = 0; m < 21; ++m) {
+        cfd[m] = (double)cf[m];
+        cpd[m] = (double)cp[m];
+      }
+      transported(J, cfd, X);
+      fxOk = spdSolvePivots(cpd, X) && fxOk;
+    }
+    double P[6][6];
+#pragma unroll
+    for (int r = 0; r < 6; ++r) {
+      double t[6];
+#pragma unroll
+      for (int g = 0; g < 3; ++g) fxLoad(kFxRow * r + g, t[2 * g], t[2 * g + 1]);
+#pragma unroll
+      for (int c = 0; c < 6; ++c) {
+        double v = t[0] * X[c][0];
+#pragma unroll
+        for (int m = 1; m < 6; ++m) v = v + t[m] * X[c][m];
+        P[r][c] = v;
+      }
+#pragma unroll
+      for (int g = 0; g < 3; ++g) fxStore(kFxRow * r + g, P[r][2 * g], P[r][2 * g + 1]);
+    }
+    double x0[6], c0[22], D[21];
+#pragma unroll
+    for (int g = 0; g < 3; ++g) fxLoad(kFxX0 + g, x0[2 * g], x0[2 * g + 1]);
+#pragma unroll
+    for (int g = 0; g < 11; ++g) fxLoad(kFxC0 + g, c0[2 * g], c0[2 * g + 1]);
+#pragma unroll
+    for (int m = 0; m < 21; ++m) D[m] = (double)cov[m] - (double)cp[m];
+#pragma unroll
+    for (int r = 0; r < 6; ++r) {
+#pragma unroll
+      for (int c = 0; c < 6; ++c) x0[r] = x0[r] + P[r][c] * (xf[c] - xp[c]);
+      double w[6];  // row r of P (C_f - C_p)
+#pragma unroll
+      for (int c = 0; c < 6; ++c) {
+        double v = P[r][0] * D[sidx(0, c)];
+#pragma unroll
+        for (int m = 1; m < 6; ++m) v = v + P[r][m] * D[sidx(m, c)];
+        w[c] = v;
+      }
+#pragma unroll
+      for (int c = r; c < 6; ++c) {
+        double v = w[0] * P[c][0];
+#pragma unroll
+        for (int m = 1; m < 6; ++m) v = v + w[m] * P[c][m];
+        c0[sidx(r, c)] = c0[sidx(r, c)] + v;
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < 3; ++g) fxStore(kFxX0 + g, x0[2 * g], x0[2 * g + 1]);
+#pragma unroll
+    for (int g = 0; g < 11; ++g) fxStore(kFxC0 + g, c0[2 * g], c0[2 * g + 1]);
+  }
   KFD_INLINE void fxSmooth(double xs[6], double cs[21]) const {
+    if constexpr (kFxRts) {
+      double c0[22];
+#pragma unroll
+      for (int g = 0; g < 3; ++g) fxLoad(kFxX0 + g, xs[2 * g], xs[2 * g + 1]);
+#pragma unroll
+      for (int g = 0; g < 11; ++g) fxLoad(kFxC0 + g, c0[2 * g], c0[2 * g + 1]);
+#pragma unroll
+      for (int m = 0; m < 21; ++m) cs[m] = c0[m];
+      correctParams(xs);
+      return;
+    }
     double x0[6], c0[21];
 #pragma unroll
     for (int m = 0; m < 6; ++m) x0[m] = cd(m);
@@ -1603,7 +1715,19 @@ struct TrackFit {
     if (k == 0) firstPlane = sp;
     double xp[6];
     S jb[6][6];
+    S cfPrev[21], cPred[21];  // kFxRts
+    if constexpr (kFxRts) {
+#pragma unroll
+      for (int m = 0; m < 21; ++m) cfPrev[m] = cov[m];
+      cfPrev[sidx(2, 2)] = fxDiag[0];
+      cfPrev[sidx(3, 3)] = fxDiag[1];
+      cfPrev[sidx(4, 4)] = fxDiag[2];
+    }
     boundStatePlane(pl, xp, jb);
+    if constexpr (kFxRts) {
+#pragma unroll
+      for (int m = 0; m < 21; ++m) cPred[m] = cov[m];
+    }
     // predicted parameters and the transport Jacobian to the store, with the
     // slot of the state two measurements back (the smoother's look-ahead)
     if constexpr (kStore) {
@@ -1618,7 +1742,7 @@ struct TrackFit {
 #pragma unroll
       for (int m = KF_SS_LINK + 1; m < KF_SS_CF - KF_SS_J; ++m) jv[m] = (S)0;
       storeS<KF_SS_CF - KF_SS_J>(s, KF_SS_J, jv);
-    } else if constexpr (kFirst) {
+    } else if constexpr (kFirst && !kMixed) {
       if (k == 0)
         fxInit();
       else
@@ -1666,14 +1790,30 @@ struct TrackFit {
     }
 #pragma unroll
     for (int r = 0; r < 6; ++r) xf[r] = xp[r] + (K0[r] * r0 + K1[r] * r1);
-    if constexpr (kFirst) {
+    if constexpr (kFirst && !kMixed) {
       if (k > 0) fxMeasure(K0, K1, i00, i01, i11, i00 * r0 + i01 * r1, i10 * r0 + i11 * r1);
     }
     // the update in place on cov: rows 0 and 1 of the result go to t01 first
     // (every entry reads the old rows 0 and 1), then rows 2..5 overwrite
     // cov, then rows 0 and 1 are written back
     double t01[11];
-    if constexpr (kMixed) {
+    if (kFxRts && 1e-6 * (S00 * S11) < det) {
+      // the same matrix for the gain as computed here, (I - K H) P, with its
+      // rows 0 and 1 as K V: no cancellation in them, and the other entries
+      // cancel as in the Joseph form's first term.  First order in the error
+      // of K, so only where the innovation is well conditioned (an error of K
+      // below 1e-10, under the float rounding of the result); 42 operations
+      // for ~200
+#pragma unroll
+      for (int c = 0; c < 6; ++c) t01[c] = K0[c] * V00 + K1[c] * V01;
+#pragma unroll
+      for (int c = 1; c < 6; ++c) t01[5 + c] = K0[c] * V01 + K1[c] * V11;
+#pragma unroll
+      for (int r = 2; r < 6; ++r)
+#pragma unroll
+        for (int c = r; c < 6; ++c)
+          cov[sidx(r, c)] = (S)(cov[sidx(r, c)] - K0[r] * cov[sidx(0, c)] - K1[r] * cov[sidx(1, c)]);
+    } else if constexpr (kMixed) {
       // B = (I - K H) P: columns 0 and 1 here, the other (r <= c) entries
       // where they are consumed
       double B0[6], B1[6];
@@ -1730,6 +1870,16 @@ struct TrackFit {
     correctParams(xf);
     if constexpr (kStore) {
       storePar(s, KF_SD_XF, xf);
+    } else if constexpr (kFxRts) {
+      if (a.smoothing) {
+        if (k == 0)
+          fxRtsInit(xf);
+        else
+          fxRtsStep(jb, cfPrev, cPred, xp, xf);
+        fxDiag[0] = cov[sidx(2, 2)];
+        fxDiag[1] = cov[sidx(3, 3)];
+        fxDiag[2] = cov[sidx(4, 4)];
+      }
     } else if constexpr (kFirst) {
       if (k == 0) fxKeepFirst(xf);
     }
@@ -1832,6 +1982,70 @@ struct TrackFit {
     }
   }
 
+  // X = J C_f (C_f symmetric); row 4 of J is e4 and column 5 is e5.
+  KFD_INLINE static void transported(const S J[6][6], const double cf[21], double X[6][6]) {
+#pragma unroll
+    for (int r = 0; r < 6; ++r)
+#pragma unroll
+      for (int c = 0; c < 6; ++c) {
+        double s;
+        if (r == 4) {
+          s = cf[sidx(4, c)];
+        } else {
+          s = (double)J[r][0] * cf[sidx(0, c)];
+#pragma unroll
+          for (int m = 1; m < 5; ++m) s = s + (double)J[r][m] * cf[sidx(m, c)];
+          if (r == 5) s = s + cf[sidx(5, c)];
+        }
+        X[r][c] = s;
+      }
+  }
+
+  // spdSolve without the diagonal scaling (the pivots of L D L^T and what they
+  // lose do not depend on it, 130 of 430 operations), for the fixed-point sums.
+  // False where a pivot is not positive: such a track takes the RTS program,
+  // whose scaled solver decides what its gain is.
+  KFD_INLINE static bool spdSolvePivots(const double C[21], double M[6][6]) {
+    double Lo[6][6], W[6][6], Dinv[6];
+    bool ok = true;
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+      double dj = C[sidx(j, j)];
+#pragma unroll
+      for (int k = 0; k < j; ++k) dj = dj - W[j][k] * Lo[j][k];
+      ok = ok && 0.0 < dj;
+      Dinv[j] = recipD(dj);
+#pragma unroll
+      for (int r = j + 1; r < 6; ++r) {
+        double w = C[sidx(r, j)];
+#pragma unroll
+        for (int k = 0; k < j; ++k) w = w - W[r][k] * Lo[j][k];
+        W[r][j] = w;
+        Lo[r][j] = w * Dinv[j];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+      double y[6];
+#pragma unroll
+      for (int r = 0; r < 6; ++r) {
+        double v = M[r][c];
+#pragma unroll
+        for (int k = 0; k < r; ++k) v = v - Lo[r][k] * y[k];
+        y[r] = v;
+      }
+#pragma unroll
+      for (int r = 5; r >= 0; --r) {
+        double v = y[r] * Dinv[r];
+#pragma unroll
+        for (int k = r + 1; k < 6; ++k) v = v - Lo[k][r] * y[k];
+        y[r] = v;
+        M[r][c] = v;
+      }
+    }
+    return ok;
+  }
+
   // Filtered covariance of state k, in double.
   KFD_INLINE void loadFilteredCov(int k, double c[21]) const {
     S cm[KF_SS_N - KF_SS_CF];
@@ -1893,26 +2107,11 @@ struct TrackFit {
     double cf[21];
 #pragma unroll
     for (int m = 0; m < 21; ++m) cf[m] = (double)in.cf[m];
-    // G^T = C_p^-1 (J C_f) (C_f, C_p symmetric); row 4 of J is e4 and
-    // column 5 is e5
+    // G^T = C_p^-1 (J C_f) (C_p symmetric)
     double G[6][6];
     {
       double X[6][6];
-#pragma unroll
-      for (int r = 0; r < 6; ++r)
-#pragma unroll
-        for (int c = 0; c < 6; ++c) {
-          double s;
-          if (r == 4) {
-            s = cf[sidx(4, c)];
-          } else {
-            s = (double)J[r][0] * cf[sidx(0, c)];
-#pragma unroll
-            for (int m = 1; m < 5; ++m) s = s + (double)J[r][m] * cf[sidx(m, c)];
-            if (r == 5) s = s + cf[sidx(5, c)];
-          }
-          X[r][c] = s;
-        }
+      transported(J, cf, X);
       spdSolve(Cp, X);
 #pragma unroll
       for (int r = 0; r < 6; ++r)

@@ -5,9 +5,9 @@
 
 namespace {
 
-template <int FK>
+template <typename S, int FK>
 void fusedTracks(Host &h, int32_t *redo) {
-  using Fit = TrackFit<double, true, 1, false, false, FK, kKeepFirst>;
+  using Fit = TrackFit<S, true, 1, false, false, FK, kKeepFirst>;
   std::vector<typename Fit::FxPair> sums((size_t)Fit::kFxN * KF_FUSED_BLOCK);
   for (int64_t i = 0; i < h.a.n; ++i) {
     Fit tf(h.a, i, nullptr, nullptr, nullptr, nullptr, 0u, i);
@@ -22,7 +22,7 @@ void fusedTracks(Host &h, int32_t *redo) {
 extern "C" {
 
 // The fit of every track by the fused program, built for either field kind
-// (0), the constant field (1) or the grid (2): params [6][n], cov [21][n],
+// (0, the mixed mode's only), the constant field (1) or the grid (2): params [6][n], cov [21][n],
 // chi2, n_measured, status [n], and redo [n], nonzero for a track that it
 // leaves to the RTS program (its params, cov and status are not set).
 int kfh_fit_fused_kind(const kf_plane *planes, int32_t n_planes, const kfh_field *f,
@@ -36,12 +36,14 @@ int kfh_fit_fused_kind(const kf_plane *planes, int32_t n_planes, const kfh_field
   h.a.out_nmeas = n_measured;
   h.a.out_status = status;
   h.a.out_ndf = nullptr;
-  if (field_kind == kFieldGrid)
-    fusedTracks<kFieldGrid>(h, redo);
+  if (opt->precision == KF_PRECISION_MIXED)
+    fusedTracks<float, kFieldAny>(h, redo);
+  else if (field_kind == kFieldGrid)
+    fusedTracks<double, kFieldGrid>(h, redo);
   else if (field_kind == kFieldConst)
-    fusedTracks<kFieldConst>(h, redo);
+    fusedTracks<double, kFieldConst>(h, redo);
   else
-    fusedTracks<kFieldAny>(h, redo);
+    fusedTracks<double, kFieldAny>(h, redo);
   return 0;
 }
 

@@ -115,6 +115,31 @@ def test_fused_program_equals_rts_program(built, name, cfg, stay):
         assert (np.abs(f["params"][2, kept]) < np.pi).all()
 
 
+@pytest.mark.parametrize("name,cfg,stay", CASES)
+def test_mixed_fused_program_equals_rts_program(built, name, cfg, stay):
+    """The mixed mode's sums (RTS gains of the float covariances) against its RTS
+    program.  The float operations are the same and the rest is double, so the two
+    differ by 1e-13 and, where that turns the rounding of a float covariance entry
+    (one entry in a million), by what 6e-8 of it becomes: a tenth of the mode's
+    bars against the oracle."""
+    b = variant(name, 400, cfg)
+    opt = abi.default_options(precision=abi.KF_PRECISION_MIXED, **W)
+    f, r = fused_fit(b, opt), host_fit(b, opt)
+    kept = f["redo"] == 0
+    assert {"all": kept.all(), "none": not kept.any(),
+            "some": kept.any() and not kept.all()}[stay]
+    if not kept.any():
+        return
+    assert np.array_equal(f["n_measured"][kept], r["n_measured"][kept])
+    assert np.array_equal(f["status"][kept], r["status"][kept])
+    sig = np.sqrt(np.abs(r["cov"][abi.DIAG_INDEX]))[:, kept]
+    p = r["params"][:, kept]
+    assert (np.abs(f["params"][:, kept] - p) <= 1e-6 * np.maximum(np.abs(p), sig)).all()
+    for (i, j), k in abi.SYM_INDEX.items():
+        d = np.abs(f["cov"][k, kept] - r["cov"][k, kept])
+        assert (d <= 1e-4 * sig[i] * sig[j]).all(), (i, j)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,cfg,n", [("one plane", 1, 1), ("two planes", 1, 65),
                                         ("phi wrap", 1, 20000), ("no time variance", 1, 20000),
@@ -163,3 +188,50 @@ def test_gpu_fused_fit_with_handed_back_tracks(name, cfg, n, sched):
     pd, cd, c2 = compare_fit(g, o)
     bar = 1e-6 if name == "phi wrap" else 1e-10
     assert max(pd, cd, c2) <= bar, (pd, cd, c2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,cfg,n", [("one plane", 1, 1), ("two planes", 1, 65),
+                                        ("phi wrap", 1, 20000), ("no time variance", 1, 20000)])
+@pytest.mark.parametrize("sched", [dict(), dict(sort_by_length=1, persistent=1, graph=1),
+                                   dict(lanes_per_track=4), dict(store_by_plane=1)])
+def test_gpu_mixed_fused_fit_with_handed_back_tracks(name, cfg, n, sched):
+    """The same in the mixed mode: repeated calls and every schedule give the same
+    bits, and tracks that are not at the phi wrap are within twice the mode's
+    bars (1e-5, 1e-3) of the fit with track states."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from gpukalmanfitter_amd.fitter import DeviceBatch, KalmanFitter, KalmanFitterOptions
+    b = variant(name, n, cfg)
+    kf = KalmanFitter(b.planes, b.field)
+    opts = KalmanFitterOptions(precision="mixed", **W)
+    ref_dev = DeviceBatch(b, track_states=True)
+    kf.fit_batch(ref_dev, opts)
+    ref = ref_dev.results_numpy()
+    dev = DeviceBatch(b)
+    kf.fit_batch(dev, opts)
+    got = [dev.results_numpy()]
+    kf.set_schedule(**sched)
+    for _ in range(2):
+        dev.clear_results()
+        kf.fit_batch(dev, opts)
+        got.append(dev.results_numpy())
+    kf.close()
+    for k in ("ndf", "n_measured"):
+        assert np.array_equal(got[0][k], ref[k]), k
+    if sched.get("lanes_per_track", 1) == 1:
+        for k in ("params", "cov", "chi2", "ndf", "n_measured", "status"):
+            assert np.array_equal(got[0][k], got[1][k], equal_nan=True), k
+    for k in ("params", "cov", "chi2", "ndf", "n_measured", "status"):
+        assert np.array_equal(got[1][k], got[2][k], equal_nan=True), k
+    if name in ("no time variance", "phi wrap"):
+        return
+    assert np.array_equal(got[1]["status"], ref["status"])
+
+    class R:
+        pass
+    o = R()
+    o.status, o.params, o.cov, o.chi2 = (ref[k] for k in ("status", "params", "cov", "chi2"))
+    pd, cd, _ = compare_fit(got[1], o)
+    assert pd <= 2e-5 and cd <= 2e-3, (pd, cd)
