@@ -52,7 +52,8 @@ struct kf_ctx {
   uint64_t budget = KF_DEFAULT_MEMORY_BUDGET;  // per-batch working buffers
   hipEvent_t ev0 = nullptr, evm = nullptr, ev1 = nullptr;
   bool timed = false;
-  bool phase_timed = false;  // evm was recorded (not under graph replay)
+  bool phase_timed = false;  // the last call was not a graph replay or in slices
+  bool one_kernel = false;   // the last call was one kernel: evm not recorded
   // scheduling (kf_schedule) and its buffers: track order, sort counters,
   // work-queue counters
   kf_schedule sched{};
@@ -643,6 +644,7 @@ int kf_fit_noalloc(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt,
   KF_HIP(ctx, hipEventRecord(ctx->ev1, s));
   ctx->timed = true;
   ctx->phase_timed = slice >= a.n;
+  ctx->one_kernel = false;
   return KF_OK;
 }
 
@@ -723,7 +725,12 @@ int kf_fit(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt, const kf_res
     ctx->phase_timed = false;
   } else {
     KF_HIP(ctx, hipEventRecord(ctx->ev0, s));
-    e = launchSlices(a, L, opt->precision, res->track_states, slice, ctx->evm, s);
+    // a fit that is one kernel has no second phase to time
+    kfd::FitArgs whole = a;
+    sliceRange(whole, 0, slice);
+    ctx->one_kernel = fused && slice >= a.n && kfd::redoChunkPerWave(whole, std::max(L.lanes_per_track, 1));
+    e = launchSlices(a, L, opt->precision, res->track_states, slice,
+                     ctx->one_kernel ? nullptr : ctx->evm, s);
     ctx->phase_timed = slice >= a.n;
   }
   if (e != hipSuccess) {
@@ -906,6 +913,7 @@ int kf_chi2_gradient(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt, do
     if (e == hipSuccess) e = kfd_launch_adjoint(&a, &g, sums, first > 0, s);
   }
   ctx->phase_timed = slice >= a.n;
+  ctx->one_kernel = false;
   if (e == hipSuccess)
     e = kfd_launch_adjoint_finish(&a, sums, grad_planes, grad_field_scale, chi2_sum, s);
   if (e == hipSuccess && grad_raw)
@@ -963,6 +971,12 @@ int kf_last_phase_ms(const kf_ctx *ctx, double *forward_ms, double *backward_ms)
   if (!ctx->timed || !ctx->phase_timed) return KF_E_STATE;
   if (hipEventSynchronize(ctx->ev1) != hipSuccess) return KF_E_HIP;
   float f = 0.0f, b = 0.0f;
+  if (ctx->one_kernel) {
+    if (hipEventElapsedTime(&f, ctx->ev0, ctx->ev1) != hipSuccess) return KF_E_HIP;
+    *forward_ms = (double)f;
+    *backward_ms = 0.0;
+    return KF_OK;
+  }
   if (hipEventElapsedTime(&f, ctx->ev0, ctx->evm) != hipSuccess ||
       hipEventElapsedTime(&b, ctx->evm, ctx->ev1) != hipSuccess)
     return KF_E_HIP;

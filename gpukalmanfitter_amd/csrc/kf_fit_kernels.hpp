@@ -120,8 +120,9 @@ __global__ void __launch_bounds__(KF_BLOCK) kf_fit_kernel(FitArgs args) {
 //
 // A track that the fixed-point smoother leaves to the RTS program (TrackFit::
 // fxSafe; 1 in 200,000 of the material workload) is fitted again by its own
-// wave while the others go on, over a store chunk it takes from a pool; when
-// the pool is used up it goes to the list of the redo kernel.  Waiting for
+// wave while the others go on, over a store chunk it takes from a pool (or its
+// own, redoChunkPerWave); when the pool is used up it goes to the list of the
+// redo kernel.  Waiting for
 // the redo kernel with all of them cost the material workload 0.9 ms per
 // call for a single track: the latency of one wave's fit of 40 planes.
 //
@@ -175,6 +176,10 @@ __global__ void __launch_bounds__(KF_FUSED_BLOCK) kf_fused_kernel(FitArgs args) 
   }
   const uint64_t redoMask = __ballot(redo);
   if (redoMask == 0) return;
+  if (redoChunkPerWave(args, L)) {
+    if (redo) redoTrack<S>((const FitArgs *)__builtin_amdgcn_kernarg_segment_ptr(), i, t);
+    return;
+  }
   const int first = __ffsll((unsigned long long)redoMask) - 1;
   const int lane = (int)(threadIdx.x & 63u);
   uint32_t chunk = 0;
@@ -312,7 +317,7 @@ hipError_t launchFit(const FitArgs *args, hipStream_t stream, hipEvent_t between
     const hipError_t e = hipEventRecord(between, stream);
     if (e != hipSuccess) return e;
   }
-  if (args->smoothing)
+  if (args->smoothing && !redoChunkPerWave(*args, lpt))
     hipLaunchKernelGGL((kf_redo_kernel<S>), dim3((unsigned)(args->redo_lanes / 64)), dim3(64), 0,
                        stream, *args);
   return hipGetLastError();

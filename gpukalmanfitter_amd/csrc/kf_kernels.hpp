@@ -152,6 +152,14 @@ struct FitArgs {
 };
 #define KF_REDO_LIST 64
 
+// Whether every wave of a fused fit has a store chunk of its own for tracks it
+// hands to the RTS program (up to 256 waves, 16,384 tracks): no chunk is then
+// drawn from the pool, no list kept, and no redo kernel follows.  For small
+// batches that launch was 5 of 96 us.
+KFD_INLINE bool redoChunkPerWave(const FitArgs &a, int lanes_per_track) {
+  return (a.count * lanes_per_track + 63) / 64 * 64 <= a.redo_lanes;
+}
+
 }  // namespace kfd
 
 // Step-stack depth per track of the chi2 adjoint: a segment between two
@@ -198,7 +206,8 @@ struct KfdLaunch {
 // [work-queue reset] -> forward kernel -> record `between` (if not NULL) ->
 // smoother/back-propagation kernel (unless smoothing is off) -> track-state
 // export (if track_states_out is not NULL).  Without them: [work-queue
-// reset] -> fused kernel -> record `between` -> redo kernel.  `launch` may be NULL (one thread per
+// reset] -> fused kernel -> record `between` -> redo kernel (the last not where
+// redoChunkPerWave holds).  `launch` may be NULL (one thread per
 // track, identity order).  With a persistent grid, args->queue and
 // args->chunks_per_grab must be set; with sorting, args->order.
 extern "C" hipError_t kfd_launch_fit(const kfd::FitArgs *args, int precision, hipStream_t stream,

@@ -303,10 +303,10 @@ double kf_last_kernel_ms(const kf_ctx *ctx);
 /* The same split at the hand-over between the kernels of a fit: the
  * forward filter (up to the reference's finalize()) and the smoother plus
  * back-propagation to the perigee.  The backward time includes the
- * track-state export when track states were requested.  An FP64 fit without
+ * track-state export when track states were requested.  A fit without
  * track states runs as one kernel: its time is the forward time, and the
  * backward time is that of the pass over tracks it left for the RTS smoother
- * (none as a rule).  No reference
+ * (none as a rule, and 0 in a small batch).  No reference
  * counterpart (the reference times the whole batch from the host,
  * Run/GPU/KalmanFitterGPUTest.cu:382-513). */
 int kf_last_phase_ms(const kf_ctx *ctx, double *forward_ms, double *backward_ms);
