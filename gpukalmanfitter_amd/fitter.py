@@ -162,25 +162,36 @@ class KalmanFitterResult:
     fitted_states: np.ndarray = None  # [n_states, KF_TS_STRIDE]
 
 
+_TRIU = np.triu_indices(6)
+_SYM_OF = np.empty((6, 6), dtype=np.intp)
+for (_i, _j), _k in abi.SYM_INDEX.items():
+    _SYM_OF[_i, _j] = _k
+
+
 def unpack_sym(packed):
     """[21, ...] packed upper triangle -> [..., 6, 6]."""
     packed = np.asarray(packed)
-    out = np.empty(packed.shape[1:] + (6, 6), dtype=packed.dtype)
-    for (i, j), k in abi.SYM_INDEX.items():
-        out[..., i, j] = packed[k]
-    return out
+    return np.ascontiguousarray(np.moveaxis(packed[_SYM_OF], (0, 1), (-2, -1)))
 
 
 def pack_sym(m):
     """[..., 6, 6] -> [21, ...] upper triangle."""
-    m = np.asarray(m)
-    out = np.empty((21,) + m.shape[:-2], dtype=m.dtype)
-    k = 0
-    for i in range(6):
-        for j in range(i, 6):
-            out[k] = m[..., i, j]
-            k += 1
-    return out
+    return np.ascontiguousarray(np.moveaxis(np.asarray(m)[..., _TRIU[0], _TRIU[1]], -1, 0))
+
+
+# Arrays up to this size in total travel in one copy (the copy's 15 us are
+# latency); beyond it the extra pass over host memory would cost more.
+_ONE_COPY_BYTES = 1 << 20
+
+
+def _layout(fields):
+    """Offsets of (name, shape, dtype) fields in one buffer, each 256-byte aligned,
+    and the buffer's size."""
+    offsets, at = [], 0
+    for _, shape, dtype in fields:
+        offsets.append(at)
+        at += -(-math.prod(shape) * np.dtype(dtype).itemsize // 256) * 256
+    return offsets, at
 
 
 class DeviceBatch:
@@ -194,12 +205,23 @@ class DeviceBatch:
         self.device = torch.device(device)
         self.n_tracks = batch.n_tracks
         self.n_hits = batch.n_hits
-        self.t = {}
+        arrays = {}
         for name in self._INPUTS:
             arr = np.ascontiguousarray(getattr(batch, name))
             if arr.size == 0:
                 arr = np.zeros(1, dtype=arr.dtype)
-            self.t[name] = torch.from_numpy(arr).to(self.device)
+            arrays[name] = arr
+        fields = [(name, arr.shape, arr.dtype) for name, arr in arrays.items()]
+        offsets, size = _layout(fields)
+        if size <= _ONE_COPY_BYTES:
+            host = np.empty(size, dtype=np.uint8)
+            for (name, shape, dtype), at in zip(fields, offsets):
+                host[at:at + arrays[name].nbytes].view(dtype).reshape(shape)[...] = arrays[name]
+            dev = torch.from_numpy(host).to(self.device)
+            self.t = {name: self._view(dev, at, shape, torch.from_numpy(arrays[name]).dtype)
+                      for (name, shape, _), at in zip(fields, offsets)}
+        else:
+            self.t = {name: torch.from_numpy(arr).to(self.device) for name, arr in arrays.items()}
         self._outputs(track_states, max_states if max_states else max(batch.max_states, 1))
 
     @classmethod
@@ -214,22 +236,31 @@ class DeviceBatch:
         self._outputs(track_states, max(int(max_states), 1))
         return self
 
+    @staticmethod
+    def _view(buffer, at, shape, dtype):
+        """The tensor of this shape and type at byte `at` of a uint8 buffer."""
+        return buffer[at:at + math.prod(shape) * dtype.itemsize].view(dtype).view(shape)
+
     def _outputs(self, track_states, max_states):
         torch = _torch()
         n = max(self.n_tracks, 1)
-        f64 = dict(dtype=torch.float64, device=self.device)
-        self.out = {
-            "params": torch.zeros((6, n), **f64),
-            "cov": torch.zeros((21, n), **f64),
-            "chi2": torch.zeros(n, **f64),
-            "ndf": torch.zeros(n, dtype=torch.int32, device=self.device),
-            "n_measured": torch.zeros(n, dtype=torch.int32, device=self.device),
-            "status": torch.zeros(n, dtype=torch.int32, device=self.device),
-        }
         self.max_states = int(max_states)
+        f64, i32 = np.float64, np.int32
+        fields = [("params", (6, n), f64), ("cov", (21, n), f64), ("chi2", (n,), f64),
+                  ("ndf", (n,), i32), ("n_measured", (n,), i32), ("status", (n,), i32)]
         if track_states:
-            self.out["track_states"] = torch.zeros(
-                (self.max_states, abi.KF_TS_STRIDE, n), **f64)
+            fields.append(("track_states", (self.max_states, abi.KF_TS_STRIDE, n), f64))
+        types = {f64: torch.float64, i32: torch.int32}
+        offsets, size = _layout(fields)
+        self._out_layout = None
+        if size <= _ONE_COPY_BYTES:
+            buffer = torch.zeros(size, dtype=torch.uint8, device=self.device)
+            self.out = {name: self._view(buffer, at, shape, types[dtype])
+                        for (name, shape, dtype), at in zip(fields, offsets)}
+            self._out_layout = buffer, dict(self.out), fields, offsets
+        else:
+            self.out = {name: torch.zeros(shape, dtype=types[dtype], device=self.device)
+                        for name, shape, dtype in fields}
 
     def c_tracks(self):
         t = abi.kf_tracks()
@@ -252,7 +283,16 @@ class DeviceBatch:
 
     def results_numpy(self):
         """Copies the outputs to host numpy arrays (synchronising)."""
-        res = {k: v.cpu().numpy() for k, v in self.out.items()}
+        # one copy, while the outputs are the ones allocated together
+        if self._out_layout and self.out.keys() == self._out_layout[1].keys() and all(
+                self.out[k] is v for k, v in self._out_layout[1].items()):
+            buffer, _, fields, offsets = self._out_layout
+            host = buffer.cpu().numpy()
+            res = {name: host[at:at + math.prod(shape) * np.dtype(dtype).itemsize]
+                   .view(dtype).reshape(shape)
+                   for (name, shape, dtype), at in zip(fields, offsets)}
+        else:
+            res = {k: v.cpu().numpy() for k, v in self.out.items()}
         res["status"] = res["status"].view(np.uint32)
         return res
 
