@@ -400,6 +400,20 @@ size_t firstBytes(int precision) {
 }
 size_t fusedBytesPerTrack(int precision) { return firstBytes(precision) + sizeof(uint32_t); }
 
+// Whether a fused fit in input order is sorted by length of itself.  A wave takes
+// as long as its longest track, so where the tracks fill fewer than 4/5 of the
+// states they may have (the caller's max_states; a batch whose longest track is
+// not stated is left alone) and the waves exceed one per SIMD, lengths sorted
+// into waves shorten the launch by more than the sort and the scattered reads
+// cost: filled to 0.55-0.60, 66,000 tracks 745 -> 450 us (FP64, 5-30 planes) and
+// 1,334 -> 831 us (mixed, 8-40 planes with material), 500,003 tracks 2,719 ->
+// 2,036 us; with equal lengths 100,000 tracks would go from 188 to 208 us.  Up to
+// one wave per SIMD the longest track decides, sorted or not.
+bool sortPays(const kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt, int lanes_per_track) {
+  return opt->max_states > 0 && tr->n_tracks * lanes_per_track > (int64_t)256 * ctx->n_cu &&
+         (double)tr->n_hits < 0.8 * (double)tr->n_tracks * (double)opt->max_states;
+}
+
 // Positions per slice: the largest multiple of 64 whose working set fits the
 // budget (at least 64), or the whole batch.
 int64_t sliceTracks(const kf_ctx *ctx, int64_t n, size_t bytes_per_track) {
@@ -667,15 +681,16 @@ int kf_fit(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt, const kf_res
   KfdLaunch L{};
   L.lanes_per_track = sc.lanes_per_track;
   L.store_by_plane = sc.store_by_plane;
-  if (sc.sort_by_length || sc.persistent) {
+  const bool sort = sc.sort_by_length || (fused && sortPays(ctx, tr, opt, sc.lanes_per_track));
+  if (sort || sc.persistent) {
     const size_t order_bytes = ((size_t)a.n * sizeof(int32_t) + 255) / 256 * 256;
     rc = grow(ctx, &ctx->sched_buf, &ctx->sched_bytes, order_bytes + 514 * sizeof(uint32_t), s,
               "schedule buffers");
     if (rc != KF_OK) return rc;
     L.order = (int32_t *)ctx->sched_buf;
     L.sort_scratch = (uint32_t *)((char *)ctx->sched_buf + order_bytes);
-    L.sort_by_length = sc.sort_by_length;
-    a.order = sc.sort_by_length ? L.order : nullptr;
+    L.sort_by_length = sort;
+    a.order = sort ? L.order : nullptr;
     a.queue = L.sort_scratch + 512;
     if (sc.persistent) {
       const int waves = sc.waves_per_cu * ctx->n_cu;

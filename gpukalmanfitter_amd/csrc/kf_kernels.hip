@@ -40,8 +40,11 @@ __global__ void __launch_bounds__(256) kf_export_states(FitArgs args, double *ou
 // Counting sort of the tracks by decreasing sequence length (lengths >= 255
 // share the top bin): tracks of one wave then take similar numbers of steps,
 // and a persistent grid starts on the longest.  Per-block LDS histograms keep
-// the global atomics to one per block and bin.
+// the global atomics to one per block and bin; a thread takes kSortTracks tracks,
+// so that the blocks' atomics on the few bins in use do not queue up.
 constexpr int kLenBins = 256;
+constexpr int kSortTracks = 4;
+constexpr int kSortBlock = 256 * kSortTracks;
 
 KFD_INLINE int lengthBin(const FitArgs &a, int64_t i) {
   int l = a.seq_count[i];
@@ -68,8 +71,10 @@ __global__ void __launch_bounds__(256) kf_len_hist(FitArgs a, uint32_t *hist) {
   __shared__ uint32_t h[kLenBins];
   h[threadIdx.x] = 0u;
   __syncthreads();
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < a.n) atomicAdd(&h[lengthBin(a, i)], 1u);
+  const int64_t i0 = (int64_t)blockIdx.x * kSortBlock + threadIdx.x;
+#pragma unroll
+  for (int q = 0; q < kSortTracks; ++q)
+    if (i0 + 256 * q < a.n) atomicAdd(&h[lengthBin(a, i0 + 256 * q)], 1u);
   __syncthreads();
   if (h[threadIdx.x]) atomicAdd(&hist[threadIdx.x], h[threadIdx.x]);
 }
@@ -93,14 +98,21 @@ __global__ void __launch_bounds__(256) kf_len_scatter(FitArgs a, uint32_t *off, 
   __shared__ uint32_t cnt[kLenBins], base[kLenBins];
   cnt[threadIdx.x] = 0u;
   __syncthreads();
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int bin = (i < a.n) ? lengthBin(a, i) : 0;
-  uint32_t local = 0;
-  if (i < a.n) local = atomicAdd(&cnt[bin], 1u);
+  const int64_t i0 = (int64_t)blockIdx.x * kSortBlock + threadIdx.x;
+  int bin[kSortTracks];
+  uint32_t local[kSortTracks];
+#pragma unroll
+  for (int q = 0; q < kSortTracks; ++q) {
+    const int64_t i = i0 + 256 * q;
+    bin[q] = (i < a.n) ? lengthBin(a, i) : 0;
+    local[q] = (i < a.n) ? atomicAdd(&cnt[bin[q]], 1u) : 0u;
+  }
   __syncthreads();
   if (cnt[threadIdx.x]) base[threadIdx.x] = atomicAdd(&off[threadIdx.x], cnt[threadIdx.x]);
   __syncthreads();
-  if (i < a.n) order[base[bin] + local] = (int32_t)i;
+#pragma unroll
+  for (int q = 0; q < kSortTracks; ++q)
+    if (i0 + 256 * q < a.n) order[base[bin[q]] + local[q]] = (int32_t)(i0 + 256 * q);
 }
 
 }  // namespace kfd
@@ -109,7 +121,8 @@ extern "C" hipError_t kfd_launch_fit(const kfd::FitArgs *args, int precision, hi
                                      double *track_states_out, hipEvent_t between,
                                      const KfdLaunch *launch) {
   if (args->count <= 0) return hipSuccess;
-  if (launch && launch->persistent_blocks > 0)
+  // the fused kernel takes one position per lane whatever the schedule
+  if (launch && launch->persistent_blocks > 0 && args->tsf)
     hipLaunchKernelGGL(kfd::kf_queue_reset, dim3(1), dim3(64), 0, stream, args->queue);
   const hipError_t e = (precision == KF_PRECISION_FP64)
                            ? kfd_launch_fit_fp64(args, stream, between, launch)
@@ -132,7 +145,7 @@ extern "C" hipError_t kfd_launch_redo_reset(uint32_t *redo, hipStream_t stream) 
 extern "C" hipError_t kfd_launch_sort(const kfd::FitArgs *args, const KfdLaunch *launch,
                                       hipStream_t stream) {
   if (args->n <= 0) return hipSuccess;
-  const unsigned sb = (unsigned)((args->n + 255) / 256);
+  const unsigned sb = (unsigned)((args->n + kfd::kSortBlock - 1) / kfd::kSortBlock);
   uint32_t *hist = launch->sort_scratch, *off = launch->sort_scratch + kfd::kLenBins;
   hipLaunchKernelGGL(kfd::kf_sort_reset, dim3(1), dim3(256), 0, stream, launch->sort_scratch);
   hipLaunchKernelGGL(kfd::kf_len_hist, dim3(sb), dim3(256), 0, stream, *args, hist);

@@ -174,7 +174,10 @@ typedef struct kf_results {
  * launches one thread per track on a fixed grid, Run/GPU/Kernels.cu:6-55). */
 typedef struct kf_schedule {
   int32_t sort_by_length;  /* fit tracks in order of decreasing sequence length, so a
-                              wave's tracks take similar numbers of steps (default 0) */
+                              wave's tracks take similar numbers of steps (default 0: a
+                              fit without track states does so of itself where
+                              options.max_states and n_hits show unequal lengths and
+                              the batch exceeds one wave per SIMD; same bits) */
   int32_t persistent;      /* 1: resident waves pull 64-track chunks from a work queue */
   int32_t waves_per_cu;    /* persistent grid size, waves per compute unit (default 4) */
   int32_t chunks_per_grab; /* work-queue granularity, 64-track chunks per grab (default 1) */
