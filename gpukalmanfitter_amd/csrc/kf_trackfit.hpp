@@ -1665,7 +1665,7 @@ struct TrackFit {
   // covariance; each (i, j) pair is formed once, so the result is symmetric
   // by construction.  The 2x2 inversion and the update are double in both.
   KFD_INLINE bool filter(int sp) {
-    const DevPlane &pl = plane(sp);
+    const DevPlane pl = plane(sp);
     // the track's hit on this plane: first match in hit order (SurfaceFinder,
     // KalmanFitter.hpp:31-38); the loaded-ahead next hit, else a scan with
     // four independent geo-id loads per round trip
