@@ -79,6 +79,12 @@ KFD_INLINE constexpr int cidx(int r, int c) {
   return (r <= c) ? (r * 5 - (r * (r - 1)) / 2 + (c - r)) : (c * 5 - (c * (c - 1)) / 2 + (r - c));
 }
 
+// Quotients: the sweep's divisors are well scaled, so they are recipD / rootD
+// (Newton on the hardware's estimate, 5-11 instructions, within an ulp) and
+// products with 1/3 and 1/6; 105 library quotients were a tenth of its code and
+// most of them in the loop over a step's columns.
+constexpr double kThird = 1.0 / 3.0, kSixth = 1.0 / 6.0;
+
 // a x b
 KFD_INLINE void crs(const double a[3], const double b[3], double r[3]) {
   r[0] = a[1] * b[2] - a[2] * b[1];
@@ -96,11 +102,12 @@ KFD_INLINE void crsVJP(const double a[3], const double b[3], const double cb[3],
 #pragma unroll
   for (int k = 0; k < 3; ++k) bb[k] += t[k];
 }
-// B = s F(x): sb += Bb . F(x) = Bb . B / s; xb += (dB/dx)^T Bb on a grid.
+// B = s F(x): sb += Bb . B (= s Bb . F(x); the sweep divides the sum by s at its
+// end); xb += (dB/dx)^T Bb on a grid.
 template <int FK>
 KFD_INLINE void fieldVJP(const DevField &fld, const double x[3], const double B[3],
                          const double Bb[3], double xb[3], double &sb) {
-  sb += (Bb[0] * B[0] + Bb[1] * B[1] + Bb[2] * B[2]) / fld.scale;
+  sb += Bb[0] * B[0] + Bb[1] * B[1] + Bb[2] * B[2];
   if constexpr (FK == kFieldConst) return;
   if (fld.grid) {
     double Bg[3], dB[3][3];
@@ -113,9 +120,9 @@ KFD_INLINE void fieldVJP(const DevField &fld, const double x[3], const double B[
 // Grid field: the backward of a lookup whose gradient the forward recompute
 // stored (dB[k][a] of stage point `pt` at dBs[(9 pt + 3 k + a) * KF_BLOCK],
 // float), instead of reading the corners again.
-KFD_INLINE void fieldVJPStored(const DevField &fld, const float *dBs, int pt, const double B[3],
+KFD_INLINE void fieldVJPStored(const float *dBs, int pt, const double B[3],
                                const double Bb[3], double xb[3], double &sb) {
-  sb += (Bb[0] * B[0] + Bb[1] * B[1] + Bb[2] * B[2]) / fld.scale;
+  sb += Bb[0] * B[0] + Bb[1] * B[1] + Bb[2] * B[2];
 #pragma unroll
   for (int a = 0; a < 3; ++a)
     xb[a] += Bb[0] * (double)dBs[(9 * pt + a) * KF_BLOCK] +
@@ -132,7 +139,7 @@ struct StepFwd {
   double t2[3], t3[3], t4[3];
   double p1[3], p2[3];
   double L1[3], L2[3], L3[3], L4[3];
-  double du[3], dun;
+  double du[3], idun;
 
   // dBs: for a grid field, the field gradient at the three stage points is
   // stored there (one lookup gives the value and the gradient); nullptr: the
@@ -184,8 +191,9 @@ struct StepFwd {
 #pragma unroll
     for (int k = 0; k < 3; ++k) k4[k] *= qop;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) du[k] = d[k] + (h / 6.0) * (k1[k] + 2.0 * (k2[k] + k3[k]) + k4[k]);
-    dun = sqrt(du[0] * du[0] + du[1] * du[1] + du[2] * du[2]);
+    for (int k = 0; k < 3; ++k) du[k] = d[k] + (h * kSixth) * (k1[k] + 2.0 * (k2[k] + k3[k]) + k4[k]);
+    double dun;
+    rootD(du[0] * du[0] + du[1] * du[1] + du[2] * du[2], dun, idun);
     // q/p column of the transport (EigenStepper.ipp:50-124): the dk/dlambda
     // vectors
     double c[3];
@@ -241,9 +249,9 @@ KFD_INLINE void dirColumnVJP(const StepFwd<FK> &F, double h, double qop, const d
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     gb[k] += h * aF[k] + aG[k];
-    hb += aF[k] * (g[k] + (h / 3.0) * (v1[k] + v2[k] + v3[k])) +
-          aG[k] * (v1[k] + 2.0 * (v2[k] + v3[k]) + v4[k]) / 6.0;
-    const double a = (h * h / 6.0) * aF[k], b = (h / 6.0) * aG[k];
+    hb += aF[k] * (g[k] + (h * kThird) * (v1[k] + v2[k] + v3[k])) +
+          aG[k] * kSixth * (v1[k] + 2.0 * (v2[k] + v3[k]) + v4[k]);
+    const double a = (h * h * kSixth) * aF[k], b = (h * kSixth) * aG[k];
     v1b[k] = a + b;
     v2b[k] = a + 2.0 * b;
     v3b[k] = a + 2.0 * b;
@@ -352,9 +360,9 @@ KFD_INLINE void stepVJP(const DevField &fld, const StepFwd<FK> &F, const double 
   double L1b[3], L2b[3], L3b[3], L4b[3];
 #pragma unroll
   for (int r = 0; r < 3; ++r) {
-    hb += dFdLb[r] * (h / 3.0) * (F.L1[r] + F.L2[r] + F.L3[r]) +
-          dGdLb[r] * (F.L1[r] + 2.0 * (F.L2[r] + F.L3[r]) + F.L4[r]) / 6.0;
-    const double a = (h * h / 6.0) * dFdLb[r], g = (h / 6.0) * dGdLb[r];
+    hb += dFdLb[r] * (h * kThird) * (F.L1[r] + F.L2[r] + F.L3[r]) +
+          dGdLb[r] * kSixth * (F.L1[r] + 2.0 * (F.L2[r] + F.L3[r]) + F.L4[r]);
+    const double a = (h * h * kSixth) * dFdLb[r], g = (h * kSixth) * dGdLb[r];
     L1b[r] = a + g;
     L2b[r] = a + 2.0 * g;
     L3b[r] = a + 2.0 * g;
@@ -390,25 +398,25 @@ KFD_INLINE void stepVJP(const DevField &fld, const StepFwd<FK> &F, const double 
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     dInb[k] += h * pb[k];
-    hb += pb[k] * (d[k] + (h / 3.0) * (F.k1[k] + F.k2[k] + F.k3[k]));
-    k1b[k] += (h * h / 6.0) * pb[k];
-    k2b[k] += (h * h / 6.0) * pb[k];
-    k3b[k] += (h * h / 6.0) * pb[k];
+    hb += pb[k] * (d[k] + (h * kThird) * (F.k1[k] + F.k2[k] + F.k3[k]));
+    k1b[k] += (h * h * kSixth) * pb[k];
+    k2b[k] += (h * h * kSixth) * pb[k];
+    k3b[k] += (h * h * kSixth) * pb[k];
   }
   {
-    double dn[3] = {F.du[0] / F.dun, F.du[1] / F.dun, F.du[2] / F.dun};
+    double dn[3] = {F.du[0] * F.idun, F.du[1] * F.idun, F.du[2] * F.idun};
     const double pr = dn[0] * db[0] + dn[1] * db[1] + dn[2] * db[2];
     double dub[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) dub[k] = (db[k] - dn[k] * pr) / F.dun;
+    for (int k = 0; k < 3; ++k) dub[k] = (db[k] - dn[k] * pr) * F.idun;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       dInb[k] += dub[k];
-      hb += dub[k] * (F.k1[k] + 2.0 * (F.k2[k] + F.k3[k]) + F.k4[k]) / 6.0;
-      k1b[k] += (h / 6.0) * dub[k];
-      k2b[k] += (h / 3.0) * dub[k];
-      k3b[k] += (h / 3.0) * dub[k];
-      k4b[k] += (h / 6.0) * dub[k];
+      hb += dub[k] * kSixth * (F.k1[k] + 2.0 * (F.k2[k] + F.k3[k]) + F.k4[k]);
+      k1b[k] += (h * kSixth) * dub[k];
+      k2b[k] += (h * kThird) * dub[k];
+      k3b[k] += (h * kThird) * dub[k];
+      k4b[k] += (h * kSixth) * dub[k];
     }
   }
   // ---- stages, last to first
@@ -429,7 +437,7 @@ KFD_INLINE void stepVJP(const DevField &fld, const StepFwd<FK> &F, const double 
   // Bl = s F(p2)
   double p2b[3] = {0, 0, 0};
   if (FK != kFieldConst && dBs && fld.grid)
-    fieldVJPStored(fld, dBs, 2, F.Bl, Blb, p2b, sb);
+    fieldVJPStored(dBs, 2, F.Bl, Blb, p2b, sb);
   else
     fieldVJP<FK>(fld, F.p2, F.Bl, Blb, p2b, sb);
   // p2 = pos + h d + h^2/2 k3
@@ -469,7 +477,7 @@ KFD_INLINE void stepVJP(const DevField &fld, const StepFwd<FK> &F, const double 
   // Bm = s F(p1)
   double p1b[3] = {0, 0, 0};
   if (FK != kFieldConst && dBs && fld.grid)
-    fieldVJPStored(fld, dBs, 1, F.Bm, Bmb, p1b, sb);
+    fieldVJPStored(dBs, 1, F.Bm, Bmb, p1b, sb);
   else
     fieldVJP<FK>(fld, F.p1, F.Bm, Bmb, p1b, sb);
   // p1 = pos + hh d + h^2/8 k1
@@ -488,7 +496,7 @@ KFD_INLINE void stepVJP(const DevField &fld, const StepFwd<FK> &F, const double 
   crsVJP(d, F.B1, w, dInb, B1b);
   // B1 = s F(pos)
   if (FK != kFieldConst && dBs && fld.grid)
-    fieldVJPStored(fld, dBs, 0, F.B1, B1b, posInb, sb);
+    fieldVJPStored(dBs, 0, F.B1, B1b, posInb, sb);
   else
     fieldVJP<FK>(fld, pos, F.B1, B1b, posInb, sb);
 #pragma unroll
@@ -528,8 +536,9 @@ struct PlaneFwd {
       nr[k] = pl.r[3 * k + 2];
       cc[k] = pl.c[k];
     }
-    rho = sqrt(d[0] * d[0] + d[1] * d[1]);
-    const double cosT = d[2], sinT = rho, invSinT = 1.0 / rho;
+    double invSinT;
+    rootD(d[0] * d[0] + d[1] * d[1], rho, invSinT);
+    const double cosT = d[2], sinT = rho;
     const double cosP = d[0] * invSinT, sinP = d[1] * invSinT;
     l20 = -sinP * invSinT;
     l21 = cosP * invSinT;
@@ -537,7 +546,7 @@ struct PlaneFwd {
     l31 = sinP * cosT;
     l32 = -sinT;
     dp = nr[0] * d[0] + nr[1] * d[1] + nr[2] * d[2];
-    const double idp = 1.0 / dp;
+    const double idp = recipD(dp);
 #pragma unroll
     for (int k = 0; k < 3; ++k) nv[k] = nr[k] * idp;
 #pragma unroll
@@ -588,7 +597,7 @@ struct PlaneFwd {
     V11 = v11;
     const double S00 = Cp[0][0] + V00, S01 = Cp[0][1] + V01, S11 = Cp[1][1] + V11;
     const double det = S00 * S11 - S01 * S01;
-    const double idet = 1.0 / det;
+    const double idet = recipD(det);
     Si00 = S11 * idet;
     Si01 = -S01 * idet;
     Si11 = S00 * idet;
@@ -766,28 +775,29 @@ struct PlaneFwd {
         Ab[q][c] += svb[c] * nv[q];
       }
     double nrb[3];
-    const double dpb = -(nvb[0] * nr[0] + nvb[1] * nr[1] + nvb[2] * nr[2]) / (dp * dp);
+    const double idp = recipD(dp);
+    const double dpb = -(nvb[0] * nr[0] + nvb[1] * nr[1] + nvb[2] * nr[2]) * (idp * idp);
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-      nrb[q] = nvb[q] / dp + dpb * d[q];
+      nrb[q] = nvb[q] * idp + dpb * d[q];
       db[q] += dpb * nr[q];
     }
     // l's as functions of d (rho^2 = d0^2 + d1^2)
     {
-      const double r2 = rho * rho, r3 = r2 * rho, r4 = r2 * r2;
+      const double ir = recipD(rho), ir2 = ir * ir, ir3 = ir2 * ir, ir4 = ir2 * ir2;
       const double d0 = d[0], d1 = d[1], d2 = d[2];
-      db[0] += l20b * (2.0 * d1 * d0 / r4) + l21b * (1.0 / r2 - 2.0 * d0 * d0 / r4) +
-               l30b * (d2 / rho - d0 * d0 * d2 / r3) + l31b * (-d0 * d1 * d2 / r3) +
-               l32b * (-d0 / rho);
-      db[1] += l20b * (-1.0 / r2 + 2.0 * d1 * d1 / r4) + l21b * (-2.0 * d0 * d1 / r4) +
-               l30b * (-d0 * d1 * d2 / r3) + l31b * (d2 / rho - d1 * d1 * d2 / r3) +
-               l32b * (-d1 / rho);
-      db[2] += l30b * (d0 / rho) + l31b * (d1 / rho);
+      db[0] += l20b * (2.0 * d1 * d0 * ir4) + l21b * (ir2 - 2.0 * d0 * d0 * ir4) +
+               l30b * (d2 * ir - d0 * d0 * d2 * ir3) + l31b * (-d0 * d1 * d2 * ir3) +
+               l32b * (-d0 * ir);
+      db[1] += l20b * (-ir2 + 2.0 * d1 * d1 * ir4) + l21b * (-2.0 * d0 * d1 * ir4) +
+               l30b * (-d0 * d1 * d2 * ir3) + l31b * (d2 * ir - d1 * d1 * d2 * ir3) +
+               l32b * (-d1 * ir);
+      db[2] += l30b * (d0 * ir) + l31b * (d1 * ir);
       // parameters: phi = atan2(d1, d0), theta = atan2(rho, d2)
-      const double rr = r2 + d2 * d2;
-      db[0] += xpb[2] * (-d1 / r2) + xpb[3] * (d2 / rr) * (d0 / rho);
-      db[1] += xpb[2] * (d0 / r2) + xpb[3] * (d2 / rr) * (d1 / rho);
-      db[2] += xpb[3] * (-rho / rr);
+      const double irr = recipD(rho * rho + d2 * d2);
+      db[0] += xpb[2] * (-d1 * ir2) + xpb[3] * (d2 * irr) * (d0 * ir);
+      db[1] += xpb[2] * (d0 * ir2) + xpb[3] * (d2 * irr) * (d1 * ir);
+      db[2] += xpb[3] * (-rho * irr);
     }
     // loc = (u0, u1) . (pos - c)
 #pragma unroll
@@ -827,7 +837,7 @@ KFD_INLINE void freeFromBoundVJP(const PlaneFwd &P, const double posb[3], const 
   xfb[2] += db[0] * (-sp * st) + db[1] * (cp * st);
   xfb[3] += db[0] * (cp * ct) + db[1] * (sp * ct) + db[2] * (-st);
   const double x4 = P.xf[4];
-  xfb[4] += pBar * (-((x4 < 0.0) ? -1.0 : 1.0) / (x4 * x4));
+  xfb[4] += pBar * (-((x4 < 0.0) ? -1.0 : 1.0) * recipD(x4 * x4));
 }
 
 // Backward of the Jacobian re-initialisation on a plane (PlaneSurface.ipp:
@@ -841,13 +851,15 @@ KFD_INLINE void jacInitVJP(const double d[3], const double Ab[3][5], const doubl
     Rb[k][0] += Ab[k][0];
     Rb[k][1] += Ab[k][1];
   }
-  const double rho = sqrt(d[0] * d[0] + d[1] * d[1]), r3 = rho * rho * rho;
+  double rho, ir;
+  rootD(d[0] * d[0] + d[1] * d[1], rho, ir);
+  const double ir3 = ir * ir * ir;
   const double d0 = d[0], d1 = d[1], d2 = d[2];
-  db[0] += Gb[0][1] * (d2 / rho - d2 * d0 * d0 / r3) + Gb[1][0] +
-           Gb[1][1] * (-d2 * d1 * d0 / r3) + Gb[2][1] * (-d0 / rho);
-  db[1] += -Gb[0][0] + Gb[0][1] * (-d2 * d0 * d1 / r3) +
-           Gb[1][1] * (d2 / rho - d2 * d1 * d1 / r3) + Gb[2][1] * (-d1 / rho);
-  db[2] += Gb[0][1] * (d0 / rho) + Gb[1][1] * (d1 / rho);
+  db[0] += Gb[0][1] * (d2 * ir - d2 * d0 * d0 * ir3) + Gb[1][0] +
+           Gb[1][1] * (-d2 * d1 * d0 * ir3) + Gb[2][1] * (-d0 * ir);
+  db[1] += -Gb[0][0] + Gb[0][1] * (-d2 * d0 * d1 * ir3) +
+           Gb[1][1] * (d2 * ir - d2 * d1 * d1 * ir3) + Gb[2][1] * (-d1 * ir);
+  db[2] += Gb[0][1] * (d0 * ir) + Gb[1][1] * (d1 * ir);
 }
 
 // ---------------------------------------------------------------------------
@@ -857,9 +869,9 @@ KFD_INLINE void jacInitVJP(const double d[3], const double Ab[3][5], const doubl
 // added to cov(2,2), cov(3,3), cov(4,4).
 struct MaterialFwd {
   bool on;
-  double p, m, sgn, c, pcor, q2b2, dq2b2, eps, depsP, depsC, running, drunP, Eloss;
-  double E0, nextE, pOut;
-  double tt, theta0, rho, dn, sigPhi, vPhi, vTheta, sq, vQop;
+  double p, m, ip, sgn, pcor, q2b2, sq2b2, isq2b2, dq2b2, eps, depsP, depsC, running, drunP, Eloss;
+  double iE0, nextE, pOut, ipOut;
+  double tt, itt, theta0, irho, dn, idn, sigPhi, vPhi, vTheta, sq, vQop;
   bool ms, el, dens;
 
   KFD_INLINE void run(const FitArgs &a, const DevPlane &pl, double pIn, const double d[3]) {
@@ -874,11 +886,13 @@ struct MaterialFwd {
     const double nr[3] = {pl.r[2], pl.r[5], pl.r[8]};
     const double nd = nr[0] * d[0] + nr[1] * d[1] + nr[2] * d[2];
     sgn = (nd < 0.0) ? -1.0 : 1.0;
-    c = fabs(nd);
-    pcor = 1.0 / c;
+    pcor = recipD(fabs(nd));
     const double thick = pl.thickness * pcor, xOverX0 = pl.thicknessInX0 * pcor;
-    q2b2 = 1.0 + (m / p) * (m / p);
-    dq2b2 = -2.0 * m * m / (p * p * p);
+    ip = recipD(p);
+    const double mp = m * ip;
+    q2b2 = 1.0 + mp * mp;
+    rootD(q2b2, sq2b2, isq2b2);
+    dq2b2 = -2.0 * mp * mp * ip;
     const double K = 0.5 * a.kK * pl.molarElectronDensity;
     eps = K * thick * q2b2;
     depsP = K * thick * dq2b2;
@@ -887,35 +901,41 @@ struct MaterialFwd {
     drunP = 0.0;
     Eloss = 0.0;
     if (el) {
-      const double I = pl.meanExcitation, me = a.kMe, bg = p / m, gamma = sqrt(1.0 + bg * bg);
-      const double mfrac = me / m, den = 1.0 + 2.0 * gamma * mfrac + mfrac * mfrac;
-      const double u = 2.0 * me * bg * bg, wmax = u / den;
-      const double beta2 = 1.0 / (1.0 + (m / p) * (m / p));
+      const double im = recipD(m), iI = recipD(pl.meanExcitation), me = a.kMe, bg = p * im;
+      double gamma, igamma;
+      rootD(1.0 + bg * bg, gamma, igamma);
+      const double mfrac = me * im, iden = recipD(1.0 + 2.0 * gamma * mfrac + mfrac * mfrac);
+      const double u = 2.0 * me * bg * bg, wmax = u * iden;
+      const double beta2 = isq2b2 * isq2b2;
       dens = !(bg < 10.0);
       const double dhalf =
-          dens ? oolLog(bg) + oolLog(a.kPlasma * sqrt(pl.molarElectronDensity) / I) - 0.5 : 0.0;
-      running = 0.5 * oolLog(u / I) + 0.5 * oolLog(wmax / I) - beta2 - dhalf;
-      const double dgamma = bg / (gamma * m);
-      const double dbeta2 = 2.0 * p * m * m / ((p * p + m * m) * (p * p + m * m));
-      drunP = 1.0 / p + 0.5 * (2.0 / p - 2.0 * mfrac * dgamma / den) - dbeta2 - (dens ? 1.0 / p : 0.0);
+          dens ? oolLog(bg) + oolLog(a.kPlasma * sqrt(pl.molarElectronDensity) * iI) - 0.5 : 0.0;
+      running = 0.5 * oolLog(u * iI) + 0.5 * oolLog(wmax * iI) - beta2 - dhalf;
+      const double dgamma = bg * igamma * im;
+      // d(beta^2)/dp = 2 p m^2 / (p^2 + m^2)^2 = 2 (m/p)^2 beta^4 / p
+      const double dbeta2 = 2.0 * mp * mp * (beta2 * beta2) * ip;
+      drunP = ip + (ip - mfrac * dgamma * iden) - dbeta2 - (dens ? ip : 0.0);
       Eloss = eps * running;
     }
     if (ms) {
-      tt = sqrt(xOverX0 * q2b2);
-      theta0 = a.kHighland * (1.0 / p) * tt * (1.0 + a.kHighlandLog * oolLog(tt));
-      rho = sqrt(d[0] * d[0] + d[1] * d[1]);
-      dn = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
-      sigPhi = theta0 * (dn / rho);
+      rootD(xOverX0 * q2b2, tt, itt);
+      theta0 = a.kHighland * ip * tt * (1.0 + a.kHighlandLog * oolLog(tt));
+      double rho;
+      rootD(d[0] * d[0] + d[1] * d[1], rho, irho);
+      rootD(d[0] * d[0] + d[1] * d[1] + d[2] * d[2], dn, idn);
+      sigPhi = theta0 * (dn * irho);
       vPhi = sigPhi * sigPhi;
       vTheta = theta0 * theta0;
     }
     if (el) {
-      sq = sqrt(q2b2) * (1.0 / (p * p)) * (4.0 * eps / a.kLandauConv);
+      sq = sq2b2 * (ip * ip) * (4.0 * eps * recipD(a.kLandauConv));
       vQop = sq * sq;
     }
-    E0 = sqrt(m * m + p * p);
+    double E0;
+    rootD(m * m + p * p, E0, iE0);
     nextE = E0 - Eloss;
-    pOut = (m < nextE) ? sqrt(nextE * nextE - m * m) : 0.0;
+    pOut = ipOut = 0.0;
+    if (m < nextE) rootD(nextE * nextE - m * m, pOut, ipOut);
   }
 
   // In: pOutb, the adjoints of the three variances.  Out: the adjoint of the
@@ -928,17 +948,17 @@ struct MaterialFwd {
     // p' = sqrt(nextE^2 - m^2), nextE = E0 - Eloss
     double Elossb = 0.0;
     if (m < nextE && pOut > 0.0) {
-      const double nEb = pOutb * nextE / pOut;
-      pb += nEb * p / E0;
+      const double nEb = pOutb * nextE * ipOut;
+      pb += nEb * p * iE0;
       Elossb = -nEb;
     }
     double epsb = 0.0;
     if (el) {
       // vQop = sq^2, sq = sqrt(q2b2) p^-2 (4 eps / conv)
       const double sqb = 2.0 * sq * vQopb;
-      const double s2 = sqrt(q2b2), f = 4.0 / a.kLandauConv;
-      pb += sqb * (s2 * (-2.0 / (p * p * p)) * f * eps + (dq2b2 / (2.0 * s2)) * (1.0 / (p * p)) * f * eps);
-      epsb += sqb * s2 * (1.0 / (p * p)) * f;
+      const double f = 4.0 * recipD(a.kLandauConv), ip2 = ip * ip;
+      pb += sqb * (sq2b2 * (-2.0 * ip2 * ip) * f * eps + (0.5 * dq2b2 * isq2b2) * ip2 * f * eps);
+      epsb += sqb * sq2b2 * ip2 * f;
       // Eloss = eps running(p)
       epsb += Elossb * running;
       pb += Elossb * eps * drunP;
@@ -946,25 +966,25 @@ struct MaterialFwd {
     if (ms) {
       // vPhi = (theta0 dn / rho)^2, vTheta = theta0^2
       const double sigb = 2.0 * sigPhi * vPhib;
-      double theta0b = 2.0 * theta0 * vThetab + sigb * (dn / rho);
+      double theta0b = 2.0 * theta0 * vThetab + sigb * (dn * irho);
       const double rb = sigb * theta0;  // adjoint of dn / rho
-      const double r3 = rho * rho * rho;
-      db[0] += rb * (d[0] / (dn * rho) - dn * d[0] / r3);
-      db[1] += rb * (d[1] / (dn * rho) - dn * d[1] / r3);
-      db[2] += rb * (d[2] / (dn * rho));
+      const double ir3 = irho * irho * irho;
+      db[0] += rb * (d[0] * (idn * irho) - dn * d[0] * ir3);
+      db[1] += rb * (d[1] * (idn * irho) - dn * d[1] * ir3);
+      db[2] += rb * (d[2] * (idn * irho));
       // theta0 = kH tt (1 + kHL log tt) / p, tt = sqrt(xOverX0 q2b2)
-      const double dth_dtt = a.kHighland / p * (1.0 + a.kHighlandLog * oolLog(tt) + a.kHighlandLog);
+      const double dth_dtt = a.kHighland * ip * (1.0 + a.kHighlandLog * oolLog(tt) + a.kHighlandLog);
       const double ttb = theta0b * dth_dtt;
-      pb += theta0b * (-theta0 / p);
+      pb += theta0b * (-theta0 * ip);
       const double xOverX0 = pl.thicknessInX0 * pcor;
-      pb += ttb * (xOverX0 / (2.0 * tt)) * dq2b2;
-      pcorb += ttb * (q2b2 / (2.0 * tt)) * pl.thicknessInX0;
+      pb += ttb * (0.5 * xOverX0 * itt) * dq2b2;
+      pcorb += ttb * (0.5 * q2b2 * itt) * pl.thicknessInX0;
     }
     // eps = K thick(pcor) q2b2(p)
     pb += epsb * depsP;
     pcorb += epsb * depsC;
     // pcor = 1 / |n . d|
-    const double cb = -pcorb / (c * c) * sgn;
+    const double cb = -pcorb * (pcor * pcor) * sgn;
     const double nr[3] = {pl.r[2], pl.r[5], pl.r[8]};
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -1081,7 +1101,7 @@ struct TrackAdjoint {
       zeroPlanes(planePrev - tf.seqFirst + 1, plane - tf.seqFirst);
       tf.pathLimit();
       tf.navTarget();
-      const double qop = tf.q / tf.p;
+      const double qop = divD(tf.q, tf.p);
       int nst = 0;
       for (;;) {
         if (nst >= g.max_seg_steps) {
@@ -1154,21 +1174,22 @@ struct TrackAdjoint {
         jacInitVJP(dEnd, Ab, Gb, dPre, Rb);
       }
       // material on this plane, recomputed from the filtered state
-      const double pF = fabs(1.0 / P.xf[4]);
+      const double pF = fabs(recipD(P.xf[4]));
       double dF[3];
       {
         const SinCos s3 = oolSinCos(P.xf[3]), s2 = oolSinCos(P.xf[2]);
         const double ct = s3.c, stt = s3.s;
         const double v0 = s2.c * stt, v1 = s2.s * stt, v2 = ct;
-        const double vn = sqrt(v0 * v0 + v1 * v1 + v2 * v2);
-        dF[0] = v0 / vn;
-        dF[1] = v1 / vn;
-        dF[2] = v2 / vn;
+        double vn, ivn;
+        rootD(v0 * v0 + v1 * v1 + v2 * v2, vn, ivn);
+        dF[0] = v0 * ivn;
+        dF[1] = v1 * ivn;
+        dF[2] = v2 * ivn;
       }
       MaterialFwd Mt;
       Mt.run(a, pl, pF, dF);
       // adjoint of the momentum after the plane from that of q/p
-      const double pAfterb = -qb * tf.q / (Mt.pOut * Mt.pOut);
+      const double pAfterb = -qb * tf.q * recipD(Mt.pOut * Mt.pOut);
       double dbm[3] = {db[0], db[1], db[2]}, nbm[3] = {0, 0, 0};
       const double pFb = Mt.vjp(a, pl, dF, pAfterb, lds[(kLDS_CB + cidx(2, 2)) * KF_BLOCK],
                                 lds[(kLDS_CB + cidx(3, 3)) * KF_BLOCK],
@@ -1265,11 +1286,8 @@ struct TrackAdjoint {
       }
       qb = qbb;
     }
-    if (st) {
-      zeroPlanes(0, slots);
-      sb = 0.0;
-    }
-    g.scale_adj[loc] = sb;
+    if (st) zeroPlanes(0, slots);
+    g.scale_adj[loc] = st ? 0.0 : sb / a.field.scale;
     if (g.status) g.status[i] = st;
   }
 };
