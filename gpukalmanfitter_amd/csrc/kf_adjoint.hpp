@@ -594,25 +594,29 @@ struct PlaneFwd {
     for (int q = 0; q < 5; ++q)
 #pragma unroll
       for (int c = 0; c < 5; ++c) Cm[q][c] = cm[sidx(q, c)];
+    // Cp = jb Cm jb^T, upper triangle; row 4 of jb is e4
     double T[5][5];  // jb Cm
 #pragma unroll
-    for (int q = 0; q < 5; ++q)
+    for (int q = 0; q < 4; ++q)
 #pragma unroll
       for (int c = 0; c < 5; ++c) {
-        double s = 0.0;
+        double s = jb[q][0] * Cm[0][c];
 #pragma unroll
-        for (int m = 0; m < 5; ++m) s += jb[q][m] * Cm[m][c];
+        for (int m = 1; m < 5; ++m) s += jb[q][m] * Cm[m][c];
         T[q][c] = s;
       }
 #pragma unroll
-    for (int q = 0; q < 5; ++q)
+    for (int q = 0; q < 4; ++q) {
 #pragma unroll
-      for (int c = 0; c < 5; ++c) {
-        double s = 0.0;
+      for (int c = q; c < 4; ++c) {
+        double s = T[q][0] * jb[c][0];
 #pragma unroll
-        for (int m = 0; m < 5; ++m) s += T[q][m] * jb[c][m];
-        Cp[q][c] = s;
+        for (int m = 1; m < 5; ++m) s += T[q][m] * jb[c][m];
+        Cp[q][c] = Cp[c][q] = s;
       }
+      Cp[q][4] = Cp[4][q] = T[q][4];
+    }
+    Cp[4][4] = Cm[4][4];
     xp[0] = u0[0] * (pos[0] - cc[0]) + u0[1] * (pos[1] - cc[1]) + u0[2] * (pos[2] - cc[2]);
     xp[1] = u1[0] * (pos[0] - cc[0]) + u1[1] * (pos[1] - cc[1]) + u1[2] * (pos[2] - cc[2]);
     xp[2] = oolAtan2(d[1], d[0]);
@@ -640,7 +644,7 @@ struct PlaneFwd {
   // Backward of chi2 + update + bound state.  In: xfb (adjoint of the
   // filtered parameters), Cfb (symmetric adjoint of the filtered covariance),
   // chi2 weight 1.  Out: the adjoints of pos, d, A, G, k4, q/p and of the
-  // segment-start covariance (Cmb, symmetric), and of the plane (cb, Rb).
+  // segment-start covariance (Cmb, the upper triangle), and of the plane (cb, Rb).
   KFD_INLINE void vjp(const double d[3], const double pos[3], const double A[3][5],
                       const double k4[3], const double xfb[5], const double Cfb[5][5],
                       double posb[3], double db[3], double Ab[3][5], double Gb[3][3],
@@ -726,29 +730,38 @@ struct PlaneFwd {
     xpb[1] -= rb[1];
 
     // ---- covariance transport Cp = jb Cm jb^T
-    double jbb[5][5];
+    double jbb[4][5];
     {
       double T[5][5];  // Cpb jb
 #pragma unroll
       for (int q = 0; q < 5; ++q)
 #pragma unroll
         for (int c = 0; c < 5; ++c) {
-          double s = 0.0;
+          double s = Cpb[q][0] * jb[0][c];
 #pragma unroll
-          for (int m = 0; m < 5; ++m) s += Cpb[q][m] * jb[m][c];
+          for (int m = 1; m < 4; ++m) s += Cpb[q][m] * jb[m][c];
+          if (c == 4) s += Cpb[q][4];
           T[q][c] = s;
         }
+      // jb^T Cpb jb, upper triangle
 #pragma unroll
       for (int q = 0; q < 5; ++q)
 #pragma unroll
-        for (int c = 0; c < 5; ++c) {
-          double s = 0.0, w2 = 0.0;
+        for (int c = q; c < 5; ++c) {
+          double s = jb[0][q] * T[0][c];
 #pragma unroll
-          for (int m = 0; m < 5; ++m) {
-            s += jb[m][q] * T[m][c];  // jb^T Cpb jb
-            w2 += T[q][m] * Cm[m][c];  // Cpb jb Cm
-          }
+          for (int m = 1; m < 4; ++m) s += jb[m][q] * T[m][c];
+          if (q == 4) s += T[4][c];
           Cmb[q][c] = s;
+        }
+      // 2 Cpb jb Cm; row 4 of jb is fixed
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int c = 0; c < 5; ++c) {
+          double w2 = T[q][0] * Cm[0][c];
+#pragma unroll
+          for (int m = 1; m < 5; ++m) w2 += T[q][m] * Cm[m][c];
           jbb[q][c] = 2.0 * w2;
         }
     }
@@ -1102,6 +1115,11 @@ struct TrackAdjoint {
       tf.targetReached = false;
       tf.cur = -1;
       int planePrev = tf.seqFirst - 1, hitPrev = 0;
+      // the hit, loaded with the checkpoint (one wait for both) and kept in the
+      // LDS slots of the plane's adjoint until that is formed
+      const int64_t hit = tf.h0 + hitRel;
+      const double hm[5] = {a.hit_meas[hit], a.hit_meas[a.n_hits + hit], a.hit_cov[hit],
+                            a.hit_cov[a.n_hits + hit], a.hit_cov[2 * a.n_hits + hit]};
       if (k == 0) {
         double pv[6];
 #pragma unroll
@@ -1124,7 +1142,8 @@ struct TrackAdjoint {
         tf.q = charge;
         tf.measured = k;
       }
-      const int64_t hit = tf.h0 + hitRel;
+#pragma unroll
+      for (int m = 0; m < 5; ++m) lds[(kLDS_PL + m) * KF_BLOCK] = hm[m];
       zeroPlanes(planePrev - tf.seqFirst + 1, plane - tf.seqFirst);
       tf.pathLimit();
       tf.navTarget();
@@ -1183,9 +1202,9 @@ struct TrackAdjoint {
         for (int c = 0; c < 3; ++c) GEnd[r][c] = tf.G[r][c];
       }
       PlaneFwd P;
-      P.run(pl, dEnd, posEnd, AEnd, GEnd, k4, qop, tf.cov, a.hit_meas[hit],
-            a.hit_meas[a.n_hits + hit], a.hit_cov[hit], a.hit_cov[a.n_hits + hit],
-            a.hit_cov[2 * a.n_hits + hit]);
+      P.run(pl, dEnd, posEnd, AEnd, GEnd, k4, qop, tf.cov, lds[kLDS_PL * KF_BLOCK],
+            lds[(kLDS_PL + 1) * KF_BLOCK], lds[(kLDS_PL + 2) * KF_BLOCK],
+            lds[(kLDS_PL + 3) * KF_BLOCK], lds[(kLDS_PL + 4) * KF_BLOCK]);
       // ---- backward at the plane
       double cb[3] = {0, 0, 0}, Rb[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
       double dPre[3] = {0, 0, 0};  // adjoint of the direction at the plane (before the update)
