@@ -9,21 +9,19 @@ whole batch with inputs already resident in HBM; the timed region is exactly
 --steps fits bracketed by device synchronisation.  Fits run in every precision
 given by --precision (first one is the headline `value`).
 
-A fit is two launches on one stream: the forward filter (start, steps,
-gain-matrix update on every surface, per-surface store writes) and the
-smoother plus back-propagation to the perigee (store reads).  The roofline
-object is for the longer launch of the headline precision.  The path is bound
+A fit without track states is one launch (forward filter with the smoothed first
+state carried along, then back to the perigee), for which the roofline object is.
+The path is bound
 by the vector ALU: the roofline time of a launch is T_roof = F32 / 157.3 +
 F64 / 78.6 TFLOP/s (the MI355X vector peaks) for its algorithmic flops, the
 flops of the reference formulation with structural zeros and identities
 removed, counted per track by the counting build of the CPU oracle and split
 into the float and double classes of the mixed mode; achieved = F / T, peak
 = F / T_roof, frac = T_roof / T.  Beside it: the launch's external I/O bytes
-(inputs it reads, results it writes) against 8 TB/s, the bytes of its
-working storage (smoother store, hand-over) and the HBM traffic rocprofv3
+(inputs it reads, results it writes) against 8 TB/s and the HBM traffic rocprofv3
 measured (FETCH_SIZE + WRITE_SIZE).  Launch durations are the mean over the
-timed steps of HIP events the library records on the launch stream before,
-between and after the two launches.
+timed steps of HIP events the library records on the launch stream around the
+launch and the (as a rule empty) pass over tracks handed to the RTS smoother.
 """
 import argparse
 import json
@@ -45,8 +43,9 @@ FLOPS32_PER_TRACK = 8109.0
 FLOPS32_BWD_PER_TRACK = 784.0
 FP64_PEAK_TFLOPS = 78.6
 FP32_PEAK_TFLOPS = 157.3
-# External I/O bytes per config-2 track and launch (10 hits): what the caller
-# hands in and gets back, read or written by that launch.
+# External I/O bytes per config-2 track (10 hits): what the caller hands in and
+# gets back, read or written by the two launches of a fit with track states (the
+# fused launch reads and writes both but the 48 bytes the second one reads again).
 #   forward  = inputs 696 (start parameters 48 + covariance 168 + perigee 24
 #              + sequence 8 + hit offset 8 + 10 hits x 44) + chi2/ndf/n_measured 16;
 #   backward = perigee, sequence and hit offsets 48 + outputs 220 (params 48,
@@ -59,14 +58,11 @@ EXT_BYTES_PER_TRACK = {"forward": 712, "backward": 268}
 DESIGN_BYTES_PER_TRACK = {("fp64", "forward"): 5944, ("fp64", "backward"): 5500,
                           ("mixed", "forward"): 3944, ("mixed", "backward"): 3500}
 HBM_PEAK_GBS = 8000.0
-# HBM bytes per launch (fetched + written) of the two fit kernels on this
-# workload, from rocprofv3 FETCH_SIZE / WRITE_SIZE scaled by the copy-kernel
-# calibration (profiles/kf_fit_config2_1M_tracks.md).
+# HBM bytes per launch (fetched + written) of the fused fit on this workload, from
+# rocprofv3 FETCH_SIZE / WRITE_SIZE scaled by the copy-kernel calibration
+# (profiles/kf_fused_fit_and_adjoint.md).
 TRAFFIC_TRACKS = 1048576
-TRAFFIC_BYTES_PER_LAUNCH = {
-    ("fp64", "forward"): 2.318e9 + 5.662e9, ("fp64", "backward"): 5.555e9 + 0.231e9,
-    ("mixed", "forward"): 2.265e9 + 3.481e9, ("mixed", "backward"): 3.510e9 + 0.231e9,
-}
+TRAFFIC_BYTES_PER_LAUNCH = {"fp64": 2.562e9 + 0.474e9, "mixed": 2.170e9 + 0.247e9}
 PARAM_NAMES = ("loc0", "loc1", "phi", "theta", "qop", "t")
 
 
@@ -190,52 +186,28 @@ def param_errors(gpu_results, ores, n):
     return errors
 
 
-def launch_figures(prec, phase, n, ms):
-    """Flops, roofline time and bytes of one launch of `phase` (module docstring)."""
-    mixed = prec == "mixed"
-    f = FLOPS_PER_TRACK - FLOPS_BWD_PER_TRACK if phase == "forward" else FLOPS_BWD_PER_TRACK
-    g = 0.0
-    if mixed:
-        g = FLOPS32_PER_TRACK - FLOPS32_BWD_PER_TRACK if phase == "forward" else FLOPS32_BWD_PER_TRACK
-    t_roof = n * (g / (FP32_PEAK_TFLOPS * 1e12) + (f - g) / (FP64_PEAK_TFLOPS * 1e12))
-    t = ms * 1e-3
-    ext = EXT_BYTES_PER_TRACK[phase]
-    design = DESIGN_BYTES_PER_TRACK[(prec, phase)]
-    traffic = TRAFFIC_BYTES_PER_LAUNCH.get((prec, phase))
-    if traffic is not None:
-        traffic *= n / TRAFFIC_TRACKS
-    # the launch of the default schedule on a constant field without track
-    # states (the last two template arguments: kFieldConst = 1, no recording)
-    return {"kernel": "kf_fit_kernel<%s, %s, true, false, 1, false, 1, false>" % (
-                "float" if mixed else "double", "true" if phase == "forward" else "false"),
-            "kernel_ms": ms, "flops_per_track": f, "fp32_flops_per_track": g,
-            "t_roof_ms": t_roof * 1e3, "tflop_per_s": f * n / t / 1e12,
-            "vector_peak_tflop_per_s": f * n / t_roof / 1e12, "vector_frac": t_roof / t,
-            "hbm_ext": {"bytes_per_track": ext, "gb_per_s": ext * n / t / 1e9,
-                        "frac": ext * n / t / 1e9 / HBM_PEAK_GBS},
-            "hbm_design": {"bytes_per_track": design, "gb_per_s": design * n / t / 1e9,
-                           "frac": design * n / t / 1e9 / HBM_PEAK_GBS},
-            "traffic": traffic,
-            "traffic_over_ext": traffic / (ext * n) if traffic else None,
-            "traffic_over_design": traffic / (design * n) if traffic else None}
-
-
 def roofline(prec, n, phase_ms):
-    """Vector-ALU roofline of the dominant launch (see the module docstring)."""
-    ms = {"forward": phase_ms[0], "backward": phase_ms[1]}
-    k = max(ms, key=ms.get)
-    other = "backward" if k == "forward" else "forward"
-    dom = launch_figures(prec, k, n, ms[k])
-    return {"bound": "vector_alu", "achieved": dom["tflop_per_s"],
-            "peak": dom["vector_peak_tflop_per_s"], "unit": "TFLOP/s",
-            "frac": dom["vector_frac"], "traffic": dom["traffic"],
-            "kernel": dom["kernel"], "kernel_ms": ms[k], "t_roof_ms": dom["t_roof_ms"],
+    """Vector-ALU roofline of the fused launch (see the module docstring)."""
+    mixed = prec == "mixed"
+    f, g = FLOPS_PER_TRACK, FLOPS32_PER_TRACK if mixed else 0.0
+    t_roof = n * (g / (FP32_PEAK_TFLOPS * 1e12) + (f - g) / (FP64_PEAK_TFLOPS * 1e12))
+    ms = phase_ms[0]
+    t = ms * 1e-3
+    ext = EXT_BYTES_PER_TRACK["forward"] + EXT_BYTES_PER_TRACK["backward"] - 48
+    traffic = TRAFFIC_BYTES_PER_LAUNCH[prec] * n / TRAFFIC_TRACKS
+    # constant field (kFieldConst = 1), plane table in LDS, one lane per track
+    return {"bound": "vector_alu", "achieved": f * n / t / 1e12, "peak": f * n / t_roof / 1e12,
+            "unit": "TFLOP/s", "frac": t_roof / t, "traffic": traffic,
+            "kernel": "kf_fused_kernel<%s, true, 1, 1>" % ("float" if mixed else "double"),
+            "kernel_ms": ms, "t_roof_ms": t_roof * 1e3, "flops_per_track": f,
+            "fp32_flops_per_track": g,
             "peak_note": "F / (F32 / 157.3 + F64 / 78.6 TFLOP/s): the MI355X FP32 and FP64 "
                          "vector peaks weighted by the launch's float and double flops",
-            "hbm": dict(dom["hbm_ext"], peak_gb_per_s=HBM_PEAK_GBS,
-                        note="external I/O of the launch (inputs read, results written) "
-                             "against 8 TB/s"),
-            "dominant_launch": dom, "other_launch": launch_figures(prec, other, n, ms[other])}
+            "hbm": {"bytes_per_track": ext, "gb_per_s": ext * n / t / 1e9,
+                    "frac": ext * n / t / 1e9 / HBM_PEAK_GBS, "peak_gb_per_s": HBM_PEAK_GBS,
+                    "note": "external I/O of the launch (inputs read, results written) "
+                            "against 8 TB/s"},
+            "traffic_over_ext": traffic / (ext * n)}
 
 
 def adjoint_leg(steps, warmup, sample):
