@@ -178,7 +178,8 @@ typedef struct kf_schedule {
                               fit without track states does so of itself where
                               options.max_states and n_hits show unequal lengths and
                               the batch exceeds one wave per SIMD; same bits) */
-  int32_t persistent;      /* 1: resident waves pull 64-track chunks from a work queue */
+  int32_t persistent;      /* 1: resident waves pull 64-track chunks from a work queue (fits
+                              with track states; the others take one track per lane) */
   int32_t waves_per_cu;    /* persistent grid size, waves per compute unit (default 4) */
   int32_t chunks_per_grab; /* work-queue granularity, 64-track chunks per grab (default 1) */
   int32_t lanes_per_track; /* lanes cooperating on one track (the counterpart of the
