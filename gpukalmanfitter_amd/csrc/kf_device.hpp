@@ -323,6 +323,14 @@ KFD_INLINE double recipD(double x) {
   return 1.0 / x;
 #endif
 }
+// 1 / x to about seven digits
+KFD_INLINE double recipEstimate(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_rcp(x);
+#else
+  return 1.0 / x;
+#endif
+}
 // n / d with the quotient's residual added back
 KFD_INLINE double divD(double n, double d) {
 #if defined(__HIP_DEVICE_COMPILE__)

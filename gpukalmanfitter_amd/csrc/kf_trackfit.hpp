@@ -952,8 +952,7 @@ struct TrackFit {
   FxPair *fx = nullptr;  // this lane's first pair
   bool fxOk = true;
   S fxDiag[3];                          // kFxRts: (2,2), (3,3), (4,4) before the material update
-  S fxVphi = (S)0, fxVth = (S)0;        // largest filtered variances of phi and theta
-  double fxPhi = 0.0, fxTheta = 0.0;    // largest |phi| and |theta - pi/2| of a filtered state
+  double fxLimit = kDblMax;  // total chi2 below which no smoothed angle can wrap (fxAngles)
 
   KFD_INLINE void fxLoad(int p, double &x, double &y) const {
     const FxPair v = fx[p * KF_FUSED_BLOCK];
@@ -1184,17 +1183,28 @@ struct TrackFit {
     }
     return ok;
   }
+  // Whether the smoothed phi and theta of this state can pass their bounds.  A
+  // smoothed state lies within sqrt(X) of the filtered one in units of the
+  // filtered errors, X the chi2 that the later measurements add (it minimises
+  // that distance squared plus a sum of squares, whose minimum is X), so the
+  // angle stays a distance d away from its bound while X < d^2 / V: the total
+  // chi2 must stay below the chi2 so far plus d^2 / V, for every state and both
+  // angles; 2 % and 1e-6 cover rounding.  Not asked for state 0, whose smoothed
+  // value is wrapped last, by both smoothers.
+  KFD_INLINE void fxAngles(const double xf[6]) {
+    const double dp = (kPi - 1e-6) - fabs(xf[2]), dt = (0.5 * kPi - 1e-6) - fabs(xf[3] - 0.5 * kPi);
+    const double vp = (double)cov[sidx(2, 2)], vt = (double)cov[sidx(3, 3)];
+    fxOk = fxOk && 0.0 < fmin(dp, dt) && 0.0 <= fmin(vp, vt) && vp + vt < kDblMax;
+    // the smaller of dp^2 / vp and dt^2 / vt by one reciprocal, whose estimate is
+    // far within the 2 % (variances of 0 set no limit: the state is exact)
+    const double x = fmin((dp * dp) * vt, (dt * dt) * vp) * recipEstimate(vp * vt);
+    fxLimit = fmin(fxLimit, chi2sum + x * (1.0 / (1.02 * 1.02)));
+  }
   // Whether the RTS recursion over this track's states is free of wraps,
   // clamps and non-finite gains, so that its result for state 0 is this
-  // smoother's.  A smoothed state lies within sqrt(X) of the filtered one in
-  // units of the filtered errors, X the chi2 the later measurements add (it
-  // minimises that distance squared plus a sum of squares, whose minimum is
-  // X), so |phi| and |theta - pi/2| of every smoothed state are below the
-  // largest filtered value plus sqrt(largest filtered variance X); 2 % and
-  // 1e-6 cover rounding.  False on NaN.
+  // smoother's.  False on NaN.
   KFD_INLINE bool fxSafe(const double xs[6], const double cs[21]) const {
-    bool ok = fxOk && fxPhi + (1.02 * sqrt((double)fxVphi * chi2sum) + 1e-6) < kPi &&
-              fxTheta + (1.02 * sqrt((double)fxVth * chi2sum) + 1e-6) < 0.5 * kPi;
+    bool ok = fxOk && chi2sum < fxLimit;
 #pragma unroll
     for (int m = 0; m < 6; ++m) ok = ok && fabs(xs[m]) < kDblMax;
 #pragma unroll
@@ -1867,13 +1877,8 @@ struct TrackFit {
     for (int c = 1; c < 6; ++c) cov[sidx(1, c)] = (S)t01[5 + c];
     chi2sum = chi2sum + chi2;
     }
-    if constexpr (kFirst) {
-      const double ap = fabs(xf[2]), at = fabs(xf[3] - 0.5 * kPi);
-      fxPhi = (ap < fxPhi) ? fxPhi : ap;
-      fxTheta = (at < fxTheta) ? fxTheta : at;
-      fxVphi = (cov[sidx(2, 2)] < fxVphi) ? fxVphi : cov[sidx(2, 2)];
-      fxVth = (cov[sidx(3, 3)] < fxVth) ? fxVth : cov[sidx(3, 3)];
-    }
+    if constexpr (kFirst)
+      if (k > 0) fxAngles(xf);
     correctParams(xf);
     if constexpr (kStore) {
       storePar(s, KF_SD_XF, xf);
