@@ -471,31 +471,26 @@ int setupStores(kf_ctx *ctx, int precision, bool track_states, bool checkpoints,
 
 // Working storage of a fused fit for slices of up to `slice` positions: the
 // kept first states (carry), and for tracks that go to the RTS program the
-// list, and `waves` store chunks with their hand-over (redo).
+// list, and store chunks with their hand-over (redo), the first `rts` of them
+// for the waves near the wrap.
 struct FusedLayout {
   StoreLayout store;   // of waves x 64 lanes
   size_t carry_bytes, list_bytes;
-  int64_t lanes;
+  int64_t lanes, rts;
   size_t redo_bytes() const { return list_bytes + store.carry_bytes; }
 };
-FusedLayout fusedLayout(int precision, int64_t slice, int64_t waves, int32_t max_states) {
+FusedLayout fusedLayout(int precision, int64_t slice, int32_t max_states, size_t budget) {
   FusedLayout F;
-  F.lanes = waves * 64;
+  // as many chunks of each kind as the slice has waves, within the limits and,
+  // between the two, the budget; one for handed-back tracks at least
+  const size_t one = storeLayout(precision, false, false, 64, max_states).store();
+  const int64_t waves = (slice + 63) / 64, fit = std::max<int64_t>((int64_t)(budget / one), 1);
+  F.rts = std::min(std::min<int64_t>(waves, KF_RTS_WAVES), fit / 2);
+  F.lanes = (F.rts + std::min(std::min<int64_t>(waves, KF_REDO_WAVES), fit - F.rts)) * 64;
   F.store = storeLayout(precision, false, false, F.lanes, max_states);
   F.carry_bytes = ((size_t)slice * firstBytes(precision) + 255) / 256 * 256;
   F.list_bytes = ((KF_REDO_LIST + (size_t)slice) * sizeof(uint32_t) + 255) / 256 * 256;
   return F;
-}
-
-// Store chunks for tracks fitted again: as many as the slice has waves, within
-// the store budget and KF_REDO_WAVES (none or a few are used as a rule).
-int64_t redoWaves(int precision, int64_t slice, int32_t max_states, size_t budget) {
-  const size_t one = storeLayout(precision, false, false, 64, max_states).store();
-  int64_t w = (slice + 63) / 64;
-  if (w > KF_REDO_WAVES) w = KF_REDO_WAVES;
-  const int64_t fit = (int64_t)(budget / one);
-  if (w > fit) w = fit;
-  return w < 1 ? 1 : w;
 }
 
 void carveFused(const FusedLayout &F, void *store, void *carry, void *redo, kfd::FitArgs &a) {
@@ -508,6 +503,7 @@ void carveFused(const FusedLayout &F, void *store, void *carry, void *redo, kfd:
   a.redo_d = (double *)((char *)redo + F.list_bytes);
   a.redo_i = (int32_t *)(a.redo_d + KF_CARRY_D * (size_t)F.lanes);
   a.redo_lanes = F.lanes;
+  a.rts_waves = (int32_t)F.rts;
 }
 
 // The working storage of a fused fit, from the context's buffers (grown as
@@ -516,9 +512,7 @@ void carveFused(const FusedLayout &F, void *store, void *carry, void *redo, kfd:
 int setupFused(kf_ctx *ctx, int precision, int64_t slice, hipStream_t s, kfd::FitArgs &a) {
   const size_t budget = (ctx->budget < KF_REDO_STORE_BYTES) ? (size_t)ctx->budget
                                                             : (size_t)KF_REDO_STORE_BYTES;
-  const FusedLayout F = fusedLayout(precision, slice,
-                                    redoWaves(precision, slice, a.max_states, budget),
-                                    a.max_states);
+  const FusedLayout F = fusedLayout(precision, slice, a.max_states, budget);
   int rc = grow(ctx, &ctx->store, &ctx->store_bytes, F.store.store(), s, "state store");
   if (rc != KF_OK) return rc;
   rc = grow(ctx, &ctx->carry, &ctx->carry_bytes, F.carry_bytes, s, "hand-over buffer");
@@ -601,10 +595,8 @@ int kf_fit_noalloc(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt,
   // a fused fit: the redo store takes at most half of the workspace (one
   // chunk as a minimum)
   auto fused = [&](int64_t slice) {
-    return fusedLayout(opt->precision, slice,
-                       redoWaves(opt->precision, slice, a.max_states,
-                                 (size_t)KF_NOALLOC_WORKSPACE_BYTES / 2),
-                       a.max_states);
+    return fusedLayout(opt->precision, slice, a.max_states,
+                       (size_t)KF_NOALLOC_WORKSPACE_BYTES / 2);
   };
   // the largest multiple of 64 positions whose storage fits the workspace
   auto fits = [&](int64_t slice) {
@@ -743,7 +735,7 @@ int kf_fit(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt, const kf_res
     // a fit that is one kernel has no second phase to time
     kfd::FitArgs whole = a;
     sliceRange(whole, 0, slice);
-    ctx->one_kernel = fused && slice >= a.n && kfd::redoChunkPerWave(whole, std::max(L.lanes_per_track, 1));
+    ctx->one_kernel = fused && slice >= a.n && kfd::redoSlotPerTrack(whole);
     e = launchSlices(a, L, opt->precision, res->track_states, slice,
                      ctx->one_kernel ? nullptr : ctx->evm, s);
     ctx->phase_timed = slice >= a.n;

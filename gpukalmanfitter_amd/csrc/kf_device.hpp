@@ -212,6 +212,25 @@ KFD_INLINE void fieldGrid(const DevField &f, double x, double y, double z, doubl
   }
 }
 
+// Either kind, in float, a grid's at the nearest lower corner: for estimates.
+KFD_INLINE void fieldNear(const DevField &f, const float x[3], float B[3]) {
+  if (!f.grid) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) B[k] = (float)(f.scale * f.b[k]);
+    return;
+  }
+  int idx[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const float q = (x[d] - (float)f.lo[d]) * (float)f.iw[d];
+    idx[d] = (int)fminf(fmaxf(q, 0.0f), (float)(f.n[d] - 1));
+    idx[d] = idx[d] > f.n[d] - 1 ? f.n[d] - 1 : idx[d];
+  }
+  const float *v = f.values + 3 * (((int64_t)idx[0] * f.n[1] + idx[1]) * f.n[2] + idx[2]);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) B[k] = (float)f.scale * v[k];
+}
+
 // Either kind, chosen by f.grid at run time.
 KFD_INLINE void fieldAt(const DevField &f, double x, double y, double z, double B[3]) {
   if (!f.grid) {

@@ -118,33 +118,100 @@ __global__ void __launch_bounds__(KF_BLOCK) kf_fit_kernel(FitArgs args) {
 // passed 304 B per state through memory: 1,048,576 tracks 2.03 -> 1.75 ms,
 // 500,003 ragged ones 2.81 -> 2.30 ms, 100,003 with material 1.93 -> 1.70 ms.
 //
-// A track that the fixed-point smoother leaves to the RTS program (TrackFit::
-// fxSafe; 1 in 200,000 of the material workload) is fitted again by its own
-// wave while the others go on, over a store chunk it takes from a pool (or its
-// own, redoChunkPerWave); when the pool is used up it goes to the list of the
-// redo kernel.  Waiting for
-// the redo kernel with all of them cost the material workload 0.9 ms per
-// call for a single track: the latency of one wave's fit of 40 planes.
+// Tracks for the RTS program (redoTrack), in three ways:
+//  - a track near the phi wrap (nearWrap) is left out by its lane and fitted by
+//    the waves at the front of the grid, rts_waves of them, which go through a
+//    share of the positions each and take the tracks they pick 64 at a time;
+//  - a track that the fixed-point smoother leaves in the end (TrackFit::fxSafe; 1
+//    in 2,000 of the material workload spread over azimuth) is fitted again by
+//    its own wave while the others go on, over a store slot of its own
+//    (redoSlotPerTrack) or a chunk that the wave takes from a pool;
+//  - when the pool is used up it goes to the list of the redo kernel.
+// Fitted after the fused pass alone, a single handed-back track cost a small
+// batch the RTS program's latency on top.  10,007 tracks of ten planes facing
+// phi = pi: 318 us so, 127 beside the others, 159 in the forward and backward kernels
+// (FP64; 361, 138 and 153 mixed); 1,048,576 of them 2,410, 1,791 and 2,881 us;
+// facing +x 96 us and 1,300 us either way.  Waiting for the redo kernel with all of
+// them cost the material workload 0.9 ms a call.
 //
-// redoTrack is a call so that its code and registers stay out of the fit's;
-// it reads the kernel's arguments where the kernel finds them.
-template <typename S>
-__device__ __attribute__((noinline)) void redoTrack(const FitArgs *args, int64_t i,
-                                                    int64_t slot) {
-  const FitArgs &a = *args;
+// redoTrack is a call so that its code and registers stay out of the fit's and
+// that a track's bits do not depend on which of the three it takes; it reads the
+// kernel's arguments where the kernel finds them, and the plane table in LDS
+// where the kernel has it there.
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __attribute__((address_space(3))) const DevPlane LdsPlane;
+#else
+typedef const DevPlane LdsPlane;
+#endif
+template <typename S, bool PLDS, int FK>
+static __device__ __attribute__((noinline)) void redoTrack(const FitArgs *args, int64_t i,
+                                                           int64_t slot, LdsPlane *table) {
+  const FitArgs &a = *uniformArgs(args);
   const uint32_t lane = (uint32_t)(slot & 63);
-  const ChunkBases<S> cb(a, slot);
+  const size_t per = (size_t)(slot >> 6) * (size_t)a.max_states * 64u;
+  double *d = a.tsd + per * KF_SD_N;
+  S *s = (S *)a.tss + per * KF_SS_N;
+  const DevPlane *planes = PLDS ? (const DevPlane *)table : a.planes;
   {
-    TrackFit<S, true, 1, false, false, kFieldAny, kKeepStates> tf(a, i, cb.d, cb.s, nullptr, nullptr,
-                                                                  lane, slot);
+    TrackFit<S, true, 1, false, false, FK, kKeepStates> tf(a, i, d, s, nullptr, nullptr, lane,
+                                                           slot);
+    tf.pls = planes;
     tf.redoSlots();
     tf.runForward();
   }
   {
-    TrackFit<S, false, 1, false, false, kFieldAny, kKeepStates> tf(a, i, cb.d, cb.s, nullptr,
-                                                                   nullptr, lane, slot);
+    TrackFit<S, false, 1, false, false, FK, kKeepStates> tf(a, i, d, s, nullptr, nullptr, lane,
+                                                            slot);
+    tf.pls = planes;
     tf.redoSlots();
     tf.runBackward();
+  }
+}
+
+// The plane table to dynamic LDS.
+KFD_INLINE const DevPlane *tableToLds(const FitArgs &args, double *lds_table) {
+  const double *src = (const double *)args.planes;
+  const int words = args.n_planes * (int)(sizeof(DevPlane) / sizeof(double));
+  for (int w = threadIdx.x; w < words; w += (int)blockDim.x) lds_table[w] = src[w];
+  __syncthreads();
+  return (const DevPlane *)lds_table;
+}
+
+// One of the waves for tracks near the wrap: its share of the positions, every
+// rts_waves-th 64 of them (sorted by length or by angle, each then has as much to
+// do), the picked ones collected, at most 63 + 64, until a wave is full.
+template <typename S, bool PLDS, int FK>
+KFD_INLINE void fitNearWrap(const FitArgs &args, int64_t wave, uint32_t *list, LdsPlane *table) {
+  const FitArgs *ka = (const FitArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+  if (wave >= args.rts_waves) return;
+  const int lane = (int)(threadIdx.x & 63u);
+  int n = 0;
+  for (int64_t at = wave * 64; at < args.count || n > 0;) {
+    while (n < 64 && at < args.count) {
+      const int64_t local = at + lane;
+      bool pick = false;
+      if (local < args.count) {
+        const int64_t pos = args.first + local;
+        const int64_t i = args.order ? (int64_t)args.order[pos] : pos;
+        pick = nearWrap(ka, i);
+      }
+      const uint64_t m = __ballot(pick);
+      if (pick) list[n + __popcll(m & ((1ull << lane) - 1ull))] = (uint32_t)local;
+      n += __popcll(m);
+      at += args.rts_waves * (int64_t)64;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const int take = (n < 64) ? n : 64;
+    const uint32_t local = (lane < take) ? list[lane] : 0u;
+    const uint32_t rest = (lane + 64 < n) ? list[lane + 64] : 0u;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (lane + 64 < n) list[lane] = rest;
+    n -= take;
+    if (lane < take) {
+      const int64_t pos = args.first + (int64_t)local;
+      redoTrack<S, PLDS, FK>(ka, args.order ? (int64_t)args.order[pos] : pos, wave * 64 + lane,
+                             table);
+    }
   }
 }
 
@@ -152,16 +219,19 @@ template <typename S, bool PLDS, int L, int FK>
 __global__ void __launch_bounds__(KF_FUSED_BLOCK) kf_fused_kernel(FitArgs args) {
   using Fit = TrackFit<S, true, L, false, false, FK, kKeepFirst>;
   __shared__ typename Fit::FxPair sums[Fit::kFxN * KF_FUSED_BLOCK];
+  __shared__ uint32_t picked[KF_FUSED_BLOCK / 64][128];
   extern __shared__ double lds_table[];
   const DevPlane *planes = args.planes;
-  if constexpr (PLDS) {
-    const double *src = (const double *)args.planes;
-    const int words = args.n_planes * (int)(sizeof(DevPlane) / sizeof(double));
-    for (int w = threadIdx.x; w < words; w += KF_FUSED_BLOCK) lds_table[w] = src[w];
-    __syncthreads();
-    planes = (const DevPlane *)lds_table;
+  if constexpr (PLDS) planes = tableToLds(args, lds_table);
+  LdsPlane *table = PLDS ? (LdsPlane *)planes : nullptr;
+  const FitArgs *ka = (const FitArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+  const uint32_t rtsBlocks = (uint32_t)rtsBlocksOf(args);
+  if (blockIdx.x < rtsBlocks) {
+    const int w = (int)(threadIdx.x >> 6), per = rtsPerBlock(args);
+    if (w < per) fitNearWrap<S, PLDS, FK>(args, (int64_t)blockIdx.x * per + w, picked[w], table);
+    return;
   }
-  const int64_t t = (int64_t)blockIdx.x * KF_FUSED_BLOCK + threadIdx.x;
+  const int64_t t = (int64_t)(blockIdx.x - rtsBlocks) * KF_FUSED_BLOCK + threadIdx.x;
   const int64_t local = t / L;
   if (local >= args.count) return;
   const int64_t pos = args.first + local;
@@ -172,43 +242,48 @@ __global__ void __launch_bounds__(KF_FUSED_BLOCK) kf_fused_kernel(FitArgs args) 
     tf.setRank((uint32_t)(t % L));
     tf.pls = planes;
     tf.fx = sums + threadIdx.x;
+    if (rtsBlocks > 0) tf.picker = ka;
     redo = !tf.runFused() && tf.lead;
   }
   const uint64_t redoMask = __ballot(redo);
   if (redoMask == 0) return;
-  if (redoChunkPerWave(args, L)) {
-    if (redo) redoTrack<S>((const FitArgs *)__builtin_amdgcn_kernarg_segment_ptr(), i, t);
-    return;
+  int64_t slot = (int64_t)args.rts_waves * 64 + local;
+  if (!redoSlotPerTrack(args)) {
+    const int first = __ffsll((unsigned long long)redoMask) - 1;
+    const int lane = (int)(threadIdx.x & 63u);
+    uint32_t chunk = 0;
+    if (lane == first) chunk = atomicAdd(args.redo, 1u);
+    chunk = (uint32_t)__shfl((int)chunk, first, 64);
+    slot = ((int64_t)args.rts_waves + chunk) * 64 + lane;
+    if (slot >= args.redo_lanes) {
+      if (redo) args.redo[KF_REDO_LIST + atomicAdd(args.redo + 1, 1u)] = (uint32_t)local;
+      return;
+    }
   }
-  const int first = __ffsll((unsigned long long)redoMask) - 1;
-  const int lane = (int)(threadIdx.x & 63u);
-  uint32_t chunk = 0;
-  if (lane == first) chunk = atomicAdd(args.redo, 1u);
-  chunk = (uint32_t)__shfl((int)chunk, first, 64);
-  if (!redo) return;
-  if ((int64_t)chunk * 64 < args.redo_lanes)
-    redoTrack<S>((const FitArgs *)__builtin_amdgcn_kernarg_segment_ptr(), i,
-                 (int64_t)chunk * 64 + lane);
-  else
-    args.redo[KF_REDO_LIST + atomicAdd(args.redo + 1, 1u)] = (uint32_t)local;
+  if (redo) redoTrack<S, PLDS, FK>(ka, i, slot, table);
 }
 
 // The tracks that found no store chunk in the fused kernel, 64 at a time per
-// wave.  Usually the list is empty and the kernel ends at once.  The last
-// block zeroes the counters for the next fit (every block has read the count
-// when it takes its ticket).
-template <typename S>
-__global__ void __launch_bounds__(64) kf_redo_kernel(FitArgs args) {
+// wave, over all the chunks.  Usually the list is empty and the kernel ends at
+// once.  The last block zeroes the counters for the next fit (every wave has read
+// the count when its block takes its ticket).
+template <typename S, bool PLDS, int FK>
+__global__ void __launch_bounds__(KF_FUSED_BLOCK) kf_redo_kernel(FitArgs args) {
+  extern __shared__ double lds_table[];
   const uint32_t n = __hip_atomic_load(args.redo + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const uint32_t lane = threadIdx.x;
-  const int64_t slot = (int64_t)blockIdx.x * 64 + lane;
-  for (int64_t e = slot; e < (int64_t)n; e += args.redo_lanes) {
-    const int64_t pos = args.first + (int64_t)args.redo[KF_REDO_LIST + e];
-    redoTrack<S>((const FitArgs *)__builtin_amdgcn_kernarg_segment_ptr(),
-                 args.order ? (int64_t)args.order[pos] : pos, slot);
-  }
+  const DevPlane *planes = args.planes;
+  if constexpr (PLDS)
+    if (n > 0) planes = tableToLds(args, lds_table);
+  const int64_t slot = (int64_t)blockIdx.x * KF_FUSED_BLOCK + threadIdx.x;
+  if (slot < args.redo_lanes)
+    for (int64_t e = slot; e < (int64_t)n; e += args.redo_lanes) {
+      const int64_t pos = args.first + (int64_t)args.redo[KF_REDO_LIST + e];
+      redoTrack<S, PLDS, FK>((const FitArgs *)__builtin_amdgcn_kernarg_segment_ptr(),
+                             args.order ? (int64_t)args.order[pos] : pos, slot,
+                             PLDS ? (LdsPlane *)planes : nullptr);
+    }
   __syncthreads();
-  if (lane == 0 && atomicAdd(args.redo + 2, 1u) == gridDim.x - 1) {
+  if (threadIdx.x == 0 && atomicAdd(args.redo + 2, 1u) == gridDim.x - 1) {
     args.redo[0] = 0u;
     args.redo[1] = 0u;
     args.redo[2] = 0u;
@@ -291,7 +366,8 @@ hipError_t launchFit(const FitArgs *args, hipStream_t stream, hipEvent_t between
   }
   const bool plds = args->n_planes <= (sizeof(S) == sizeof(double) ? KF_FUSED_LDS_PLANES_FP64
                                                                    : KF_FUSED_LDS_PLANES_MIXED);
-  const dim3 fgrid((unsigned)((args->count * lpt + KF_FUSED_BLOCK - 1) / KF_FUSED_BLOCK));
+  const dim3 fgrid((unsigned)((args->count * lpt + KF_FUSED_BLOCK - 1) / KF_FUSED_BLOCK +
+                              rtsBlocksOf(*args)));
   const unsigned table = plds ? (unsigned)(args->n_planes * sizeof(DevPlane)) : 0u;
 #define KFD_FUSED2(PLDS_, L_, FK_)                                                             \
   hipLaunchKernelGGL((kf_fused_kernel<S, PLDS_, L_, FK_>), fgrid, dim3(KF_FUSED_BLOCK), table, \
@@ -317,9 +393,19 @@ hipError_t launchFit(const FitArgs *args, hipStream_t stream, hipEvent_t between
     const hipError_t e = hipEventRecord(between, stream);
     if (e != hipSuccess) return e;
   }
-  if (args->smoothing && !redoChunkPerWave(*args, lpt))
-    hipLaunchKernelGGL((kf_redo_kernel<S>), dim3((unsigned)(args->redo_lanes / 64)), dim3(64), 0,
-                       stream, *args);
+  if (args->smoothing && !redoSlotPerTrack(*args)) {
+    const dim3 rgrid((unsigned)((args->redo_lanes + KF_FUSED_BLOCK - 1) / KF_FUSED_BLOCK));
+#define KFD_REDO(PLDS_, FK_)                                                                  \
+  hipLaunchKernelGGL((kf_redo_kernel<S, PLDS_, FK_>), rgrid, dim3(KF_FUSED_BLOCK), table, stream, \
+                     *args)
+    if (!plds)
+      KFD_REDO(false, kFieldAny);
+    else if (args->field.grid)
+      KFD_REDO(true, kFieldGrid);
+    else
+      KFD_REDO(true, kFieldConst);
+#undef KFD_REDO
+  }
   return hipGetLastError();
 }
 

@@ -21,10 +21,14 @@
 // blocks (one wave per SIMD) still fit the 160 KB of a compute unit.
 #define KF_FUSED_LDS_PLANES_FP64 224
 #define KF_FUSED_LDS_PLANES_MIXED 112
-// Store chunks for tracks that the fused kernel hands to the RTS program, and
-// the memory they may take together.
-#define KF_REDO_WAVES 256
-#define KF_REDO_STORE_BYTES (256ull << 20)
+// Waves of the fused launch that run the RTS program over the tracks near the phi
+// wrap (nearWrap) beside the others, each with a store chunk of its own; store
+// chunks for tracks that turn out to need it later; and the memory all chunks
+// may take together.  Half the chip's SIMDs each: with 1,024 waves of the first
+// kind a bulk batch spread over azimuth fills a quarter of their lanes.
+#define KF_RTS_WAVES 512
+#define KF_REDO_WAVES 512
+#define KF_REDO_STORE_BYTES (2ull << 30)
 // doubles per track of the fused kernel's kept first state
 #define KF_FIRST_D 27
 
@@ -139,25 +143,53 @@ struct FitArgs {
   int32_t chunks_per_grab;
   uint32_t *queue;
   // Fused fits (no track states or checkpoints): carry_d holds the kept
-  // first states of FP64 ([KF_FIRST_D][count]).  Tracks handed back to the RTS
-  // program use tsd, tss (redo_lanes slots, one store chunk per wave) and
-  // redo_d, redo_i ([KF_CARRY_D], [KF_CARRY_I][redo_lanes]).  redo[0]: store
-  // chunks taken by waves of the fused kernel itself, redo[1]: positions
-  // left in the list for the redo kernel, redo[2]: its ticket (all 0 between
-  // fits); redo[KF_REDO_LIST ...]: the positions.
+  // first states of FP64 ([KF_FIRST_D][count]).  Tracks on the RTS program use
+  // tsd, tss (redo_lanes slots, one store chunk per 64) and redo_d, redo_i
+  // ([KF_CARRY_D], [KF_CARRY_I][redo_lanes]): the first rts_waves chunks are
+  // those of the waves for tracks near the wrap, the others are for tracks
+  // handed back later.  redo[0]: chunks of the latter taken by waves of the
+  // fused kernel, redo[1]: positions left in the list for the redo kernel,
+  // redo[2]: its ticket (all 0 between fits); redo[KF_REDO_LIST ...]: the
+  // positions.
   double *redo_d;
   int32_t *redo_i;
   uint32_t *redo;
   int64_t redo_lanes;
+  int32_t rts_waves;
 };
 #define KF_REDO_LIST 64
 
-// Whether every wave of a fused fit has a store chunk of its own for tracks it
-// hands to the RTS program (up to 256 waves, 16,384 tracks): no chunk is then
-// drawn from the pool, no list kept, and no redo kernel follows.  For small
-// batches that launch was 5 of 96 us.
-KFD_INLINE bool redoChunkPerWave(const FitArgs &a, int lanes_per_track) {
-  return (a.count * lanes_per_track + 63) / 64 * 64 <= a.redo_lanes;
+// Kernel arguments that a function called by a kernel is handed by address: the
+// address from scalar registers again, in the constant address space, so that what
+// is read there takes scalar loads and not one load per lane.
+KFD_INLINE const FitArgs *uniformArgs(const FitArgs *p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint64_t u = (uint64_t)p;
+  const uint64_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u);
+  const uint64_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
+  return (const FitArgs *)(const __attribute__((address_space(4))) FitArgs *)((hi << 32) | lo);
+#else
+  return p;
+#endif
+}
+
+// Whether every position of a fused fit has a store slot of its own for being
+// handed back (up to KF_REDO_WAVES x 64 tracks): no chunk is then drawn from the
+// pool, no list kept, and no redo kernel follows.  For small batches that launch
+// was 5 of 96 us.
+KFD_INLINE bool redoSlotPerTrack(const FitArgs &a) {
+  return a.rts_waves * (int64_t)64 + (a.count + 63) / 64 * 64 <= a.redo_lanes;
+}
+// Blocks of a fused launch that hold the waves for tracks near the wrap, and how
+// many each holds: one up to 256, whose compute unit it then has to itself (two
+// waves of one unit, in different parts of the program, refill each other's
+// instruction cache: 117 tracks facing phi = pi 124 -> 165 us), else all of its waves.
+KFD_INLINE int rtsPerBlock(const FitArgs &a) {
+  return a.rts_waves <= 256 ? 1 : KF_FUSED_BLOCK / 64;
+}
+KFD_INLINE int64_t rtsBlocksOf(const FitArgs &a) {
+  const int per = rtsPerBlock(a);
+  return a.smoothing ? (a.rts_waves + per - 1) / per : 0;
 }
 
 }  // namespace kfd
@@ -207,7 +239,7 @@ struct KfdLaunch {
 // smoother/back-propagation kernel (unless smoothing is off) -> track-state
 // export (if track_states_out is not NULL).  Without them: [work-queue
 // reset] -> fused kernel -> record `between` -> redo kernel (the last not where
-// redoChunkPerWave holds).  `launch` may be NULL (one thread per
+// redoSlotPerTrack holds).  `launch` may be NULL (one thread per
 // track, identity order).  With a persistent grid, args->queue and
 // args->chunks_per_grab must be set; with sorting, args->order.
 extern "C" hipError_t kfd_launch_fit(const kfd::FitArgs *args, int precision, hipStream_t stream,

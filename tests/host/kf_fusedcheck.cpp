@@ -54,4 +54,12 @@ int kfh_fit_fused(const kf_plane *planes, int32_t n_planes, const kfh_field *f,
                             n_measured, status, redo);
 }
 
+// Whether each track is given to the RTS program from the start (nearWrap).
+int kfh_near_wrap(const kf_plane *planes, int32_t n_planes, const kfh_field *f,
+                  const kf_tracks *tr, const kf_options *opt, int32_t *pick) {
+  Host h(planes, n_planes, f, tr, opt, true);
+  for (int64_t i = 0; i < h.a.n; ++i) pick[i] = nearWrap(&h.a, i) ? 1 : 0;
+  return 0;
+}
+
 }  // extern "C"

@@ -1,4 +1,5 @@
 """How many tracks the fused fit leaves to the RTS program, on the CPU build of both."""
+import ctypes as C
 import dataclasses
 
 import numpy as np
@@ -7,7 +8,9 @@ import pytest
 from gpukalmanfitter_amd import abi, configs
 from gpukalmanfitter_amd import generate as G
 
-from test_fused_fit import fused_fit, turned
+import oracle
+from test_adjoint_cpu import field_of
+from test_fused_fit import fused_fit, fused_lib, turned
 from test_host_fit import host_fit
 
 W = configs.WORKLOAD_FIT_OPTIONS
@@ -41,3 +44,97 @@ def test_facing_the_wrap(built, precision):
     b = turned(G.generate(1, n_tracks=2000), np.pi)
     f = fused_fit(b, abi.default_options(precision=precision, **W))
     assert 0.0 < (f["redo"] != 0).mean() < 0.06
+
+
+def near_wrap(b, opt):
+    lib = fused_lib()
+    P = C.c_void_p
+    lib.kfh_near_wrap.argtypes = [P, C.c_int32, P, C.POINTER(abi.kf_tracks),
+                                  C.POINTER(abi.kf_options), P]
+    pick = np.zeros(b.n_tracks, dtype=np.int32)
+    tr, fld = oracle.host_tracks(b), field_of(b, b.field.scale)
+    assert lib.kfh_near_wrap(b.planes, len(b.planes), C.addressof(fld), C.byref(tr),
+                             C.byref(opt), pick.ctypes.data) == 0
+    return pick != 0
+
+
+@pytest.mark.parametrize("cfg,most", [(1, 0.0), (3, 0.0), (5, 0.01)])
+def test_tracks_near_the_wrap_are_known_at_the_start(built, cfg, most):
+    """Of the tracks that the fused fit would leave in the end, next to none are
+    fitted by both programs: the rest are picked from their start, with few
+    others, and none where phi stays away from the wrap."""
+    b = G.generate(cfg, n_tracks=1500)
+    opt = abi.default_options(**dict(W, max_rk_trials=20))
+    assert not near_wrap(b, opt).any()
+    assert not near_wrap(turned(b, np.pi / 2), opt).any() or cfg == 5
+    back = turned(b, np.pi)
+    left, pick = fused_fit(back, opt)["redo"] != 0, near_wrap(back, opt)
+    assert left.any()
+    assert (left & ~pick).mean() <= most
+    assert pick.mean() <= 0.25
+
+
+def test_near_wrap_of_bad_input(built):
+    """Tracks that the fit refuses, and values that are not finite, are read
+    without going out of the plane table, and are not picked."""
+    b = turned(G.generate(1, n_tracks=6), np.pi)
+    b.seq_first[:] = [-1, 5, 2**31 - 1, 0, 0, 0]
+    b.seq_count[:] = [10, 6, 10, 0, 10, 10]
+    b.start_params[2, 4] = np.nan
+    b.start_params[4, 5] = np.nan
+    assert not near_wrap(b, abi.default_options(**W)).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("cfg,n", [(1, 117), (1, 16385), (3, 40003), (1, 70001)])
+def test_gpu_every_way_to_the_rts_program(cfg, n, precision):
+    """Tracks around phi = pi, every fiftieth without time variance, so that tracks
+    reach the RTS program in all three ways: picked from their start, over their
+    own slot, and (beyond 32,768 tracks, or within a few MB) through the pool and
+    the list.  The same bits in input order and sorted, replayed, in slices, and
+    in the fixed workspace; the counts and flags of the fit with track states, and
+    in FP64 its parameters: 1e-6 of an error, as a 2 pi jump of ~6,000 errors takes
+    the rounding of 1e-10 there."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from gpukalmanfitter_amd.fitter import DeviceBatch, KalmanFitter, KalmanFitterOptions
+    b = turned(G.generate(cfg, n_tracks=n), np.pi)
+    plain = np.arange(n) % 50 != 25
+    b.start_cov[20, ~plain] = 0.0
+    opts = KalmanFitterOptions(precision=precision, **dict(W, max_rk_trials=20))
+    keys = ("params", "cov", "chi2", "ndf", "n_measured", "status")
+
+    def fit(budget=0, call="fit_batch", calls=1, **sched):
+        kf = KalmanFitter(b.planes, b.field)
+        kf.set_memory_budget(budget)
+        kf.set_schedule(**sched)
+        dev = DeviceBatch(b)
+        for _ in range(calls):
+            dev.clear_results()
+            getattr(kf, call)(dev, opts)
+        res = dev.results_numpy()
+        kf.close()
+        return res
+
+    want = fit()
+    for how in (dict(calls=2), dict(sort_by_length=1), dict(graph=1, calls=3),
+                dict(budget=4 << 20), dict(budget=4 << 20, graph=1, calls=3),
+                dict(budget=4 << 20, sort_by_length=1), dict(call="fit_batch_noalloc", calls=2)):
+        got = fit(**how)
+        for k in keys:
+            assert np.array_equal(got[k], want[k], equal_nan=True), (how, k)
+    kf = KalmanFitter(b.planes, b.field)
+    dev = DeviceBatch(b, track_states=True)
+    kf.fit_batch(dev, opts)
+    ref = dev.results_numpy()
+    kf.close()
+    for k in ("ndf", "n_measured"):
+        assert np.array_equal(want[k], ref[k]), k
+    if precision == "fp64":
+        assert np.array_equal(want["status"][plain], ref["status"][plain])
+        ok = plain & ((ref["status"] & abi.KF_STATUS_OK) != 0)
+        sig = np.sqrt(np.abs(ref["cov"][abi.DIAG_INDEX]))[:, ok]
+        p = ref["params"][:, ok]
+        assert (np.abs(want["params"][:, ok] - p) <= 1e-6 * np.maximum(np.abs(p), sig)).all()
