@@ -122,9 +122,9 @@ __global__ void __launch_bounds__(KF_BLOCK) kf_fit_kernel(FitArgs args) {
 //  - a track near the phi wrap (nearWrap) is left out by its lane and fitted by
 //    the waves at the front of the grid, rts_waves of them, which go through a
 //    share of the positions each and take the tracks they pick 64 at a time;
-//  - a track that the fixed-point smoother leaves in the end (TrackFit::fxSafe; 1
-//    in 2,000 of the material workload spread over azimuth) is fitted again by
-//    its own wave while the others go on, over a store slot of its own
+//  - a track that the fixed-point smoother leaves, for its start covariance before
+//    the pass (TrackFit::fxDefinite) or in the end (fxSafe; 1 in 2,000 of the
+//    material workload spread over azimuth), is fitted by its own wave while the others go on, over a store slot of its own
 //    (redoSlotPerTrack) or a chunk that the wave takes from a pool;
 //  - when the pool is used up it goes to the list of the redo kernel.
 // Fitted after the fused pass alone, a single handed-back track cost a small
@@ -243,6 +243,7 @@ __global__ void __launch_bounds__(KF_FUSED_BLOCK) kf_fused_kernel(FitArgs args) 
     tf.pls = planes;
     tf.fx = sums + threadIdx.x;
     if (rtsBlocks > 0) tf.picker = ka;
+    tf.leaveEarly = true;
     redo = !tf.runFused() && tf.lead;
   }
   const uint64_t redoMask = __ballot(redo);

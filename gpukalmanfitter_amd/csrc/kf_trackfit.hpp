@@ -1006,6 +1006,9 @@ struct TrackFit {
   // wrap (nearWrap), and whether this is one of them
   const FitArgs *picker = nullptr;
   bool elsewhere = false;
+  // whether to leave a track with a singular start covariance before the pass (its
+  // outputs are then not set at all), and whether this is one
+  bool leaveEarly = false, left = false;
   S fxDiag[3];                          // kFxRts: (2,2), (3,3), (4,4) before the material update
   double fxLimit = kDblMax;  // total chi2 below which no smoothed angle can wrap (fxAngles)
 
@@ -2492,9 +2495,16 @@ struct TrackFit {
     // (its code is most of the kernel): `at` says which of the three this is.
     int resume = kResumeNone;
     if (!bad) {
-      if constexpr (kFirst) fxOk = fxDefinite();
       prefetchHit();
       start(pv);
+      // (after what waits for no covariance)
+      if constexpr (kFirst) {
+        fxOk = fxDefinite();
+        if (leaveEarly && a.smoothing && !fxOk) {
+          left = true;
+          return kResumeNone;
+        }
+      }
       navStatus();
       int at = kResumePreLoop;
       for (;;) {
@@ -2600,6 +2610,7 @@ struct TrackFit {
     bool terminated, bad;
     const int resume = forwardPass(steps, terminated, bad);
     if (elsewhere) return true;
+    if (left) return false;
     if (resume == kResumeNone) {
       writeFinal(bad ? KF_STATUS_BAD_INPUT : statusBits(steps, terminated), false);
       return true;

@@ -6,13 +6,14 @@
 namespace {
 
 template <typename S, int FK>
-void fusedTracks(Host &h, int32_t *redo) {
+void fusedTracks(Host &h, int32_t *redo, bool early = false) {
   using Fit = TrackFit<S, true, 1, false, false, FK, kKeepFirst>;
   std::vector<typename Fit::FxPair> sums((size_t)Fit::kFxN * KF_FUSED_BLOCK);
   for (int64_t i = 0; i < h.a.n; ++i) {
     Fit tf(h.a, i, nullptr, nullptr, nullptr, nullptr, 0u, i);
     tf.pls = h.planes.data();
     tf.fx = sums.data();
+    tf.leaveEarly = early;
     redo[i] = tf.runFused() ? 0 : 1;
   }
 }
@@ -52,6 +53,25 @@ int kfh_fit_fused(const kf_plane *planes, int32_t n_planes, const kfh_field *f,
                   double *chi2, int32_t *n_measured, uint32_t *status, int32_t *redo) {
   return kfh_fit_fused_kind(planes, n_planes, f, tr, opt, kFieldAny, params, cov, chi2,
                             n_measured, status, redo);
+}
+
+// As the kernel runs it: a track with a singular start covariance is left before
+// the pass, its chi2 and n_measured not set either.
+int kfh_fit_fused_early(const kf_plane *planes, int32_t n_planes, const kfh_field *f,
+                        const kf_tracks *tr, const kf_options *opt, double *params, double *cov,
+                        double *chi2, int32_t *n_measured, uint32_t *status, int32_t *redo) {
+  Host h(planes, n_planes, f, tr, opt, true);
+  h.a.out_params = params;
+  h.a.out_cov = cov;
+  h.a.out_chi2 = chi2;
+  h.a.out_nmeas = n_measured;
+  h.a.out_status = status;
+  h.a.out_ndf = nullptr;
+  if (opt->precision == KF_PRECISION_MIXED)
+    fusedTracks<float, kFieldAny>(h, redo, true);
+  else
+    fusedTracks<double, kFieldAny>(h, redo, true);
+  return 0;
 }
 
 // Whether each track is given to the RTS program from the start (nearWrap).

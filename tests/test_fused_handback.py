@@ -85,6 +85,41 @@ def test_near_wrap_of_bad_input(built):
     assert not near_wrap(b, abi.default_options(**W)).any()
 
 
+@pytest.mark.parametrize("precision", PRECISIONS)
+def test_a_singular_start_covariance_is_left_before_the_pass(built, precision):
+    """Every third track without time variance: those are left with nothing of
+    them fitted, the others are fitted as by the whole batch's program; tracks that
+    the fit refuses keep their flag, and without smoothing nothing is left."""
+    b = G.generate(1, n_tracks=60)
+    b.start_cov[20, ::3] = 0.0
+    b.seq_count[3] = 0
+    opt = abi.default_options(precision=precision, **W)
+    P = C.c_void_p
+    lib = fused_lib()
+    lib.kfh_fit_fused_early.argtypes = [P, C.c_int32, P, C.POINTER(abi.kf_tracks),
+                                        C.POINTER(abi.kf_options)] + [P] * 6
+
+    def early(o):
+        n = b.n_tracks
+        out = dict(params=np.zeros((6, n)), cov=np.zeros((21, n)), chi2=np.full(n, -1.0),
+                   n_measured=np.full(n, -1, dtype=np.int32),
+                   status=np.zeros(n, dtype=np.uint32), redo=np.zeros(n, dtype=np.int32))
+        tr, fld = oracle.host_tracks(b), field_of(b, b.field.scale)
+        assert lib.kfh_fit_fused_early(b.planes, len(b.planes), C.addressof(fld), C.byref(tr),
+                                       C.byref(o), *[v.ctypes.data for v in out.values()]) == 0
+        return out
+
+    f, g = early(opt), fused_fit(b, opt)
+    left = np.arange(60) % 3 == 0
+    left[3] = False
+    assert np.array_equal(f["redo"] != 0, left)
+    assert (f["chi2"][left] == -1.0).all() and (f["n_measured"][left] == -1).all()
+    for k in ("params", "cov", "chi2", "n_measured", "status"):
+        assert np.array_equal(f[k][..., ~left], g[k][..., ~left]), k
+    assert f["status"][3] == abi.KF_STATUS_BAD_INPUT
+    assert not early(abi.default_options(precision=precision, **dict(W, smoothing=0)))["redo"].any()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("cfg,n", [(1, 117), (1, 16385), (3, 40003), (1, 70001)])
