@@ -100,6 +100,9 @@ class kf_tracks(C.Structure):
     ]
 
 
+KF_SORT_AUTO = -1
+
+
 class kf_schedule(C.Structure):
     _fields_ = [
         ("sort_by_length", C.c_int32),

@@ -400,20 +400,6 @@ size_t firstBytes(int precision) {
 }
 size_t fusedBytesPerTrack(int precision) { return firstBytes(precision) + sizeof(uint32_t); }
 
-// Whether a fused fit in input order is sorted by length of itself.  A wave takes
-// as long as its longest track, so where the tracks fill fewer than 4/5 of the
-// states they may have (the caller's max_states; a batch whose longest track is
-// not stated is left alone) and the waves exceed one per SIMD, lengths sorted
-// into waves shorten the launch by more than the sort and the scattered reads
-// cost: filled to 0.55-0.60, 66,000 tracks 745 -> 450 us (FP64, 5-30 planes) and
-// 1,334 -> 831 us (mixed, 8-40 planes with material), 500,003 tracks 2,719 ->
-// 2,036 us; with equal lengths 100,000 tracks would go from 188 to 208 us.  Up to
-// one wave per SIMD the longest track decides, sorted or not.
-bool sortPays(const kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt, int lanes_per_track) {
-  return opt->max_states > 0 && tr->n_tracks * lanes_per_track > (int64_t)256 * ctx->n_cu &&
-         (double)tr->n_hits < 0.8 * (double)tr->n_tracks * (double)opt->max_states;
-}
-
 // Positions per slice: the largest multiple of 64 whose working set fits the
 // budget (at least 64), or the whole batch.
 int64_t sliceTracks(const kf_ctx *ctx, int64_t n, size_t bytes_per_track) {
@@ -673,7 +659,8 @@ int kf_fit(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt, const kf_res
   KfdLaunch L{};
   L.lanes_per_track = sc.lanes_per_track;
   L.store_by_plane = sc.store_by_plane;
-  const bool sort = sc.sort_by_length || (fused && sortPays(ctx, tr, opt, sc.lanes_per_track));
+  const bool sort = kfd::sortsByLength(sc, fused, tr->n_tracks, tr->n_hits, opt->max_states,
+                                       ctx->n_cu);
   if (sort || sc.persistent) {
     const size_t order_bytes = ((size_t)a.n * sizeof(int32_t) + 255) / 256 * 256;
     rc = grow(ctx, &ctx->sched_buf, &ctx->sched_bytes, order_bytes + 514 * sizeof(uint32_t), s,
@@ -751,7 +738,7 @@ int kf_fit(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt, const kf_res
 
 void kf_schedule_default(kf_schedule *s) {
   if (!s) return;
-  s->sort_by_length = 0;
+  s->sort_by_length = KF_SORT_AUTO;
   s->persistent = 0;
   s->waves_per_cu = 4;
   s->chunks_per_grab = 1;
@@ -792,29 +779,7 @@ int kf_autotune(kf_ctx *ctx, const kf_tracks *tracks, const kf_options *opt, con
   if (!ctx) return fail(nullptr, KF_E_INVALID, "kf_autotune: ctx is NULL");
   if (!tracks || !opt || !res) return fail(ctx, KF_E_INVALID, "kf_autotune: NULL argument");
   if (repeats < 1) repeats = 1;
-  std::vector<kf_schedule> cand;
-  for (int sort = 0; sort <= 1; ++sort)
-    for (int byPlane = 0; byPlane <= 1; ++byPlane) {
-      kf_schedule c;
-      kf_schedule_default(&c);
-      c.sort_by_length = sort;
-      c.store_by_plane = byPlane;
-      c.graph = 1;
-      cand.push_back(c);
-      if (!byPlane)
-        for (int l : {2, 4}) {  // lane groups (one-shot grid, slots by measurement)
-          kf_schedule cl = c;
-          cl.lanes_per_track = l;
-          cand.push_back(cl);
-        }
-      for (int w : {2, 4, 8})
-        for (int g : {1, 4}) {
-          c.persistent = 1;
-          c.waves_per_cu = w;
-          c.chunks_per_grab = g;
-          cand.push_back(c);
-        }
-    }
+  const std::vector<kf_schedule> cand = kfd::scheduleCandidates(res->track_states != nullptr);
   const kf_schedule saved = ctx->sched;
   double best_t = 1e300;
   kf_schedule best_s = saved;

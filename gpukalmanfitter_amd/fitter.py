@@ -376,7 +376,8 @@ class KalmanFitter:
                                              C.byref(results), C.c_void_p(s.cuda_stream)))
 
     def set_schedule(self, **fields):
-        """Sets kf_schedule fields (unnamed ones keep the library defaults)."""
+        """Sets kf_schedule fields (unnamed ones keep the library defaults; a
+        ``sort_by_length`` of 0 keeps the input order)."""
         s = abi.kf_schedule()
         self._lib.kf_schedule_default(C.byref(s))
         for k, v in fields.items():

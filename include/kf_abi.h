@@ -172,12 +172,14 @@ typedef struct kf_results {
 
 /* How kf_fit lays the batch onto the GPU (this build's; the reference
  * launches one thread per track on a fixed grid, Run/GPU/Kernels.cu:6-55). */
+#define KF_SORT_AUTO (-1)
 typedef struct kf_schedule {
-  int32_t sort_by_length;  /* fit tracks in order of decreasing sequence length, so a
-                              wave's tracks take similar numbers of steps (default 0: a
-                              fit without track states does so of itself where
-                              options.max_states and n_hits show unequal lengths and
-                              the batch exceeds one wave per SIMD; same bits) */
+  int32_t sort_by_length;  /* 1: fit tracks in order of decreasing sequence length, so a
+                              wave's tracks take similar numbers of steps; 0: in input
+                              order; KF_SORT_AUTO (default): a fit without track states
+                              is sorted where options.max_states and n_hits show unequal
+                              lengths and the batch exceeds one wave per SIMD, others
+                              are not.  Same bits. */
   int32_t persistent;      /* 1: resident waves pull 64-track chunks from a work queue (fits
                               with track states; the others take one track per lane) */
   int32_t waves_per_cu;    /* persistent grid size, waves per compute unit (default 4) */
@@ -272,18 +274,18 @@ int kf_chi2_gradient(kf_ctx *ctx, const kf_tracks *tracks, const kf_options *opt
                      double *grad_raw, uint32_t *track_flags, void *stream);
 
 /* Schedule of later kf_fit calls on ctx (kf_schedule_default: one thread per
- * track in input order, no graph). */
+ * track, sorted where that pays, no graph). */
 void kf_schedule_default(kf_schedule *s);
 int kf_set_schedule(kf_ctx *ctx, const kf_schedule *s);
 int kf_get_schedule(const kf_ctx *ctx, kf_schedule *s);
 
-/* Autotuner: fits the batch with each candidate schedule (sort on/off x
- * store slots by measurement or by plane x one-shot grid or persistent work
- * queue with 2/4/8 waves per CU and 1/4 chunks per grab, graph replay), times
- * every candidate on `stream` with HIP events (best of `repeats` fits), keeps
- * the fastest as ctx's schedule and returns it with its time.  The results
- * buffers hold the last fit.  The one-shot candidates with slots by
- * measurement also run with 2 and 4 lanes per track. */
+/* Autotuner: fits the batch with each candidate schedule, times every one on
+ * `stream` with HIP events (best of `repeats` fits), keeps the fastest as ctx's
+ * schedule and returns it with its time.  The results buffers hold the last
+ * fit.  The candidates replay a graph and are what changes the launch: sort on
+ * and off x 1, 2 and 4 lanes per track; with track states also store slots by
+ * plane, and the persistent work queue with 2/4/8 waves per CU and 1/4 chunks
+ * per grab. */
 int kf_autotune(kf_ctx *ctx, const kf_tracks *tracks, const kf_options *opt,
                 const kf_results *res, void *stream, int32_t repeats, kf_schedule *best,
                 double *best_ms);

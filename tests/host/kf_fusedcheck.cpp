@@ -74,6 +74,18 @@ int kfh_fit_fused_early(const kf_plane *planes, int32_t n_planes, const kfh_fiel
   return 0;
 }
 
+// Whether a fit with this schedule sorts its tracks.
+int kfh_sorts(const kf_schedule *s, int32_t fused, int64_t n_tracks, int64_t n_hits,
+              int32_t max_states, int32_t n_cu) {
+  return sortsByLength(*s, fused != 0, n_tracks, n_hits, max_states, n_cu) ? 1 : 0;
+}
+// The autotuner's candidates (at most `capacity` of them); their number.
+int kfh_schedule_candidates(int32_t track_states, kf_schedule *out, int32_t capacity) {
+  const std::vector<kf_schedule> c = scheduleCandidates(track_states != 0);
+  for (size_t k = 0; k < c.size() && k < (size_t)capacity; ++k) out[k] = c[k];
+  return (int)c.size();
+}
+
 // Whether each track is given to the RTS program from the start (nearWrap).
 int kfh_near_wrap(const kf_plane *planes, int32_t n_planes, const kfh_field *f,
                   const kf_tracks *tr, const kf_options *opt, int32_t *pick) {
