@@ -20,7 +20,8 @@ namespace kfd {
 // than the sort and the scattered reads cost: filled to 0.55-0.60, 66,000 tracks
 // 745 -> 450 us (FP64, 5-30 planes) and 1,334 -> 831 us (mixed, 8-40 planes with
 // material), 500,003 tracks 2,719 -> 2,036 us; with equal lengths, where holes or a
-// loose max_states make them look unequal, 100,000 tracks go from 188 to 208 us.
+// loose max_states make them look unequal, 100,000 tracks go from 191 to 205 us (four
+// launches; a schedule with sort_by_length = 0 spares them).
 // Up to one wave per SIMD the longest track decides, sorted or not.
 inline bool sortsByLength(const kf_schedule &sc, bool fused, int64_t n_tracks, int64_t n_hits,
                           int32_t max_states, int n_cu) {
