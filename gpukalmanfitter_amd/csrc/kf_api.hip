@@ -160,6 +160,14 @@ int grow(kf_ctx *ctx, void **buf, size_t *cap, size_t need, hipStream_t s, const
   return KF_OK;
 }
 
+// Whether the caller is capturing this stream (what is launched has then not run
+// when the call returns).
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return false;
+}
 
 }  // namespace
 
@@ -509,7 +517,7 @@ int setupFused(kf_ctx *ctx, int precision, int64_t slice, hipStream_t s, kfd::Fi
   carveFused(F, ctx->store, ctx->carry, ctx->redo, a);
   if (!ctx->redo_clean) {
     KF_HIP(ctx, kfd_launch_redo_reset(a.redo, s));
-    ctx->redo_clean = true;
+    ctx->redo_clean = !capturing(s);  // captured: only a replay zeroes them
   }
   return KF_OK;
 }

@@ -1,0 +1,58 @@
+"""kf_fit recorded into a caller's graph: what it launches there must not count as run."""
+import numpy as np
+import pytest
+
+from gpukalmanfitter_amd import configs
+from gpukalmanfitter_amd import generate as G
+
+from test_fused_fit import turned
+
+pytestmark = pytest.mark.gpu
+OPTS = dict(configs.WORKLOAD_FIT_OPTIONS, max_rk_trials=20)
+KEYS = ("params", "cov", "chi2", "ndf", "n_measured", "status")
+
+
+@pytest.fixture
+def torch():
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return torch
+
+
+def record(torch, kf, dev, opts):
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream(), capture_error_mode="relaxed"):
+        kf.fit_batch(dev, opts)
+    return graph
+
+
+def same(got, want):
+    for k in KEYS:
+        assert np.array_equal(got[k], want[k], equal_nan=True), k
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_gpu_eager_fit_after_a_capture_that_never_ran(torch, precision):
+    """The first fit of a context is recorded and not replayed; an eager fit of
+    tracks that reach the pool and the list follows, then replays."""
+    from gpukalmanfitter_amd.fitter import DeviceBatch, KalmanFitter, KalmanFitterOptions
+    b = turned(G.generate(1, n_tracks=40000), np.pi)
+    b.start_cov[20, ::50] = 0.0
+    opts = KalmanFitterOptions(precision=precision, **OPTS)
+    dev = DeviceBatch(b)
+    kf = KalmanFitter(b.planes, b.field)
+    kf.fit_batch(dev, opts)
+    want = dev.results_numpy()
+    kf.close()
+    kf = KalmanFitter(b.planes, b.field)
+    graph = record(torch, kf, dev, opts)
+    dev.clear_results()
+    kf.fit_batch(dev, opts)
+    same(dev.results_numpy(), want)
+    for _ in range(3):
+        dev.clear_results()
+        graph.replay()
+        torch.cuda.synchronize()
+        same(dev.results_numpy(), want)
+    kf.close()
