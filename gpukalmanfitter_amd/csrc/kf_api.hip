@@ -160,8 +160,8 @@ int grow(kf_ctx *ctx, void **buf, size_t *cap, size_t need, hipStream_t s, const
   return KF_OK;
 }
 
-// Whether the caller is capturing this stream (what is launched has then not run
-// when the call returns).
+// Whether the caller is capturing this stream (buffers can then not grow, and
+// what is launched has not run when the call returns).
 bool capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
@@ -506,7 +506,17 @@ void carveFused(const FusedLayout &F, void *store, void *carry, void *redo, kfd:
 int setupFused(kf_ctx *ctx, int precision, int64_t slice, hipStream_t s, kfd::FitArgs &a) {
   const size_t budget = (ctx->budget < KF_REDO_STORE_BYTES) ? (size_t)ctx->budget
                                                             : (size_t)KF_REDO_STORE_BYTES;
-  const FusedLayout F = fusedLayout(precision, slice, a.max_states, budget);
+  FusedLayout F = fusedLayout(precision, slice, a.max_states, budget);
+  auto held = [&] {
+    return F.store.store() <= ctx->store_bytes && F.redo_bytes() <= ctx->redo_bytes;
+  };
+  // under capture, fewer chunks where the buffers hold no more
+  if (ctx->store && !held() && capturing(s)) {
+    const FusedLayout wanted = F;
+    for (size_t b = ctx->store_bytes; b > 0 && !held(); b /= 2)
+      F = fusedLayout(precision, slice, a.max_states, b);
+    if (!held()) F = wanted;
+  }
   int rc = grow(ctx, &ctx->store, &ctx->store_bytes, F.store.store(), s, "state store");
   if (rc != KF_OK) return rc;
   rc = grow(ctx, &ctx->carry, &ctx->carry_bytes, F.carry_bytes, s, "hand-over buffer");
@@ -667,12 +677,14 @@ int kf_fit(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt, const kf_res
   KfdLaunch L{};
   L.lanes_per_track = sc.lanes_per_track;
   L.store_by_plane = sc.store_by_plane;
-  const bool sort = kfd::sortsByLength(sc, fused, tr->n_tracks, tr->n_hits, opt->max_states,
-                                       ctx->n_cu);
+  bool sort = kfd::sortsByLength(sc, fused, tr->n_tracks, tr->n_hits, opt->max_states, ctx->n_cu);
+  const size_t order_bytes = ((size_t)a.n * sizeof(int32_t) + 255) / 256 * 256;
+  const size_t sched_bytes = order_bytes + 514 * sizeof(uint32_t);
+  // the automatic sort is left out where its buffer cannot grow
+  if (sort && sc.sort_by_length == KF_SORT_AUTO && sched_bytes > ctx->sched_bytes && capturing(s))
+    sort = false;
   if (sort || sc.persistent) {
-    const size_t order_bytes = ((size_t)a.n * sizeof(int32_t) + 255) / 256 * 256;
-    rc = grow(ctx, &ctx->sched_buf, &ctx->sched_bytes, order_bytes + 514 * sizeof(uint32_t), s,
-              "schedule buffers");
+    rc = grow(ctx, &ctx->sched_buf, &ctx->sched_bytes, sched_bytes, s, "schedule buffers");
     if (rc != KF_OK) return rc;
     L.order = (int32_t *)ctx->sched_buf;
     L.sort_scratch = (uint32_t *)((char *)ctx->sched_buf + order_bytes);

@@ -1,4 +1,5 @@
-"""kf_fit recorded into a caller's graph: what it launches there must not count as run."""
+"""kf_fit recorded into a caller's graph, with the buffers of an earlier fit or none:
+what the fit launches there must need no larger ones, and must not count as run."""
 import numpy as np
 import pytest
 
@@ -30,6 +31,35 @@ def record(torch, kf, dev, opts):
 def same(got, want):
     for k in KEYS:
         assert np.array_equal(got[k], want[k], equal_nan=True), k
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_gpu_capture_after_a_fit_of_other_shape(torch, precision):
+    """A fit of twice the tracks with 17 states each, in input order, then 70,000
+    ragged tracks with 30, which would sort of themselves, recorded.  Every replay,
+    with eager fits between, gives the eager fit's bits."""
+    from gpukalmanfitter_amd.fitter import DeviceBatch, KalmanFitter, KalmanFitterOptions
+    b = turned(G.generate(3, n_tracks=140000), np.pi)
+    opts = KalmanFitterOptions(precision=precision, **OPTS)
+    first = DeviceBatch(b, max_states=17)
+    dev = DeviceBatch(b.subset(np.arange(70000)), max_states=30)
+    kf = KalmanFitter(b.planes, b.field)
+    kf.fit_batch(dev, opts)
+    want = dev.results_numpy()
+    kf.close()
+    kf = KalmanFitter(b.planes, b.field)
+    kf.fit_batch(first, opts)
+    want_first = first.results_numpy()
+    graph = record(torch, kf, dev, opts)
+    for _ in range(3):
+        dev.clear_results()
+        graph.replay()
+        torch.cuda.synchronize()
+        same(dev.results_numpy(), want)
+        first.clear_results()
+        kf.fit_batch(first, opts)
+        same(first.results_numpy(), want_first)
+    kf.close()
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
