@@ -500,12 +500,26 @@ void carveFused(const FusedLayout &F, void *store, void *carry, void *redo, kfd:
   a.rts_waves = (int32_t)F.rts;
 }
 
+// The part of the budget that a fused fit's store chunks may take, and its slice:
+// the positions whose kept states and list fit in what the chunks leave (64 at
+// least).
+size_t fusedStoreBudget(const kf_ctx *ctx) {
+  return (size_t)std::min<uint64_t>(ctx->budget / 2, KF_REDO_STORE_BYTES);
+}
+int64_t fusedSlice(const kf_ctx *ctx, int precision, int64_t n, int32_t max_states) {
+  const FusedLayout F = fusedLayout(precision, n, max_states, fusedStoreBudget(ctx));
+  // (1,024: the rounding of the three buffers' parts)
+  const uint64_t chunks = F.store.store() + F.store.carry_bytes + 1024;
+  const uint64_t rest = ctx->budget > chunks ? ctx->budget - chunks : 0;
+  const int64_t fit = (int64_t)(rest / fusedBytesPerTrack(precision)) / 64 * 64;
+  return fit >= n ? n : std::max<int64_t>(fit, 64);
+}
+
 // The working storage of a fused fit, from the context's buffers (grown as
 // needed); the redo counters are zeroed when the buffer is new or a call failed
 // between the kernel that fills the list and the one that clears it.
 int setupFused(kf_ctx *ctx, int precision, int64_t slice, hipStream_t s, kfd::FitArgs &a) {
-  const size_t budget = (ctx->budget < KF_REDO_STORE_BYTES) ? (size_t)ctx->budget
-                                                            : (size_t)KF_REDO_STORE_BYTES;
+  const size_t budget = fusedStoreBudget(ctx);
   FusedLayout F = fusedLayout(precision, slice, a.max_states, budget);
   auto held = [&] {
     return F.store.store() <= ctx->store_bytes && F.redo_bytes() <= ctx->redo_bytes;
@@ -667,9 +681,9 @@ int kf_fit(kf_ctx *ctx, const kf_tracks *tr, const kf_options *opt, const kf_res
   hipStream_t s = (hipStream_t)stream;
   const bool ts = res->track_states != nullptr;
   const bool fused = fitIsFused(ts);
-  const int64_t slice = sliceTracks(
-      ctx, a.n,
-      fused ? fusedBytesPerTrack(opt->precision) : storeBytesPerTrack(a, opt->precision, ts, false));
+  const int64_t slice =
+      fused ? fusedSlice(ctx, opt->precision, a.n, a.max_states)
+            : sliceTracks(ctx, a.n, storeBytesPerTrack(a, opt->precision, ts, false));
   rc = fused ? setupFused(ctx, opt->precision, slice, s, a)
              : setupStores(ctx, opt->precision, ts, false, slice, s, a);
   if (rc != KF_OK) return rc;

@@ -291,7 +291,8 @@ int kf_autotune(kf_ctx *ctx, const kf_tracks *tracks, const kf_options *opt,
                 double *best_ms);
 
 /* Device-memory budget of ctx's per-batch working buffers (per-state stores,
- * kernel hand-over, adjoint stacks and per-track adjoints); 0 restores the
+ * kernel hand-over, the kept states and store chunks of a fit without track
+ * states, adjoint stacks and per-track adjoints); 0 restores the
  * default, KF_DEFAULT_MEMORY_BUDGET.  A batch whose working set exceeds the
  * budget is fitted in consecutive slices of positions (multiples of 64
  * tracks) that reuse the same buffers; results do not depend on the slicing.
