@@ -23,7 +23,7 @@ void fusedTracks(Host &h, int32_t *redo, bool early = false) {
 extern "C" {
 
 // The fit of every track by the fused program, built for either field kind
-// (0, the mixed mode's only), the constant field (1) or the grid (2): params [6][n], cov [21][n],
+// (0), the constant field (1) or the grid (2): params [6][n], cov [21][n],
 // chi2, n_measured, status [n], and redo [n], nonzero for a track that it
 // leaves to the RTS program (its params, cov and status are not set).
 int kfh_fit_fused_kind(const kf_plane *planes, int32_t n_planes, const kfh_field *f,
@@ -37,7 +37,12 @@ int kfh_fit_fused_kind(const kf_plane *planes, int32_t n_planes, const kfh_field
   h.a.out_nmeas = n_measured;
   h.a.out_status = status;
   h.a.out_ndf = nullptr;
-  if (opt->precision == KF_PRECISION_MIXED)
+  const bool mixed = opt->precision == KF_PRECISION_MIXED;
+  if (mixed && field_kind == kFieldGrid)
+    fusedTracks<float, kFieldGrid>(h, redo);
+  else if (mixed && field_kind == kFieldConst)
+    fusedTracks<float, kFieldConst>(h, redo);
+  else if (mixed)
     fusedTracks<float, kFieldAny>(h, redo);
   else if (field_kind == kFieldGrid)
     fusedTracks<double, kFieldGrid>(h, redo);
