@@ -257,7 +257,7 @@ class DeviceBatch:
             buffer = torch.zeros(size, dtype=torch.uint8, device=self.device)
             self.out = {name: self._view(buffer, at, shape, types[dtype])
                         for (name, shape, dtype), at in zip(fields, offsets)}
-            self._out_layout = buffer, dict(self.out), fields, offsets
+            self._out_layout = buffer, fields, offsets
         else:
             self.out = {name: torch.zeros(shape, dtype=types[dtype], device=self.device)
                         for name, shape, dtype in fields}
@@ -281,12 +281,22 @@ class DeviceBatch:
         for v in self.out.values():
             v.zero_()
 
+    def _outputs_in_place(self):
+        """Whether every output is still the view of the common buffer (a caller may
+        have put other tensors, or other storage, in its place)."""
+        buffer, fields, offsets = self._out_layout
+        base = buffer.data_ptr()
+        return len(self.out) == len(fields) and all(
+            name in self.out and self.out[name].data_ptr() == base + at
+            and tuple(self.out[name].shape) == shape and self.out[name].is_contiguous()
+            and self.out[name].element_size() == np.dtype(dtype).itemsize
+            for (name, shape, dtype), at in zip(fields, offsets))
+
     def results_numpy(self):
         """Copies the outputs to host numpy arrays (synchronising)."""
-        # one copy, while the outputs are the ones allocated together
-        if self._out_layout and self.out.keys() == self._out_layout[1].keys() and all(
-                self.out[k] is v for k, v in self._out_layout[1].items()):
-            buffer, _, fields, offsets = self._out_layout
+        # one copy, while the outputs lie where they were allocated together
+        if self._out_layout and self._outputs_in_place():
+            buffer, fields, offsets = self._out_layout
             host = buffer.cpu().numpy()
             res = {name: host[at:at + math.prod(shape) * np.dtype(dtype).itemsize]
                    .view(dtype).reshape(shape)
