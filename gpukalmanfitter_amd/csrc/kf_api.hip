@@ -475,12 +475,18 @@ struct FusedLayout {
 };
 FusedLayout fusedLayout(int precision, int64_t slice, int32_t max_states, size_t budget) {
   FusedLayout F;
-  // as many chunks of each kind as the slice has waves, within the limits and,
-  // between the two, the budget; one for handed-back tracks at least
+  // a chunk for every wave of the slice where the limit and the budget allow it;
+  // else chunks of each kind, between the two the budget, one for handed-back tracks
+  // at least
   const size_t one = storeLayout(precision, false, false, 64, max_states).store();
   const int64_t waves = (slice + 63) / 64, fit = std::max<int64_t>((int64_t)(budget / one), 1);
-  F.rts = std::min(std::min<int64_t>(waves, KF_RTS_WAVES), fit / 2);
-  F.lanes = (F.rts + std::min(std::min<int64_t>(waves, KF_REDO_WAVES), fit - F.rts)) * 64;
+  if (waves <= std::min<int64_t>(fit, KF_RTS_WAVES)) {
+    F.rts = waves;
+    F.lanes = waves * 64;
+  } else {
+    F.rts = std::min<int64_t>(KF_RTS_WAVES, fit / 2);
+    F.lanes = (F.rts + std::min<int64_t>(KF_REDO_WAVES, fit - F.rts)) * 64;
+  }
   F.store = storeLayout(precision, false, false, F.lanes, max_states);
   F.carry_bytes = ((size_t)slice * firstBytes(precision) + 255) / 256 * 256;
   F.list_bytes = ((KF_REDO_LIST + (size_t)slice) * sizeof(uint32_t) + 255) / 256 * 256;

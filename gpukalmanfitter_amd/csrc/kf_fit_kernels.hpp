@@ -179,8 +179,12 @@ KFD_INLINE const DevPlane *tableToLds(const FitArgs &args, double *lds_table) {
 
 // One of the waves for tracks near the wrap: its share of the positions, every
 // rts_waves-th 64 of them (sorted by length or by angle, each then has as much to
-// do), the picked ones collected, at most 63 + 64, until a wave is full.
-template <typename S, bool PLDS, int FK>
+// do), the picked ones collected, at most 63 + 64, until a wave is full.  Its
+// store slots are those of its lanes, so that a few tracks lie together; where the
+// chunk is also that of the positions' own wave (redoSlotPerTrack) that one takes
+// slots from the other end for the tracks it leaves, or, with several waves to a
+// chunk (L > 1), both take those of the positions.
+template <typename S, bool PLDS, int L, int FK>
 KFD_INLINE void fitNearWrap(const FitArgs &args, int64_t wave, uint32_t *list, LdsPlane *table) {
   const FitArgs *ka = (const FitArgs *)__builtin_amdgcn_kernarg_segment_ptr();
   if (wave >= args.rts_waves) return;
@@ -209,7 +213,9 @@ KFD_INLINE void fitNearWrap(const FitArgs &args, int64_t wave, uint32_t *list, L
     n -= take;
     if (lane < take) {
       const int64_t pos = args.first + (int64_t)local;
-      redoTrack<S, PLDS, FK>(ka, args.order ? (int64_t)args.order[pos] : pos, wave * 64 + lane,
+      redoTrack<S, PLDS, FK>(ka, args.order ? (int64_t)args.order[pos] : pos,
+                             (L > 1 && redoSlotPerTrack(args)) ? (int64_t)local
+                                                               : wave * 64 + lane,
                              table);
     }
   }
@@ -221,6 +227,11 @@ __global__ void __launch_bounds__(KF_FUSED_BLOCK) kf_fused_kernel(FitArgs args) 
   __shared__ typename Fit::FxPair sums[Fit::kFxN * KF_FUSED_BLOCK];
   __shared__ uint32_t picked[KF_FUSED_BLOCK / 64][128];
   extern __shared__ double lds_table[];
+  static_assert(sizeof sums + sizeof picked +
+                        sizeof(DevPlane) * (sizeof(S) == sizeof(double) ? KF_FUSED_LDS_PLANES_FP64
+                                                                        : KF_FUSED_LDS_PLANES_MIXED) <=
+                    160 * 1024 / 2,
+                "two blocks per compute unit");
   const DevPlane *planes = args.planes;
   if constexpr (PLDS) planes = tableToLds(args, lds_table);
   LdsPlane *table = PLDS ? (LdsPlane *)planes : nullptr;
@@ -228,7 +239,7 @@ __global__ void __launch_bounds__(KF_FUSED_BLOCK) kf_fused_kernel(FitArgs args) 
   const uint32_t rtsBlocks = (uint32_t)rtsBlocksOf(args);
   if (blockIdx.x < rtsBlocks) {
     const int w = (int)(threadIdx.x >> 6), per = rtsPerBlock(args);
-    if (w < per) fitNearWrap<S, PLDS, FK>(args, (int64_t)blockIdx.x * per + w, picked[w], table);
+    if (w < per) fitNearWrap<S, PLDS, L, FK>(args, (int64_t)blockIdx.x * per + w, picked[w], table);
     return;
   }
   const int64_t t = (int64_t)(blockIdx.x - rtsBlocks) * KF_FUSED_BLOCK + threadIdx.x;
@@ -248,10 +259,12 @@ __global__ void __launch_bounds__(KF_FUSED_BLOCK) kf_fused_kernel(FitArgs args) 
   }
   const uint64_t redoMask = __ballot(redo);
   if (redoMask == 0) return;
-  int64_t slot = (int64_t)args.rts_waves * 64 + local;
-  if (!redoSlotPerTrack(args)) {
+  const int lane = (int)(threadIdx.x & 63u);
+  int64_t slot = local;
+  if (redoSlotPerTrack(args)) {
+    if constexpr (L == 1) slot = local - lane + 63 - __popcll(redoMask & ((1ull << lane) - 1ull));
+  } else {
     const int first = __ffsll((unsigned long long)redoMask) - 1;
-    const int lane = (int)(threadIdx.x & 63u);
     uint32_t chunk = 0;
     if (lane == first) chunk = atomicAdd(args.redo, 1u);
     chunk = (uint32_t)__shfl((int)chunk, first, 64);

@@ -1,5 +1,5 @@
 // kf_kernels.hpp -- launch interface between the C ABI (kf_api.hip) and the
-// fit kernel (kf_kernels.hip).
+// fit kernels (kf_fit_kernels.hpp, kf_kernels.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -17,8 +17,9 @@
 #define KF_FUSED_BLOCK 128
 #endif
 // The same for the fused fit kernel, whose blocks also hold the smoother's sums
-// (46 KB in FP64, 64 KB in the mixed mode): the largest tables with which two
-// blocks (one wave per SIMD) still fit the 160 KB of a compute unit.
+// and a list (47 KB in FP64, 65 KB in the mixed mode): two blocks (one wave per
+// SIMD) have to fit the 160 KB of a compute unit, which 112 planes just do in the
+// mixed mode and 248 would in FP64 (kf_fused_kernel asserts it).
 #define KF_FUSED_LDS_PLANES_FP64 224
 #define KF_FUSED_LDS_PLANES_MIXED 112
 // Waves of the fused launch that run the RTS program over the tracks near the phi
@@ -147,7 +148,7 @@ struct FitArgs {
   // tsd, tss (redo_lanes slots, one store chunk per 64) and redo_d, redo_i
   // ([KF_CARRY_D], [KF_CARRY_I][redo_lanes]): the first rts_waves chunks are
   // those of the waves for tracks near the wrap, the others are for tracks
-  // handed back later.  redo[0]: chunks of the latter taken by waves of the
+  // handed back later (none: redoSlotPerTrack).  redo[0]: chunks of the latter taken by waves of the
   // fused kernel, redo[1]: positions left in the list for the redo kernel,
   // redo[2]: its ticket (all 0 between fits); redo[KF_REDO_LIST ...]: the
   // positions.
@@ -173,12 +174,12 @@ KFD_INLINE const FitArgs *uniformArgs(const FitArgs *p) {
 #endif
 }
 
-// Whether every position of a fused fit has a store slot of its own for being
-// handed back (up to KF_REDO_WAVES x 64 tracks): no chunk is then drawn from the
-// pool, no list kept, and no redo kernel follows.  For small batches that launch
-// was 5 of 96 us.
+// Whether every position of a fused fit has a store slot of its own for the RTS
+// program, whichever wave runs it (up to KF_RTS_WAVES x 64 tracks): no chunk is
+// then drawn from the pool, no list kept, and no redo kernel follows.  For small
+// batches that launch was 5 of 96 us.
 KFD_INLINE bool redoSlotPerTrack(const FitArgs &a) {
-  return a.rts_waves * (int64_t)64 + (a.count + 63) / 64 * 64 <= a.redo_lanes;
+  return a.rts_waves * (int64_t)64 == a.redo_lanes && a.count <= a.redo_lanes;
 }
 // Blocks of a fused launch that hold the waves for tracks near the wrap, and how
 // many each holds: one up to 256, whose compute unit it then has to itself (two
