@@ -105,17 +105,16 @@ __global__ void __launch_bounds__(KF_BLOCK) kf_fit_kernel(FitArgs args) {
 // nor checkpoints: forward filter with the fixed-point smoother, then back to
 // the perigee (TrackFit::runFused).  Per-track state in registers (one wave
 // per SIMD), the smoother's sums in LDS (46 KB per block in FP64, 64 KB in the
-// mixed mode), the plane table in
-// dynamic LDS (PLDS) or global memory.  FK: the field kind, so the step loop
-// carries no code of the other one (either kind where the plane table is in
-// global memory).  PERS, L as in kf_fit_kernel.
+// mixed mode), the plane table in dynamic LDS (PLDS) or global memory.  FK: the
+// field kind, so the step loop carries no code of the other one (either kind where
+// the plane table is in global memory).  L as in kf_fit_kernel.
 //
 // Bound by instruction issue: a wave of ten planes issues 24,300 vector
 // instructions in FP64 (1,048,576 tracks: 1.30 ms) and 41,000 in the mixed
 // mode (1.73 ms), a third of them the RTS gain and its sums (TrackFit::fxRtsStep; the
 // FP64 sums round differently from the recursion over float covariances, 1e-7
 // in the time variance).  Mixed, against the forward and backward kernels that
-// passed 304 B per state through memory: 1,048,576 tracks 2.03 -> 1.75 ms,
+// passed 304 B per state through memory: 1,048,576 tracks 2.03 -> 1.73 ms,
 // 500,003 ragged ones 2.81 -> 2.30 ms, 100,003 with material 1.93 -> 1.70 ms.
 //
 // Tracks for the RTS program (redoTrack), in three ways:

@@ -20,9 +20,10 @@
 // cells (a counting sort, three short launches); the surfaces need no order.
 // The cone passes every surface whose sphere test and full test a ray of it
 // could pass, so the kept pairs do not change.  16,384 rays x 37,122
-// triangles: 160 us a call (the count pass 85, the write pass 20, the rest
-// short launches) against 450 without, and 278 with boxes about 16 surfaces
-// in listed order instead of cones; 4,000 x 488 triangles 115 against 216.
+// triangles: 153 us a call (under the profiler the count pass 115, the write pass
+// 20, five short launches 27) against 453 without, and 278 with boxes about 16
+// surfaces in listed order instead of cones; 4,000 x 488 triangles 115 against
+// 216.
 //
 // Output order is (ray, surface) without atomics: the count pass keeps, per
 // (ray, chunk), the number of kept intersections and the first kIxSlots

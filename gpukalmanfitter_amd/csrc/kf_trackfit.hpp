@@ -1,5 +1,5 @@
 // kf_trackfit.hpp -- the per-track Kalman fit program (one track per lane),
-// shared by the fit kernels (kf_kernels.hip) and the chi2 adjoint
+// shared by the fit kernels (kf_fit_kernels.hpp) and the chi2 adjoint
 // (kf_adjoint.hip).
 //
 // The per-lane program is the reference's propagation loop (Propagator.ipp:

@@ -242,10 +242,11 @@ class KalmanFitter {
     kf_options o = options(kfOptions);
     o.max_states = states;
     check(kf_fit(ctx_, &t, &o, &r, nullptr), "kf_fit");
-    // A fit with track states agrees with one without to rounding (kf_abi.h):
-    // the parameters are the latter's, so a per-track call equals the batch
-    // fit bit for bit.  The second fit is one wave's
-    // latency, ~0.1 ms of the call.
+    // A fit with track states agrees with one without to rounding (kf_abi.h), and
+    // the two are different programs.  The states are the former's; the
+    // parameters, chi2 and status are the latter's, so that a per-track call
+    // equals the batch fit bit for bit.  The second fit is one wave's latency,
+    // ~0.1 ms of the call.
     r.track_states = nullptr;
     check(kf_fit(ctx_, &t, &o, &r, nullptr), "kf_fit");
     check(hipDeviceSynchronize() == hipSuccess ? KF_OK : KF_E_HIP, "hipDeviceSynchronize");

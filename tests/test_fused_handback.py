@@ -173,3 +173,42 @@ def test_gpu_every_way_to_the_rts_program(cfg, n, precision):
         sig = np.sqrt(np.abs(ref["cov"][abi.DIAG_INDEX]))[:, ok]
         p = ref["params"][:, ok]
         assert (np.abs(want["params"][:, ok] - p) <= 1e-6 * np.maximum(np.abs(p), sig)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("cfg,n", [(1, 200), (1, 40000), (3, 5000)])
+def test_gpu_handed_back_tracks_with_a_large_table(cfg, n, precision):
+    """300 planes: the table is in global memory, and the RTS program the build for
+    either field kind.  The flags and counts of the fit with the small table; in
+    FP64 its parameters as in the test above, in the mixed mode those of tracks
+    that no wrap is near (twice the mode's 1e-5 between two builds)."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from gpukalmanfitter_amd.fitter import DeviceBatch, KalmanFitter, KalmanFitterOptions
+    from test_gpu_parity import _padded_planes
+    b = turned(G.generate(cfg, n_tracks=n), np.pi)
+    plain = np.arange(n) % 50 != 25
+    b.start_cov[20, ~plain] = 0.0
+    opts = KalmanFitterOptions(precision=precision, **dict(W, max_rk_trials=20))
+    res = []
+    for x in (b, dataclasses.replace(b, planes=_padded_planes(b.planes, 300 - len(b.planes)))):
+        kf = KalmanFitter(x.planes, x.field)
+        dev = DeviceBatch(x)
+        kf.fit_batch(dev, opts)
+        res.append(dev.results_numpy())
+        kf.close()
+    ref, got = res
+    for k in ("ndf", "n_measured"):
+        assert np.array_equal(got[k], ref[k]), k
+    ok = plain & ((ref["status"] & abi.KF_STATUS_OK) != 0)
+    if precision == "fp64":
+        assert np.array_equal(got["status"][plain], ref["status"][plain])
+    else:
+        ok &= ~near_wrap(b, abi.default_options(**W))
+        assert np.array_equal(got["status"][ok], ref["status"][ok])
+    bar = 1e-6 if precision == "fp64" else 2e-5
+    sig = np.sqrt(np.abs(ref["cov"][abi.DIAG_INDEX]))[:, ok]
+    p = ref["params"][:, ok]
+    assert (np.abs(got["params"][:, ok] - p) <= bar * np.maximum(np.abs(p), sig)).all()
