@@ -109,8 +109,8 @@ __global__ void __launch_bounds__(KF_BLOCK) kf_fit_kernel(FitArgs args) {
 // field kind, so the step loop carries no code of the other one (either kind where
 // the plane table is in global memory).  L as in kf_fit_kernel.
 //
-// Bound by instruction issue: a wave of ten planes issues 24,300 vector
-// instructions in FP64 (1,048,576 tracks: 1.30 ms) and 41,000 in the mixed
+// Bound by instruction issue: a wave of ten planes issues 24,600 vector
+// instructions in FP64 (1,048,576 tracks: 1.30 ms) and 40,600 in the mixed
 // mode (1.73 ms), a third of them the RTS gain and its sums (TrackFit::fxRtsStep; the
 // FP64 sums round differently from the recursion over float covariances, 1e-7
 // in the time variance).  Mixed, against the forward and backward kernels that
