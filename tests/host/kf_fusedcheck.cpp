@@ -79,6 +79,11 @@ int kfh_fit_fused_early(const kf_plane *planes, int32_t n_planes, const kfh_fiel
   return 0;
 }
 
+// The square roots and their reciprocals of x [n] from estimates y of 1 / sqrt(x).
+void kfh_roots(int64_t n, const double *x, const double *y, double *s, double *is) {
+  for (int64_t i = 0; i < n; ++i) rootFromEven(x[i], y[i], s[i], is[i]);
+}
+
 // Whether a fit with this schedule sorts its tracks.
 int kfh_sorts(const kf_schedule *s, int32_t fused, int64_t n_tracks, int64_t n_hits,
               int32_t max_states, int32_t n_cu) {
