@@ -212,3 +212,44 @@ def test_gpu_handed_back_tracks_with_a_large_table(cfg, n, precision):
     sig = np.sqrt(np.abs(ref["cov"][abi.DIAG_INDEX]))[:, ok]
     p = ref["params"][:, ok]
     assert (np.abs(got["params"][:, ok] - p) <= bar * np.maximum(np.abs(p), sig)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("lanes", [2, 4])
+@pytest.mark.parametrize("n", [3001, 40000])
+def test_gpu_handed_back_tracks_with_lane_groups(n, lanes, precision):
+    """Several waves to 64 positions, in a small batch (slots of the positions) and
+    through the pool and the list: repeated fits give the same bits, flags and
+    counts are those of one lane per track, and so are in FP64 the parameters
+    (1e-6 as above)."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from gpukalmanfitter_amd.fitter import DeviceBatch, KalmanFitter, KalmanFitterOptions
+    b = turned(G.generate(1, n_tracks=n), np.pi)
+    plain = np.arange(n) % 50 != 25
+    b.start_cov[20, ~plain] = 0.0
+    opts = KalmanFitterOptions(precision=precision, **dict(W, max_rk_trials=20))
+    kf = KalmanFitter(b.planes, b.field)
+    dev = DeviceBatch(b)
+    kf.fit_batch(dev, opts)
+    want = dev.results_numpy()
+    kf.set_schedule(lanes_per_track=lanes)
+    got = []
+    for _ in range(2):
+        dev.clear_results()
+        kf.fit_batch(dev, opts)
+        got.append(dev.results_numpy())
+    kf.close()
+    for k in ("params", "cov", "chi2", "ndf", "n_measured", "status"):
+        assert np.array_equal(got[0][k], got[1][k], equal_nan=True), k
+    g = got[0]
+    for k in ("ndf", "n_measured"):
+        assert np.array_equal(g[k], want[k]), k
+    if precision == "fp64":
+        assert np.array_equal(g["status"][plain], want["status"][plain])
+        ok = plain & ((want["status"] & abi.KF_STATUS_OK) != 0)
+        sig = np.sqrt(np.abs(want["cov"][abi.DIAG_INDEX]))[:, ok]
+        p = want["params"][:, ok]
+        assert (np.abs(g["params"][:, ok] - p) <= 1e-6 * np.maximum(np.abs(p), sig)).all()
